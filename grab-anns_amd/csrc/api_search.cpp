@@ -149,19 +149,30 @@ int search_ex_impl(const grab_search_desc* d, bool sync, bool static_tables) {
     // visited set: LDS when it fits next to the queue, otherwise one table per query in
     // device memory (the reference switches at hash_bitlen >= 14, src/index/search.cu:188-194)
     DeviceScratch ghash;
-    // A small batch splits its merges over the waves when the partial counts fit LDS beside everything else; they
-    // never push the visited set to device memory or the queue out of LDS - such shapes take the plain merge.
-    const bool small = a.nq <= kSmallBatchQueries;
-    SearchLdsLayout lay = search_lds_layout(a.itopk, a.dim, a.cmax, a.search_width, a.hash_bitlen, true, small);
-    a.split_merge = small ? 1 : 0;
-    if (small && (a.hash_bitlen >= 20 || lay.total > kMaxLdsBytes)) {
-        const SearchLdsLayout plain = search_lds_layout(a.itopk, a.dim, a.cmax, a.search_width, a.hash_bitlen, true, false);
-        const bool table_fits_without = a.hash_bitlen < 20 && plain.total <= kMaxLdsBytes;
-        const bool queue_fits_with = search_lds_layout(a.itopk, a.dim, a.cmax, a.search_width, 0, false, true).total <= kMaxLdsBytes;
-        if (table_fits_without || !queue_fits_with) {
-            a.split_merge = 0;
-            lay = plain;
-        }
+    SearchLdsLayout lay = search_lds_layout(a.itopk, a.dim, a.cmax, a.search_width, a.hash_bitlen, true);
+    // Batches of up to 512 queries run on the kernel made for the time of one query (search_small.hip): 1024 threads a
+    // query while every query can have a CU to itself, 512 while two share one.  Measured (kernel times, us, 100k x 128,
+    // itopk 128, width 4; workgroup kernel of 256 threads / 512 threads / 1024 threads): 1 query 115 / 86 / 80, 256: 167 /
+    // 121 / 112, 300: 164 / 129 / 195, 512: 173 / 139 / 207, 600: 172 / 218 / 292; in the same order for other shapes
+    // (itopk 64 and 256, 96 and 256 dimensions, 10 % windows).
+    bool use_small = !use_wave && a.nq <= 2 * kSmallBatchQueries && a.itopk <= kSmallMaxItopk && !(d->flags & GRAB_FLAG_STRICT_REFERENCE);
+    if (static_tables && (a.hash_bitlen >= 20 || lay.total > kMaxLdsBytes)) use_small = false;  // the static array's rules
+    if (use_small) {
+        const bool alone = a.nq <= kSmallBatchQueries;
+        const uint32_t room = alone ? kMaxLdsBytes : kMaxLdsBytes / 2;
+        a.threads = alone ? 1024 : 512;
+        a.degree_shift = (a.degree & (a.degree - 1)) == 0 ? (uint32_t)__builtin_ctz(a.degree) : 32u;
+        // The table always sits in LDS.  It holds 2^hash_bitlen ids at most, and never more than the seeds, the queue and
+        // 30 iterations' neighbours between two rebuilds; with twice as many slots a probe sequence is a slot or two (2 - 9 %
+        // of the kernel against the size that only just holds them).
+        const uint64_t most = std::min<uint64_t>(1ull << a.hash_bitlen, std::max(a.n_seeds, a.itopk) + 30ull * a.search_width * a.degree);
+        auto bytes = [&](uint32_t bits) { return search_small_lds_layout(a.itopk, a.dim, a.cmax, a.search_width, bits).total; };
+        uint32_t bits = 4;
+        while ((1ull << bits) < most) ++bits;
+        use_small = bits <= 15 && bytes(bits) <= room;
+        if (use_small && (1ull << bits) < 2 * most && bytes(bits + 1) <= room) ++bits;
+        a.table_bitlen = bits;
+        if (use_small) lay.total = bytes(bits);
     }
     if (use_wave) {
         lay.total = wlay.total;
@@ -170,8 +181,8 @@ int search_ex_impl(const grab_search_desc* d, bool sync, bool static_tables) {
         a.single_queue = wave_single ? 1 : 0;
         a.reg_queue = wave_reg ? 1 : 0;
         a.fixed_shape = wave_fixed ? 1 : 0;
-    } else if (a.hash_bitlen >= 20 || lay.total > kMaxLdsBytes) {
-        lay = search_lds_layout(a.itopk, a.dim, a.cmax, a.search_width, 0, false, a.split_merge != 0);
+    } else if (!use_small && (a.hash_bitlen >= 20 || lay.total > kMaxLdsBytes)) {
+        lay = search_lds_layout(a.itopk, a.dim, a.cmax, a.search_width, 0, false);
         GRAB_REQUIRE(lay.total <= kMaxLdsBytes, "queue does not fit LDS (itopk %u)", a.itopk);
         const size_t slots = (size_t)a.nq << a.hash_bitlen;
         if (static_tables) {
@@ -221,7 +232,8 @@ int search_ex_impl(const grab_search_desc* d, bool sync, bool static_tables) {
     // an id interval that comes with a table of places is tested on the places
     const int filter = (d->filter_kind == dev::kFilterIdRange && a.rank_of_id != nullptr) ? dev::kFilterRank : d->filter_kind;
     int rc = use_wave ? launch_search_wave(a, d->metric, filter, lay.total, stream)
-                      : launch_search(a, d->metric, filter, lay.total, stream);
+             : use_small ? launch_search_small(a, d->metric, filter, lay.total, stream)
+                         : launch_search(a, d->metric, filter, lay.total, stream);
     if (d->kernel_ms && rc == GRAB_OK) {
         hipError_t e = hipEventRecord(e1, stream);
         if (e == hipSuccess) e = hipEventSynchronize(e1);
@@ -318,9 +330,9 @@ size_t grab_reference_smem_bytes(uint32_t itopk, uint32_t dim, uint32_t search_w
 size_t grab_search_lds_bytes(uint32_t itopk, uint32_t dim, uint32_t search_width, uint32_t degree,
                              uint32_t n_seeds, uint32_t hash_bitlen) {
     const uint32_t cmax = std::max(search_width * degree, std::max(n_seeds, 1u));
-    SearchLdsLayout with_hash = search_lds_layout(itopk, dim, cmax, search_width, hash_bitlen, true, false);
+    SearchLdsLayout with_hash = search_lds_layout(itopk, dim, cmax, search_width, hash_bitlen, true);
     if (hash_bitlen < 20 && with_hash.total <= kMaxLdsBytes) return with_hash.total;
-    return search_lds_layout(itopk, dim, cmax, search_width, 0, false, false).total;
+    return search_lds_layout(itopk, dim, cmax, search_width, 0, false).total;
 }
 
 void grab_search_plan(int wrapper, uint32_t k, uint32_t itopk_param, uint32_t search_width,

@@ -113,7 +113,8 @@ __device__ __forceinline__ float fold4(float s, const float4 a, const float4 b) 
 
 // Rows of any length (a multiple of four floats), query in LDS: lane j of a group of eight folds the chunks j, j + 8, ...
 // in that order.  Four chunks of each row are requested before the first is used, so that a wave keeps up to
-// 8 x 2 x 4 sixteen-byte loads in flight instead of two per lane.
+// 8 x 2 x 4 sixteen-byte loads in flight; the last ones too - a place past the end becomes the row's last chunk and is
+// folded as zeros, which leave a sum as it is - because a row costs one wait for memory per such round.
 template <int METRIC, bool TWO>
 __device__ __forceinline__ void fold_rows_any(const float4* __restrict__ r0, const float4* __restrict__ r1, const float4* q4,
                                               uint32_t j, uint32_t nchunks, float& d0, float& d1) {
@@ -133,10 +134,22 @@ __device__ __forceinline__ void fold_rows_any(const float4* __restrict__ r0, con
             if (TWO) d1 = fold4<METRIC>(d1, qq, x1[u]);
         }
     }
-    for (; c < nchunks; c += 8) {
-        const float4 x0 = r0[c], qq = q4[c];
-        d0 = fold4<METRIC>(d0, qq, x0);
-        if (TWO) d1 = fold4<METRIC>(d1, qq, r1[c]);
+    if (c < nchunks) {  // one to three chunks are left
+        float4 x0[3], x1[3];
+#pragma unroll
+        for (int u = 0; u < 3; ++u) x0[u] = r0[min(c + 8 * u, nchunks - 1u)];
+        if (TWO) {
+#pragma unroll
+            for (int u = 0; u < 3; ++u) x1[u] = r1[min(c + 8 * u, nchunks - 1u)];
+        }
+#pragma unroll
+        for (int u = 0; u < 3; ++u) {
+            const bool in = c + 8 * u < nchunks;
+            const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            const float4 qq = in ? q4[c + 8 * u] : zero;
+            d0 = fold4<METRIC>(d0, qq, in ? x0[u] : zero);
+            if (TWO) d1 = fold4<METRIC>(d1, qq, in ? x1[u] : zero);
+        }
     }
 }
 
@@ -157,12 +170,16 @@ __device__ __forceinline__ float group8_distance(const float* q, const float* ro
 // full (the reference reports "full" as "present").  `full`: the caller knows that every slot is
 // taken (it counts the successful inserts); the answer is then -1 without a walk over the whole
 // table - present or not, the id is not expanded either way.
+// READ_FIRST: look at a slot before the compare-and-swap.  Tables in LDS go without: the swap answers what the read
+// would have, and each is a trip to LDS that the lanes of a wave wait for.
+template <bool READ_FIRST = false>
 __device__ __forceinline__ int hash_insert(uint32_t* table, uint32_t bitlen, uint32_t key, bool full = false) {
     if (full) return -1;
     const uint32_t size = 1u << bitlen, mask = size - 1;
     uint32_t index = (key ^ (key >> bitlen)) & mask;
     for (uint32_t i = 0; i < size; ++i) {
-        uint32_t cur = __atomic_load_n(&table[index], __ATOMIC_RELAXED);
+        uint32_t cur = kInvalidId;
+        if (READ_FIRST) cur = __atomic_load_n(&table[index], __ATOMIC_RELAXED);
         if (cur == kInvalidId) cur = atomicCAS(&table[index], kInvalidId, key);
         if (cur == kInvalidId) return 1;
         if (cur == key) return 0;

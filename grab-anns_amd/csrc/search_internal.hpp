@@ -43,25 +43,21 @@ struct SearchArgs {
     int single_queue;       // wave-per-query kernel: one queue buffer, merged in place (itopk <= 64, ccap <= 128)
     int reg_queue;          // wave-per-query kernel: the queue lives in registers, 1/2/4 entries per lane (itopk <= 256, not strict)
     int per_query_window;
-    int split_merge;        // workgroup-per-query kernel with 1024 threads: the merge is cut into tasks whose partial counts live in LDS
+    uint32_t threads;       // small-batch kernel: threads of a workgroup
+    uint32_t table_bitlen;  // small-batch kernel: slots of the visited set's table (2^hash_bitlen ids at most are in it)
+    uint32_t degree_shift;  // log2 of the degree where that is whole, else 32
     int fixed_shape;        // register-queue kernel: rows of 64 slots all followed, <= 4 parents, <= 64 seeds, filter first, cmax >= 256
     EntryWalk entry;
 };
 
 struct SearchLdsLayout {
-    uint32_t off_query, off_top0, off_top1, off_cand, off_surv, off_parents, off_misc, off_parts, off_hash, total;
+    uint32_t off_query, off_top0, off_top1, off_cand, off_surv, off_parents, off_misc, off_hash, total;
 };
-
-// Batches of up to this many queries get 1024 threads a query instead of 256 (fewer queries than CUs: what counts is
-// how long one query takes), and split a merge over the waves, which leave their partial counts in LDS - unless
-// those counts would push the queue or the visited set out of LDS: then the plain merge runs on the 1024 threads
-constexpr uint32_t kSmallBatchQueries = 256;
-constexpr uint32_t kMergeChunks = 4;  // parts that the candidate list is cut into for a split merge
 
 // cmax = capacity of the survivor / candidate lists = max(search_width*degree, n_seeds)
 __host__ __device__ inline SearchLdsLayout search_lds_layout(uint32_t itopk, uint32_t dim, uint32_t cmax,
                                                             uint32_t search_width, uint32_t hash_bitlen,
-                                                            bool hash_in_lds, bool split_merge) {
+                                                            bool hash_in_lds) {
     SearchLdsLayout l;
     uint32_t off = 0;
     auto take = [&](uint32_t bytes) {
@@ -76,9 +72,41 @@ __host__ __device__ inline SearchLdsLayout search_lds_layout(uint32_t itopk, uin
     l.off_surv = take(cmax * 4);
     l.off_parents = take(search_width * 4);
     l.off_misc = take(16 * 4);
-    // split merge: per candidate one count per list part and one for the queue, per queue entry one count per list part
-    l.off_parts = take(split_merge ? ((kMergeChunks + 1u) * cmax + kMergeChunks * itopk) * 4u : 0u);
     l.off_hash = take(hash_in_lds ? (1u << hash_bitlen) * 4u : 0u);
+    l.total = off;
+    return l;
+}
+
+// layout of the small-batch kernel
+struct SearchSmallLdsLayout {
+    uint32_t off_query, off_top, off_open, off_marked, off_ahead, off_cand, off_surv, off_parents, off_misc, off_hash, total;
+};
+constexpr uint32_t kSmallMaxItopk = 1024;
+constexpr uint32_t kSmallBatchQueries = 256;  // CUs
+// queue places: whole blocks of 64, and as many of them as the kernel's merge reads (1, 2, 4 or 16)
+__host__ __device__ inline uint32_t search_small_padded_queue(uint32_t itopk) {
+    return itopk <= 64 ? 64u : itopk <= 128 ? 128u : itopk <= 256 ? 256u : 1024u;
+}
+__host__ __device__ inline SearchSmallLdsLayout search_small_lds_layout(uint32_t itopk, uint32_t dim, uint32_t cmax, uint32_t search_width,
+                                                                       uint32_t table_bitlen) {
+    SearchSmallLdsLayout l;
+    uint32_t off = 0;
+    auto take = [&](uint32_t bytes) {
+        uint32_t o = off;
+        off += (bytes + 15u) & ~15u;
+        return o;
+    };
+    const uint32_t queue = search_small_padded_queue(itopk);
+    l.off_query = take(dim * 4);
+    l.off_top = take(queue * 16);
+    l.off_open = take(queue * 4);
+    l.off_marked = take(kSmallMaxItopk / 8);
+    l.off_ahead = take((2u * search_width + 16u) * 8u);
+    l.off_cand = take((cmax + 64u) * 8u);  // the list is read up to 64 keys at a time
+    l.off_surv = take(cmax * 4);
+    l.off_parents = take(search_width * 4);
+    l.off_misc = take(16 * 4);
+    l.off_hash = take((1u << table_bitlen) * 4u);
     l.total = off;
     return l;
 }
@@ -113,6 +141,7 @@ __host__ __device__ inline SearchWaveLdsLayout search_wave_lds_layout(uint32_t i
 constexpr uint32_t kMaxLdsBytes = 160 * 1024;
 
 int launch_search(const SearchArgs& a, int metric, int filter, size_t lds_bytes, hipStream_t stream);
+int launch_search_small(const SearchArgs& a, int metric, int filter, size_t lds_bytes, hipStream_t stream);
 int launch_search_wave(const SearchArgs& a, int metric, int filter, size_t lds_bytes, hipStream_t stream);
 
 // grab_search_ex_static: slots (uint32) of the array in the device image that holds its visited sets, 32 MiB

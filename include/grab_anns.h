@@ -54,7 +54,7 @@ extern "C" {
 /* Work decomposition of the search.  Default: one 64-lane wave per query when the batch is
  * large enough to fill the device that way (>= 1024 queries) and a wave needs at most 20 KB
  * of LDS (a visited set of up to 4096 slots), else one workgroup per query (256 threads;
- * 1024 for batches of up to 256 queries).  Both give identical results. */
+ * 1024 for batches of up to 256 queries, 512 for up to 512).  All give identical results. */
 #define GRAB_FLAG_WAVE_PER_QUERY 4u
 #define GRAB_FLAG_BLOCK_PER_QUERY 8u
 
@@ -99,7 +99,7 @@ uint32_t grab_queue_capacity(uint32_t itopk, uint32_t search_width, uint32_t deg
 size_t grab_reference_smem_bytes(uint32_t itopk, uint32_t dim, uint32_t search_width,
                                  uint32_t degree, uint32_t hash_bitlen);
 /* LDS bytes that this library's workgroup-per-query search kernel uses for the same parameters on batches of more
- * than 256 queries (smaller batches add the scratch of their split merge when it fits beside queue and visited set) */
+ * than 512 queries (smaller batches use up to twice as much) */
 size_t grab_search_lds_bytes(uint32_t itopk, uint32_t dim, uint32_t search_width,
                              uint32_t degree, uint32_t n_seeds, uint32_t hash_bitlen);
 
