@@ -130,11 +130,11 @@ __global__ void __launch_bounds__(256) scatter_results_kernel(const int64_t* __r
     out_dist[at] = dist[i];
 }
 
-// The same walk for the scan of id intervals: one wave per tile-grid row of a dense matrix whose rows start at the first
-// column tile of their row tile (sched holds it).  The kk (<= 64) smallest (distance, column) keys of the row's columns
-// [lo, hi) go to keys[query][kk] in ascending order; rows that admit no column are padding.
-__global__ void __launch_bounds__(256) stream_select_keys_kernel(const float* __restrict__ dense, uint64_t pitch,
-                                                                 const uint32_t* __restrict__ row_query, const uint32_t* __restrict__ row_lo,
+// The same walk for the exact scans: one wave per tile-grid row of the distances that the contraction left, a row tile as
+// wide as its sweep (sched holds where it starts, in the matrix and among the columns).  The kk (<= 64) smallest
+// (distance, column) keys of the row's columns [lo, hi) go to keys[query][kk] in ascending order, or to keys[row][kk]
+// without row_query; rows that admit no column are padding.
+__global__ void __launch_bounds__(256) stream_select_keys_kernel(const float* __restrict__ dense, const uint32_t* __restrict__ row_query, const uint32_t* __restrict__ row_lo,
                                                                  const uint32_t* __restrict__ row_hi, const uint32_t* __restrict__ sched,
                                                                  uint32_t nrows, uint32_t kk, uint64_t* __restrict__ out_keys) {
     const int lane = threadIdx.x & 63;
@@ -143,7 +143,9 @@ __global__ void __launch_bounds__(256) stream_select_keys_kernel(const float* __
     const uint32_t c_lo = row_lo[row], c_hi = row_hi[row];
     if (c_lo >= c_hi) return;
     const uint32_t base = sched[kSchedLo + row / TM] * TN;  // <= c_lo: the row tile's sweep starts at or before every interval of its rows
-    const float* drow = dense + (size_t)row * pitch;
+    const uint32_t tile = row / TM;
+    const uint32_t pitch = (sched[kSchedHi + tile] - sched[kSchedLo + tile]) * TN;
+    const float* drow = dense + (size_t)sched[kSchedBase + tile] * (TM * TN) + (size_t)(row % TM) * pitch;
     uint64_t mykey = kInvalidKey, thr = kInvalidKey;
     float thr_d = __builtin_inff();
     auto offer = [&](uint64_t key) {  // every lane calls this with its own key
@@ -221,7 +223,7 @@ __global__ void __launch_bounds__(256) stream_select_keys_kernel(const float* __
         cur0 = nxt0;
         cur1 = nxt1;
     }
-    if ((uint32_t)lane < kk) out_keys[(size_t)row_query[row] * kk + lane] = mykey;
+    if ((uint32_t)lane < kk) out_keys[(size_t)(row_query ? row_query[row] : row) * kk + lane] = mykey;
 }
 
 constexpr uint32_t kScanPiece = 128 * TN;  // columns of one piece of a bucket: a work item sweeps at most this many
@@ -239,8 +241,8 @@ struct ScanRows {
     std::vector<uint32_t> list_off, lists;             // per query: its tile-grid rows
     uint32_t rows = 0;
     double tiles = 0.0;                                // (row tile, column tile) pairs that the sweep visits
+    std::vector<uint32_t> tile_lo, tile_hi;            // per row tile the column tiles [lo, hi) that its rows admit
     bool one_row_per_query = false;                    // id intervals: row tiles in the order of the intervals' starts
-    std::vector<uint32_t> tile_lo, tile_hi;            // ... and per row tile the column tiles [lo, hi) that its rows admit
 };
 
 void scan_rows(const uint64_t* h_bucket_offsets, uint32_t num_buckets, const uint64_t* h_masks, size_t num_queries, ScanRows* out) {
@@ -282,8 +284,14 @@ void scan_rows(const uint64_t* h_bucket_offsets, uint32_t num_buckets, const uin
                 r.lists[at[q]++] = row;
             }
         }
-    for (size_t pc = 0; pc < r.pieces.size(); ++pc)
-        r.tiles += (double)((r.piece_row0[pc + 1] - r.piece_row0[pc]) / TM) * ((r.pieces[pc].hi + TN - 1) / TN - r.pieces[pc].lo / TN);
+    for (size_t pc = 0; pc < r.pieces.size(); ++pc) {
+        const uint32_t lo = r.pieces[pc].lo / TN, hi = (r.pieces[pc].hi + TN - 1) / TN;
+        for (uint32_t row = r.piece_row0[pc]; row < r.piece_row0[pc + 1]; row += TM) {
+            r.tiles += hi - lo;
+            r.tile_lo.push_back(lo);
+            r.tile_hi.push_back(hi);
+        }
+    }
 }
 
 // Id intervals instead of buckets: a query is one tile-grid row whose admissible columns are its interval.  The queries
@@ -447,11 +455,13 @@ void dense_sched(const uint32_t* tile_lo, const uint32_t* tile_hi, uint32_t row_
             per = cand;
         }
     }
-    uint32_t acc = 0;
+    uint32_t acc = 0, tiles = 0;
     for (uint32_t t = 0; t < row_tiles; ++t) {
         sched[kSchedOff + t] = acc;
         sched[kSchedLo + t] = tile_lo[t];
         sched[kSchedHi + t] = tile_hi[t];
+        sched[kSchedBase + t] = tiles;
+        tiles += tile_hi[t] - tile_lo[t];
         acc += (tile_hi[t] - tile_lo[t] + per - 1) / per;
     }
     sched[kSchedOff + row_tiles] = acc;
@@ -485,45 +495,46 @@ int scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const Sc
     GRAB_HIP(hipDeviceGetAttribute(&num_cu, hipDeviceAttributeMultiprocessorCount, dev));
     const uint32_t kk = std::max<uint32_t>(2 * k + 32, 64);  // <= 288
     const uint32_t row_tiles = rows / TM, col_tiles = (uint32_t)((num_dataset + TN - 1) / TN), target = (uint32_t)num_cu * 2;
-    // enough work items for every workgroup of the grid, and no more: an item ends with a selection over each of its
-    // 128 rows, which costs as much as several tile steps (1M x 768, 10,000 queries: 2 splits 6.9 ms, 5 splits 8.2 ms)
-    const uint32_t splits = std::max(1u, std::min({(target + row_tiles - 1) / row_tiles, 8u, 1024u / kk}));
     // a prepared base has paid for its split rows; otherwise splitting a million rows pays from a thousand query rows on
     const bool split = base ? base->split
                             : knn_bf16_allowed() && dim % KC == 0 && rows >= 1024 && num_dataset >= 4096;
     DeviceScratch d_tab, buf, cand, merged, outside, norm_a, norm_b, split_a, split_b, mean, doubt;
-    const uint32_t grid = std::min(row_tiles * splits, target);
-    // Id intervals with short candidate lists go the dense way: the contraction writes the distances of the columns
-    // that a row tile sweeps, a streaming pass per query keeps the kk smallest of the query's interval.  (The
-    // thresholds of the other way start open for every row and tighten over the first hundreds of admitted columns,
-    // which is most of a narrow interval: its tiles spend their time appending and compacting.)  In passes of at most
-    // 128 row tiles whose distances fit kDenseCap bytes.
-    constexpr uint64_t kDenseCap = 4ull << 30;
+    // Short candidate lists (k <= 16) go the dense way: the contraction writes the distances of the columns that a row tile
+    // sweeps, in work items of equal length, and a streaming pass keeps the kk smallest of every row.  The other way
+    // selects inside the contraction: its thresholds start open for every row and tighten over the first hundreds of
+    // admitted columns - most of a narrow interval, and again in every item that a long sweep is cut into, so sweeps are
+    // cut only until every workgroup has an item and the longest one sets the time.  4999 queries with 1-4 of 64 buckets
+    // on 200k x 768 (mean sweep 23 column tiles, longest 128): 2.70 -> 0.35 ms of contraction, 0.16 ms of selection.  In
+    // passes of at most 128 row tiles whose distances fit a bound: for buckets what the buffers of the other way would take.
+    const uint64_t dense_cap = rw.one_row_per_query ? 4ull << 30 : (uint64_t)target * TM * CAP * sizeof(uint64_t);
+    constexpr uint64_t kTileBytes = (uint64_t)TM * TN * sizeof(float);
     struct Pass {
         uint32_t t0, t1;
-        uint64_t pitch;
     };
     std::vector<Pass> passes;
-    bool dense_way = rw.one_row_per_query && kk <= 64;
-    if (dense_way) {
-        for (uint32_t t0 = 0; t0 < row_tiles && dense_way;) {
-            uint32_t t1 = t0;
-            uint64_t width = 0;
-            while (t1 < row_tiles && t1 - t0 < 128) {
-                const uint64_t w = std::max<uint64_t>(width, rw.tile_hi[t1] - rw.tile_lo[t1]);
-                if ((uint64_t)(t1 + 1 - t0) * TM * w * TN * 4 > kDenseCap) break;
-                width = w;
-                ++t1;
-            }
-            if (t1 == t0) dense_way = false;  // one row tile's sweep alone is beyond the cap
-            passes.push_back({t0, t1, width * TN});
-            t0 = t1;
+    uint64_t dense_bytes = 0;
+    bool dense_way = kk <= 64;
+    for (uint32_t t0 = 0; t0 < row_tiles && dense_way;) {
+        uint32_t t1 = t0;
+        uint64_t bytes = 0;
+        while (t1 < row_tiles && t1 - t0 < 128) {
+            const uint64_t more = (rw.tile_hi[t1] - rw.tile_lo[t1]) * kTileBytes;
+            if (bytes + more > dense_cap) break;
+            bytes += more;
+            ++t1;
         }
+        if (t1 == t0) dense_way = false;  // one row tile's sweep alone is beyond the cap
+        dense_bytes = std::max(dense_bytes, bytes);
+        passes.push_back({t0, t1});
+        t0 = t1;
     }
-    if (!dense_way) {
-        GRAB_HIP(buf.alloc((size_t)grid * TM * CAP * sizeof(uint64_t)));
-        GRAB_HIP(cand.alloc((size_t)rows * splits * kk * sizeof(uint64_t)));
-    }
+    // enough work items for every workgroup of the grid, and no more: an item ends with a selection over each of its
+    // 128 rows, which costs as much as several tile steps (1M x 768, 10,000 queries: 2 splits 6.9 ms, 5 splits 8.2 ms)
+    const uint32_t splits = dense_way ? 1u : std::max(1u, std::min({(target + row_tiles - 1) / row_tiles, 8u, 1024u / kk}));
+    const uint32_t grid = std::min(row_tiles * splits, target);
+    const bool per_query = dense_way && rw.one_row_per_query;  // the selection leaves a query's list, nothing to merge
+    if (!dense_way) GRAB_HIP(buf.alloc((size_t)grid * TM * CAP * sizeof(uint64_t)));
+    if (!per_query) GRAB_HIP(cand.alloc((size_t)rows * splits * kk * sizeof(uint64_t)));
     GRAB_HIP(merged.alloc((size_t)nq * kk * sizeof(uint64_t)));
     GRAB_HIP(outside.alloc((size_t)nq * 4));
     GRAB_HIP(norm_a.alloc((size_t)nq * 4));
@@ -543,12 +554,10 @@ int scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const Sc
     const size_t at_rq = put(rw.row_query.data(), rows), at_lo = put(rw.row_lo.data(), rows), at_hi = put(rw.row_hi.data(), rows);
     const size_t at_loff = put(rw.list_off.data(), rw.list_off.size()), at_lists = put(rw.lists.data(), rw.lists.size());
     size_t at_sched = 0;
-    uint64_t dense_bytes = 0;
     if (dense_way) {
         std::vector<uint32_t> sched(passes.size() * (size_t)kSchedWords, 0u);
         for (size_t pi = 0; pi < passes.size(); ++pi) {
             const Pass& ps = passes[pi];
-            dense_bytes = std::max<uint64_t>(dense_bytes, (uint64_t)(ps.t1 - ps.t0) * TM * ps.pitch * 4);
             dense_sched(rw.tile_lo.data() + ps.t0, rw.tile_hi.data() + ps.t0, ps.t1 - ps.t0, target, sched.data() + pi * kSchedWords);
         }
         at_sched = put(sched.data(), sched.size());
@@ -581,7 +590,7 @@ int scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const Sc
     const uint32_t* d_lists = d_tab.as<uint32_t>() + at_lists;
     const uint32_t* d_sched_all = d_tab.as<uint32_t>() + at_sched;
     {
-        const size_t fill = dense_way ? (size_t)nq * kk : 0;  // the dense way: a query without a row keeps an empty list
+        const size_t fill = per_query ? (size_t)nq * kk : 0;  // a query without a row keeps an empty list
         hipLaunchKernelGGL(scan_init_kernel, dim3((uint32_t)std::min<size_t>(std::max<size_t>((fill + 255) / 256, 1), 1024)), dim3(256), 0, st,
                            doubt.as<uint32_t>(), nq, n_counters, merged.as<uint64_t>(), fill);
         GRAB_HIP(hipGetLastError());
@@ -650,15 +659,14 @@ int scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const Sc
             tp.row_tiles = ps.t1 - ps.t0;
             tp.nsplit = 1;
             tp.dense = dense.as<float>();
-            tp.dense_pitch = ps.pitch;
             tp.dense_rel = 1;
             tp.sched = d_sched_all + pi * kSchedWords;
             tp.work_counter = pi < n_counters ? doubt.as<uint32_t>() + nq + 3 + pi : nullptr;
             rc = launch_tile_store(tp, metric, target, st, split);
             if (rc != GRAB_OK) break;
-            hipLaunchKernelGGL(stream_select_keys_kernel, dim3((tp.M + 3) / 4), dim3(256), 0, st, dense.as<float>(), ps.pitch,
-                               tp.row_perm, d_lo + (size_t)ps.t0 * TM, d_hi + (size_t)ps.t0 * TM, tp.sched,
-                               tp.M, kk, merged.as<uint64_t>());
+            hipLaunchKernelGGL(stream_select_keys_kernel, dim3((tp.M + 3) / 4), dim3(256), 0, st, dense.as<float>(),
+                               per_query ? tp.row_perm : nullptr, tp.row_lo, tp.row_hi, tp.sched, tp.M, kk,
+                               per_query ? merged.as<uint64_t>() : cand.as<uint64_t>() + (size_t)ps.t0 * TM * kk);
             if (hipGetLastError() != hipSuccess) {
                 set_error("scan: select kernel launch failed");
                 rc = GRAB_ERR_HIP;
@@ -686,7 +694,7 @@ int scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const Sc
     const double flop = rw.tiles * 2.0 * TM * TN * dim;
     if (split) knn_stats().flop_bf16 = 3.0 * flop;  // three instructions a product
     else knn_stats().flop = flop;
-    if (!dense_way)
+    if (!per_query)
         hipLaunchKernelGGL(premerge_lists_kernel, dim3((nq + 3) / 4), dim3(256), 0, st, cand.as<uint64_t>(), splits, kk, d_loff, d_lists, nq,
                            merged.as<uint64_t>(), outside.as<float>());
     RefineArgs r{};
@@ -703,7 +711,7 @@ int scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const Sc
     r.normA = norm_a.as<float>();
     r.max_normB = d_max_norm_b;
     r.sorted = 1;
-    r.outside_in = dense_way ? nullptr : outside.as<float>();  // the dense way leaves one whole list per query: its last key is the bound
+    r.outside_in = per_query ? nullptr : outside.as<float>();  // one whole list per query: its last key is the bound
     r.doubt = doubt.as<uint32_t>();
     if (split) {
         r.split_normA = norm_a.as<float>();

@@ -103,7 +103,7 @@ __global__ void __launch_bounds__(256, 2) tile_topk_kernel(const TileArgs a) {
     // STORE: the work list (items of `per` column tiles, all non-empty) lives in LDS that the
     // selection path would use for thresholds and filter words
     uint32_t* item_off = reinterpret_cast<uint32_t*>(s.thr);  // [row_tiles+1]
-    uint32_t* tile_rng = reinterpret_cast<uint32_t*>(s.cfw);  // [0..127] first, [128..255] end column tile
+    uint32_t* tile_rng = reinterpret_cast<uint32_t*>(s.cfw);  // [0..127] first, [128..255] end column tile, [256..383] tiles before
     uint32_t nwork = a.row_tiles * a.nsplit, per_item = 0;
     if (STORE) {
         per_item = a.sched[kSchedPer];
@@ -112,6 +112,7 @@ __global__ void __launch_bounds__(256, 2) tile_topk_kernel(const TileArgs a) {
         if (tid < (int)a.row_tiles) {
             tile_rng[tid] = a.sched[kSchedLo + tid];
             tile_rng[128 + tid] = a.sched[kSchedHi + tid];
+            if (a.dense_rel) tile_rng[256 + tid] = a.sched[kSchedBase + tid];
         }
     }
 
@@ -350,7 +351,14 @@ __global__ void __launch_bounds__(256, 2) tile_topk_kernel(const TileArgs a) {
                             T[(i * 32 + (v & 3) + 4 * half + 8 * (v >> 2)) * TSTRIDE + jx * 32 + l32] = acc[i][jx][v];
                 const int c4 = lane & 15, rsub = lane >> 4;
                 const uint32_t gcol = col0 + wc * 64 + c4 * 4;
-                const uint32_t dcol = gcol - (a.dense_rel ? tile_rng[rt] * TN : 0u);
+                uint32_t dcol = gcol;
+                uint64_t pitch = a.dense_pitch;
+                float* drows = a.dense + (size_t)row0 * pitch;
+                if (a.dense_rel) {
+                    dcol -= tile_rng[rt] * TN;
+                    pitch = (tile_rng[128 + rt] - tile_rng[rt]) * TN;
+                    drows = a.dense + (size_t)tile_rng[256 + rt] * (TM * TN);
+                }
                 float4 nb = make_float4(0.f, 0.f, 0.f, 0.f);
                 if (METRIC == kMetricL2) {
                     if (gcol + 3 < a.N) {
@@ -382,10 +390,9 @@ __global__ void __launch_bounds__(256, 2) tile_topk_kernel(const TileArgs a) {
                         d = make_float4(-t.x, -t.y, -t.z, -t.w);
                     }
                     // the pitch is a whole number of tiles: columns past N are written and never read
-                    const uint32_t grow = row0 + wr * 64 + r;
-                    bool wanted = grow < a.M;
+                    bool wanted = row0 + wr * 64 + r < a.M;
                     if (a.dense_rel) wanted = wanted && gcol < (uint32_t)s.fb[wr * 64 + r] && gcol + 4u > (uint32_t)s.fa[wr * 64 + r];
-                    if (wanted) *reinterpret_cast<float4*>(a.dense + (size_t)grow * a.dense_pitch + dcol) = d;
+                    if (wanted) *reinterpret_cast<float4*>(drows + (size_t)(wr * 64 + r) * pitch + dcol) = d;
                 }
                 __syncthreads();  // the block is consumed before the next chunk lands in the tile buffers
                 continue;

@@ -15,7 +15,7 @@ constexpr int CAP = 1024;                 // per-row candidate buffer (keys)
 constexpr int COMPACT_AT = CAP - TN;      // a tile appends at most TN keys to a row
 // layout of the work list of the dense-store mode (uint32 words)
 constexpr int kSchedPer = 0, kSchedItems = 1, kSchedOff = 2, kSchedLo = kSchedOff + 129, kSchedHi = kSchedLo + 128,
-              kSchedWords = kSchedHi + 128;
+              kSchedBase = kSchedHi + 128, kSchedWords = kSchedBase + 128;
 
 struct TileArgs {
     const float* A;
@@ -32,7 +32,9 @@ struct TileArgs {
     const uint32_t* row_hi;
     float* dense;        // STORE mode: [M][dense_pitch] distances
     uint64_t dense_pitch;
-    int dense_rel;       // STORE mode: a row's distances start at the first column tile of its row tile, not at column 0
+    // STORE mode: a row tile is a matrix of its own, as wide as its sweep; they follow each other (sched has the column
+    // tiles before each), dense_pitch is not used, and only columns that a row admits are written
+    int dense_rel;
     const uint32_t* sched;  // STORE mode: work list made by bucket_order_kernel
     uint64_t* buf;       // [gridDim.x][TM][CAP]
     uint64_t* cand_out;  // [M][nsplit*kk]

@@ -26,6 +26,9 @@ def _case(grab, n, dim, n_buckets, nq, seed, unit, empty=()):
     (20000, 64, 64, 700, 10, 1, True),      # inner product on unit rows, 64 buckets
     (50000, 32, 5, 129, 33, 0, True),       # buckets longer than one piece of 16384 columns, k above 32
     (3000, 768, 64, 64, 10, 1, True),       # the row length of the high-dimensional configuration
+    (50000, 32, 5, 129, 16, 0, False),      # the longest lists that are selected from stored distances: buckets in pieces ...
+    (50000, 32, 5, 129, 17, 0, False),      # ... and the shortest beyond
+    (4200, 32, 64, 5000, 1, 0, False),      # more row tiles than one pass takes, a ragged last column tile
 ])
 def test_bucket_scan_equals_the_cpu_label_scan(oracle, grab, n, dim, n_buckets, nq, k, metric, unit):
     data, labels, q, masks, offsets, _ = _case(grab, n, dim, n_buckets, nq, 7 * n_buckets + dim, unit)
