@@ -934,14 +934,21 @@ __global__ void __launch_bounds__(256) refine_kernel(const RefineArgs a) {
     }
     const float* q = a.A + (size_t)row * a.dim;
     const int grp = lane >> 3, j = lane & 7;
-    for (uint32_t c0 = 0; c0 < n_score; c0 += 8) {
-        const uint32_t c = c0 + grp;
-        const uint64_t kc = c < n_score ? mykeys[c] : kInvalidKey;  // uniform per group of 8 lanes
-        if (kc != kInvalidKey) {
-            const uint32_t id = (uint32_t)(kc & 0xFFFFFFFFull);
-            const float d = group8_distance<METRIC>(q, a.B + (size_t)id * a.dim, a.dim, j);
-            if (j == 0) mykeys[c] = make_sel_key(d, id);
-        }
+    // Bound by the latency of its gathers: two rows per group of 8 lanes at a time, eight 16-byte loads a lane in flight
+    // (one row and what the compiler unrolled before: 1M x 128, k 128: 17.1 -> 13.8 ms; 100,003 x 768: 8.5 -> 8.0 ms)
+    const float4* q4 = reinterpret_cast<const float4*>(q);
+    for (uint32_t c0 = 0; c0 < n_score; c0 += 16) {
+        const uint32_t ca = c0 + grp, cb = ca + 8;
+        const uint64_t ka = ca < n_score ? mykeys[ca] : kInvalidKey, kb = cb < n_score ? mykeys[cb] : kInvalidKey;  // uniform per group
+        if (ka == kInvalidKey && kb == kInvalidKey) continue;
+        const uint32_t ia = (uint32_t)((ka != kInvalidKey ? ka : kb) & 0xFFFFFFFFull), ib = (uint32_t)((kb != kInvalidKey ? kb : ka) & 0xFFFFFFFFull);
+        float da = 0.0f, db = 0.0f;
+        fold_rows_any<METRIC, true>(reinterpret_cast<const float4*>(a.B + (size_t)ia * a.dim), reinterpret_cast<const float4*>(a.B + (size_t)ib * a.dim),
+                                    q4, j, a.dim >> 2, da, db);
+        da = group8_sum(da);
+        db = group8_sum(db);
+        if (j == 0 && ka != kInvalidKey) mykeys[ca] = make_sel_key(METRIC == kMetricIP ? -da : da, ia);
+        if (j == 0 && kb != kInvalidKey) mykeys[cb] = make_sel_key(METRIC == kMetricIP ? -db : db, ib);
     }
     __builtin_amdgcn_wave_barrier();
     uint64_t k[NPL];
