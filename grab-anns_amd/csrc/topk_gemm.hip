@@ -243,11 +243,14 @@ __global__ void __launch_bounds__(256, 2) tile_topk_kernel(const TileArgs a) {
             for (int i = 0; i < 4; ++i)
                 pa[i] = reinterpret_cast<const float4*>(a.A + (size_t)s.arow[(tid >> 3) + 32 * i] * a.dim) + (tid & 7);
         }
-        if (ct_begin < ct_end) load_chunk(ra, rb, ct_begin * TN, 0);
+        // Symmetric pass: from the last column tile down to the diagonal, so that workgroups that start together read the
+        // same columns at about the same time and share them in L2 (100,003 x 768, inner product: 33.9 -> 31.7 ms)
+        auto tile_at = [&](uint32_t at) { return FILTER == kFilterSymmetric ? ct_end - 1u - (at - ct_begin) : at; };
+        if (ct_begin < ct_end) load_chunk(ra, rb, tile_at(ct_begin) * TN, 0);
         int buf = 0;
 
-        for (uint32_t ct = ct_begin; ct < ct_end; ++ct) {
-            const uint32_t col0 = ct * TN;
+        for (uint32_t at = ct_begin; at < ct_end; ++at) {
+            const uint32_t ct = tile_at(at), col0 = ct * TN;
             v16f acc[2][2];  // written by the first chunk (kchunks >= 1: dim >= 4)
 
             // one chunk: `xa`, `xb` hold it; the next chunk takes their place once they are parked in LDS
@@ -259,10 +262,10 @@ __global__ void __launch_bounds__(256, 2) tile_topk_kernel(const TileArgs a) {
                     *reinterpret_cast<float4*>(&s.As[buf][r][c4 * 4]) = xa[i];
                     *reinterpret_cast<float4*>(&s.Bs[buf][r][c4 * 4]) = xb[i];
                 }
-                if (STORE && ct == ct_begin && kc == 0 && tid < TM) s.na[tid] = na_pending;
+                if (STORE && at == ct_begin && kc == 0 && tid < TM) s.na[tid] = na_pending;
                 __syncthreads();
                 if (kc + 1 < kchunks) load_chunk(xa, xb, col0, kc + 1);
-                else if (ct + 1 < ct_end) load_chunk(xa, xb, col0 + TN, 0);
+                else if (at + 1 < ct_end) load_chunk(xa, xb, tile_at(at + 1) * TN, 0);
                 // lanes 0-31 take k = 0..15 of the chunk, lanes 32-63 take k = 16..31: any
                 // assignment of k to the two MFMA k-slots gives the same sum
                 const float* pa0 = &s.As[buf][wr * 64 + l32][half * 16];
