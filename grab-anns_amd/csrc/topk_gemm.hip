@@ -91,6 +91,17 @@ __device__ __forceinline__ void compact_row(Lds& s, uint64_t* rowbuf, int r, uin
 // lo.hi + hi.lo + hi.hi with fp32 sums - 24 instructions a chunk where the fp32 path issues 64 that take twice as
 // long each - off the true dot product by at most 3 * 2^-16 |a||b|.  What such a pass returns are candidates; the
 // exact re-scoring and the check after it (refine_kernel, which is told the larger error) decide the result.
+// Symmetric pass with sweeps in slices: the slice that holds the diagonal leaves the row's own list, any other slice its
+// keys - all within the row's bound, like the keys that column walks leave - in the row's list in device memory.  One wave.
+__device__ __forceinline__ void keys_to_column_list(const TileArgs& a, uint32_t row, const uint64_t* keys, uint32_t n, int lane) {
+    if (n == 0) return;  // wave-uniform
+    uint32_t at = 0;
+    if (lane == 0) at = atomicAdd(&a.col_count[row], n);
+    at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+    for (uint32_t g = lane; g < n; g += 64)
+        if (at + g < a.col_cap) a.col_list[(size_t)row * a.col_cap + at + g] = keys[g];
+}
+
 template <int METRIC, int FILTER, bool STORE, bool SPLIT = false>
 // two waves per SIMD: keeps the 64 accumulator registers plus the epilogue under 256 VGPRs
 __global__ void __launch_bounds__(256, 2) tile_topk_kernel(const TileArgs a) {
@@ -142,8 +153,14 @@ __global__ void __launch_bounds__(256, 2) tile_topk_kernel(const TileArgs a) {
             rt = lo_rt;
             sp = work - item_off[rt];
         } else {
-            rt = work / a.nsplit;
-            sp = work - rt * a.nsplit;
+            if (FILTER == kFilterSymmetric) {  // slice by slice from the last columns down
+                sp = work / a.row_tiles;
+                rt = work - sp * a.row_tiles;
+                if (rt + sp * a.tiles_per_split >= a.col_tiles) continue;  // workgroup-uniform: the slice lies below the diagonal
+            } else {
+                rt = work / a.nsplit;
+                sp = work - rt * a.nsplit;
+            }
         }
         const uint32_t row0 = rt * TM;
 
@@ -182,7 +199,10 @@ __global__ void __launch_bounds__(256, 2) tile_topk_kernel(const TileArgs a) {
         }
         uint32_t ct_begin = sp * a.tiles_per_split;
         uint32_t ct_end = min(a.col_tiles, ct_begin + a.tiles_per_split);
-        if (FILTER == kFilterSymmetric) ct_begin = max(ct_begin, rt);  // the tiles below the diagonal are mirrored ones
+        if (FILTER == kFilterSymmetric) {  // the tiles below the diagonal are mirrored ones
+            ct_end = a.col_tiles - sp * a.tiles_per_split;
+            ct_begin = max(rt, ct_end > a.tiles_per_split ? ct_end - a.tiles_per_split : 0u);
+        }
         if (STORE) {
             ct_begin = tile_rng[rt] + sp * per_item;
             ct_end = min(tile_rng[128 + rt], ct_begin + per_item);
@@ -528,7 +548,12 @@ __global__ void __launch_bounds__(256, 2) tile_topk_kernel(const TileArgs a) {
             if (s.cnt[r] > a.kk) compact_row(s, rowbuf, r, a.kk, lane);
             __threadfence_block();
             const uint32_t n = s.cnt[r];
-            uint64_t* out = a.cand_out + ((size_t)(a.cand_by_grid_row ? row0 + r : s.arow[r]) * a.nsplit + sp) * a.kk;
+            if (FILTER == kFilterSymmetric && ct_begin != rt) {
+                keys_to_column_list(a, row0 + r, rowbuf, n, lane);
+                continue;
+            }
+            const uint32_t slot = FILTER == kFilterSymmetric ? 0u : sp, slots = FILTER == kFilterSymmetric ? 1u : a.nsplit;
+            uint64_t* out = a.cand_out + ((size_t)(a.cand_by_grid_row ? row0 + r : s.arow[r]) * slots + slot) * a.kk;
             for (uint32_t g = lane; g < a.kk; g += 64) out[g] = g < n ? rowbuf[g] : kInvalidKey;
         }
     }
@@ -587,18 +612,22 @@ __global__ void __launch_bounds__(64 * kSplitWaves, 2) sym_split_kernel(const Ti
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t wr = wave, half = lane >> 5, l32 = lane & 31;
     uint64_t* myBuf = a.buf + (size_t)blockIdx.x * TM * CAP;
-    const uint32_t nwork = a.row_tiles;
+    const uint32_t nwork = a.row_tiles * a.nsplit;
 
     __shared__ uint32_t next_item;
     for (;;) {
-        // row tile rt sweeps the column tiles from rt on, so the items shrink with rt: handed out in that order, the
-        // largest first, to whichever workgroup is free (the two workgroups of a CU do not run at the same pace)
+        // row tile rt sweeps the column tiles from rt on, in one slice or several (symmetric_slice): handed out slice by
+        // slice from the last columns down, whole slices before the rests, to whichever workgroup is free (the two
+        // workgroups of a CU do not run at the same pace)
         __syncthreads();  // the item before is fully drained
         if (tid == 0) next_item = atomicAdd(a.work_counter, 1u);
         __syncthreads();
         const uint32_t work = next_item;
         if (work >= nwork) break;  // workgroup-uniform
-        const uint32_t rt = work, row0 = rt * TM;
+        const uint32_t sp = work / a.row_tiles, rt = work - sp * a.row_tiles, row0 = rt * TM;
+        if (rt + sp * a.tiles_per_split >= a.col_tiles) continue;  // workgroup-uniform: the slice lies below the diagonal
+        const uint32_t ct_end = a.col_tiles - sp * a.tiles_per_split;
+        const uint32_t ct_begin = max(rt, ct_end > a.tiles_per_split ? ct_end - a.tiles_per_split : 0u);
         if (tid < TM) {
             const uint32_t row = row0 + tid;
             const bool valid = row < a.M;
@@ -626,7 +655,7 @@ __global__ void __launch_bounds__(64 * kSplitWaves, 2) sym_split_kernel(const Ti
         // moves piece lane & 31 of columns 16 w + (lane >> 5) + 2 i, i = 0..7 - addresses that differ by constants -
         // and the first 16 lanes the norms of one column each.  No look at n: the rows are followed by rows of zeros
         // up to a whole tile, and what such a column yields is never kept.
-        const uint32_t steps = 2u * (a.col_tiles - rt);
+        const uint32_t steps = 2u * (ct_end - ct_begin);
         const uint32_t g_lane = (16u * wave + half) * (kSplitRow * 2u) + 16u * l32, g_norm = (16u * wave + (lane & 15u)) * (kSplitRow * 2u) + 512u;
         const uint32_t l_lane = (16u * wave + half) * kSplitPitch + 16u * l32, l_norm = (16u * wave + (lane & 15u)) * kSplitPitch + 512u;
         const bool ninth = lane < 16u;
@@ -657,9 +686,9 @@ __global__ void __launch_bounds__(64 * kSplitWaves, 2) sym_split_kernel(const Ti
             *reinterpret_cast<uint4*>(dst + 7 * kL) = p7;
             if (ninth) *reinterpret_cast<uint4*>(&s.b[buf][l_norm]) = p8;
         };
-        // a step takes half a column tile: the tiles from the last one down to the diagonal, each its low half first.
+        // a step takes half a column tile: the tiles of the slice from the last one down, each its low half first.
         // (Past the end of the sweep the last columns are fetched once more, into the buffer nobody reads.)
-        auto tile_of = [&](uint32_t step) { return a.col_tiles - 1u - (min(step, steps - 1u) >> 1); };
+        auto tile_of = [&](uint32_t step) { return ct_end - 1u - (min(step, steps - 1u) >> 1); };
         auto cols_of = [&](uint32_t step) { return tile_of(step) * TN + kSplitCols * (min(step, steps - 1u) & 1u); };
         fetch_early(cols_of(0));
         fetch_late(cols_of(0));
@@ -825,6 +854,10 @@ __global__ void __launch_bounds__(64 * kSplitWaves, 2) sym_split_kernel(const Ti
             if (s.cnt[r] > a.kk) compact_row_split(s, rowbuf, (int)r, a.kk, (int)lane);
             __threadfence_block();
             const uint32_t n = s.cnt[r];
+            if (ct_begin != rt) {
+                keys_to_column_list(a, row0 + r, rowbuf, n, (int)lane);
+                continue;
+            }
             uint64_t* out = a.cand_out + (size_t)(row0 + r) * a.kk;
             for (uint32_t g = lane; g < a.kk; g += 64) out[g] = g < n ? rowbuf[g] : kInvalidKey;
         }
@@ -833,7 +866,7 @@ __global__ void __launch_bounds__(64 * kSplitWaves, 2) sym_split_kernel(const Ti
 
 int launch_sym_split(const TileArgs& a, const uint16_t* rows, uint32_t grid, hipStream_t stream) {
     static_assert(sizeof(SplitLds) <= 80 * 1024, "two workgroups per CU");
-    GRAB_REQUIRE(a.nsplit == 1 && a.M == a.N && a.dim <= 128 && a.row_tiles == a.col_tiles && a.work_counter, "internal: shape of the bf16 symmetric pass");
+    GRAB_REQUIRE(a.nsplit >= 1 && a.nsplit * a.tiles_per_split >= a.col_tiles && a.M == a.N && a.dim <= 128 && a.row_tiles == a.col_tiles && a.work_counter, "internal: shape of the bf16 symmetric pass");
     GRAB_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(sym_split_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(SplitLds)));
     hipLaunchKernelGGL(sym_split_kernel, dim3(grid), dim3(64 * kSplitWaves), sizeof(SplitLds), stream, a, rows);
     GRAB_HIP(hipGetLastError());
@@ -1109,8 +1142,8 @@ __global__ void __launch_bounds__(256) column_bound_kernel(const uint64_t* __res
     bound[row] = worst == kInvalidKey ? __builtin_inff() : ord_float((uint32_t)(worst >> 32));
 }
 
-// One wave per row: the row's own list (the kk best among the columns from its diagonal tile on) and the keys that
-// column walks left for it (columns before that tile) become the kk best of all columns.  That is certain when at
+// One wave per row: the row's own list (the kk best among the columns from its diagonal tile on, or of the first slice of
+// them) and the keys that column walks (columns before that tile) and other slices left for it become the kk best of all columns.  That is certain when at
 // least kk keys at or below the row's bound are at hand: every key at or below the bound is, on either side.  Rows
 // for which it is not (too few such keys, or more than the lists hold) are listed and redone by the plain pass.
 __global__ void __launch_bounds__(256) merge_symmetric_kernel(uint64_t* __restrict__ cand, const uint64_t* __restrict__ col_list,
@@ -1379,6 +1412,17 @@ void launch_split_rows_chunked(const float* data, uint64_t n, uint32_t dim, cons
     hipLaunchKernelGGL(split_rows_chunked_kernel, dim3((uint32_t)((n * 8 + 255) / 256)), dim3(256), 0, stream, data, n, dim, mean, out, norm);
 }
 
+// Column tiles of a slice of the symmetric pass's sweeps (row tile rt: row_tiles - rt tiles).  Whole sweeps, the longest
+// first, fill `target` workgroups evenly from 2 * target row tiles on (a short sweep follows each long one); below that
+// the first sweep alone outlasts the average, 10,000 rows give 79 workgroups work.  There: slices of a quarter of a
+// workgroup's share, and of four tiles at least (a slice ends with a pass over its 128 rows' lists).  10,000 x 128: pass
+// 2.42 -> 0.55 ms; 50,000 x 128: kNN graph 8.1 -> 5.4 ms; 100,003 x 768, inner product: pass 31.7 -> 28.5 ms.
+uint32_t symmetric_slice(uint32_t row_tiles, uint32_t target) {
+    if (row_tiles >= 2 * target) return row_tiles;
+    const uint64_t total = (uint64_t)row_tiles * (row_tiles + 1) / 2;
+    return std::min(row_tiles, std::max<uint32_t>(4u, (uint32_t)(total / (4ull * target))));
+}
+
 int exact_topk(const TopkProblem& p, hipStream_t stream, float* kernel_ms) {
     GRAB_REQUIRE(p.A && p.B, "null matrix");
     GRAB_REQUIRE(p.dim >= 4 && p.dim % 4 == 0, "unsupported dimension %u (must be a multiple of 4)", p.dim);
@@ -1593,20 +1637,23 @@ int exact_topk(const TopkProblem& p, hipStream_t stream, float* kernel_ms) {
             t.col_count = col_count.as<uint32_t>();
             t.col_cap = kSymColCap;
             t.work_counter = next_counter();
+            TileArgs ts = t;
+            ts.tiles_per_split = symmetric_slice(row_tiles, target);
+            ts.nsplit = (row_tiles + ts.tiles_per_split - 1) / ts.tiles_per_split;
+            const uint32_t sym_grid = std::min(row_tiles * ts.nsplit, target);
             if (bf16_bound) {
                 // where the bounds came from the bf16 pipe (squared L2, up to 128 dimensions) the pass runs there too,
                 // on the split rows the bounding pass left behind: three instructions a product, each at 16x the rate
-                TileArgs ts = t;
                 ts.normA = ts.normB = split_norms;
                 knn_stats().flop = 0.0;
                 const double tile_flop_bf16 = 2.0 * TM * TN * 128;
                 knn_stats().flop_bf16 = 3.0 * tile_flop_bf16 * 0.5 * row_tiles * (row_tiles + 1.0) + tile_flop_bf16 * row_tiles * ((n_sample + TN - 1) / TN);
                 hipLaunchKernelGGL(max_float_kernel, dim3((uint32_t)std::min<size_t>((p.N + 255) / 256, 512)), dim3(256), 0, stream, split_norms, (uint64_t)p.N,
                                    doubt.as<uint32_t>() + p.M + 2);
-                rc = launch_sym_split(ts, split_rows, std::min<uint32_t>(row_tiles, target), stream);
+                rc = launch_sym_split(ts, split_rows, sym_grid, stream);
             } else {
-                rc = p.metric == kMetricIP ? launch_tile<kMetricIP>(t, kFilterSymmetric, grid, stream, split_tiles)
-                                           : launch_tile<kMetricL2>(t, kFilterSymmetric, grid, stream, split_tiles);
+                rc = p.metric == kMetricIP ? launch_tile<kMetricIP>(ts, kFilterSymmetric, sym_grid, stream, split_tiles)
+                                           : launch_tile<kMetricL2>(ts, kFilterSymmetric, sym_grid, stream, split_tiles);
             }
         }
     } else {
