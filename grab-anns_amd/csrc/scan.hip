@@ -130,10 +130,58 @@ __global__ void __launch_bounds__(256) scatter_results_kernel(const int64_t* __r
     out_dist[at] = dist[i];
 }
 
+// The key of lane ^ MASK, without a trip to LDS up to 15.
+template <int MASK>
+__device__ __forceinline__ uint64_t lane_xor_u64(uint64_t v) {
+    const int lo = (int)(uint32_t)v, hi = (int)(uint32_t)(v >> 32);
+    auto dpp = [&](auto ctrl) {
+        constexpr int C = decltype(ctrl)::value;
+        return ((uint64_t)(uint32_t)__builtin_amdgcn_update_dpp(hi, hi, C, 0xF, 0xF, false) << 32) |
+               (uint32_t)__builtin_amdgcn_update_dpp(lo, lo, C, 0xF, 0xF, false);
+    };
+    if constexpr (MASK == 1) return dpp(std::integral_constant<int, 0xB1>{});        // quad_perm 1 0 3 2
+    else if constexpr (MASK == 2) return dpp(std::integral_constant<int, 0x4E>{});   // quad_perm 2 3 0 1
+    else if constexpr (MASK == 3) return dpp(std::integral_constant<int, 0x1B>{});   // quad_perm 3 2 1 0
+    else if constexpr (MASK == 4) return lane_xor_u64<3>(lane_xor_u64<7>(v));
+    else if constexpr (MASK == 7) return dpp(std::integral_constant<int, 0x141>{});  // row_half_mirror
+    else if constexpr (MASK == 8) return dpp(std::integral_constant<int, 0x128>{});  // row_ror 8
+    else if constexpr (MASK == 15) return dpp(std::integral_constant<int, 0x140>{}); // row_mirror
+    else return shfl_xor_u64(v, MASK);
+}
+// lanes that differ in MASK: the one without BIT (the highest of MASK) keeps the smaller key
+template <int MASK, int BIT>
+__device__ __forceinline__ void order_pair(uint64_t& k, int lane) {
+    const uint64_t o = lane_xor_u64<MASK>(k);
+    k = (k < o) == ((lane & BIT) == 0) ? k : o;
+}
+// a run of S lanes that first rises, then falls (or the other way) becomes ascending; S = 2 * BIT
+template <int BIT>
+__device__ __forceinline__ void bitonic_halves(uint64_t& k, int lane) {
+    order_pair<BIT, BIT>(k, lane);
+    if constexpr (BIT > 1) bitonic_halves<BIT / 2>(k, lane);
+}
+template <int SIZE>
+__device__ __forceinline__ void sort_merge_runs(uint64_t& k, int lane) {  // ascending runs of SIZE / 2 lanes to runs of SIZE
+    order_pair<SIZE - 1, SIZE / 2>(k, lane);
+    if constexpr (SIZE > 2) bitonic_halves<SIZE / 4>(k, lane);
+}
+__device__ __forceinline__ void sort_lanes(uint64_t& k, int lane) {  // one key a lane, ascending
+    sort_merge_runs<2>(k, lane);
+    sort_merge_runs<4>(k, lane);
+    sort_merge_runs<8>(k, lane);
+    sort_merge_runs<16>(k, lane);
+    sort_merge_runs<32>(k, lane);
+    sort_merge_runs<64>(k, lane);
+}
+
 // The same walk for the exact scans: one wave per tile-grid row of the distances that the contraction left, a row tile as
 // wide as its sweep (sched holds where it starts, in the matrix and among the columns).  The kk (<= 64) smallest
 // (distance, column) keys of the row's columns [lo, hi) go to keys[query][kk] in ascending order, or to keys[row][kk]
 // without row_query; rows that admit no column are padding.
+// Bound by instruction issue.  What passes the threshold - the list's kk-th key - gathers in LDS and is sorted and merged
+// into the list 64 keys at a time: a threshold that lags lets a few more keys pass (some 64 for every doubling of the
+// columns seen), but a key costs four instructions of a sort instead of the two dozen of an insertion of its own.  10,000
+// intervals of 10,000 columns (0.4 GB): 190 -> 127 us; 200k x 768 in 64 buckets, 16,500 lists: 160 -> 81 us.
 __global__ void __launch_bounds__(256) stream_select_keys_kernel(const float* __restrict__ dense, const uint32_t* __restrict__ row_query, const uint32_t* __restrict__ row_lo,
                                                                  const uint32_t* __restrict__ row_hi, const uint32_t* __restrict__ sched,
                                                                  uint32_t nrows, uint32_t kk, uint64_t* __restrict__ out_keys) {
@@ -146,50 +194,40 @@ __global__ void __launch_bounds__(256) stream_select_keys_kernel(const float* __
     const uint32_t tile = row / TM;
     const uint32_t pitch = (sched[kSchedHi + tile] - sched[kSchedLo + tile]) * TN;
     const float* drow = dense + (size_t)sched[kSchedBase + tile] * (TM * TN) + (size_t)(row % TM) * pitch;
-    uint64_t mykey = kInvalidKey, thr = kInvalidKey;
+    __shared__ uint64_t waiting_all[4][128];
+    uint64_t* waiting = waiting_all[threadIdx.x >> 6];
+    uint32_t nwait = 0;  // wave-uniform, below 64 between offers
+    uint64_t mykey = kInvalidKey;
     float thr_d = __builtin_inff();
-    auto offer = [&](uint64_t key) {  // every lane calls this with its own key
-        uint64_t b = __ballot(key < thr);
-        while (b != 0) {
-            const int bit = (int)__builtin_ctzll(b);
-            b &= b - 1;
-            const uint64_t x = readlane_u64(key, bit);
-            if (x < thr) {  // wave-uniform
-                const uint32_t p = (uint32_t)__popcll(__ballot(mykey < x));
-                const uint64_t up = shfl_up_u64(mykey);
-                if ((uint32_t)lane == p) mykey = x;
-                else if ((uint32_t)lane > p && (uint32_t)lane < kk) mykey = up;
-                thr = readlane_u64(mykey, (int)kk - 1);
-                thr_d = thr == kInvalidKey ? __builtin_inff() : ord_float((uint32_t)(thr >> 32));
-            }
-        }
+    auto merge_waiting = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        uint64_t x = (uint32_t)lane < nwait ? waiting[lane] : kInvalidKey;
+        const uint64_t rest = waiting[64 + lane];
+        sort_lanes(x, lane);
+        const uint64_t o = lane_xor_u64<63>(x);
+        mykey = mykey < o ? mykey : o;  // the 64 smallest of both
+        bitonic_halves<32>(mykey, lane);
+        const uint64_t thr = readlane_u64(mykey, (int)kk - 1);
+        const float d = ord_float((uint32_t)(thr >> 32));
+        thr_d = thr == kInvalidKey || d != d ? __builtin_inff() : d;
+        nwait = nwait > 64u ? nwait - 64u : 0u;
+        __builtin_amdgcn_wave_barrier();
+        if ((uint32_t)lane < nwait) waiting[lane] = rest;
     };
-    // The first 512 columns of the interval at once: eight keys a lane, one sort, the kk smallest a lane each.  (Taken
-    // one by one through `offer` they would nearly all be inserted - the list is empty at first - and an insertion is
-    // a dozen wave-wide steps; after 512 columns one in eight still passes, after 5000 one in eighty.)
-    uint32_t c_from = c_lo;
-    if (c_hi - c_lo >= 512u) {
-        uint64_t r[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const uint32_t c = c_lo + 64u * i + (uint32_t)lane;
-            r[i] = make_sel_key(drow[c - base], c);
-        }
-        dev::wave_bitonic_sort<8>(r);  // ascending, element lane * 8 + i in r[i]
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const uint64_t v = shfl_u64(r[i], lane >> 3);
-            if ((lane & 7) == i) mykey = v;
-        }
-        if ((uint32_t)lane >= kk) mykey = kInvalidKey;
-        thr = readlane_u64(mykey, (int)kk - 1);
-        thr_d = ord_float((uint32_t)(thr >> 32));
-        c_from = c_lo + 512u;
-    }
+    auto offer = [&](bool pass, float d, uint32_t c) {
+        const uint64_t b = __ballot(pass);
+        if (b == 0) return;
+        if (pass) waiting[nwait + (uint32_t)__popcll(b & ((1ull << lane) - 1ull))] = make_sel_key(d, c);
+        nwait += (uint32_t)__popcll(b);
+        if (nwait >= 64u) merge_waiting();
+    };
+    // of an interval of 512 columns and more the first 512 are all candidates, those without an order (NaN) among them
+    const uint32_t c_from = c_hi - c_lo >= 512u ? c_lo + 512u : c_lo;
     // 512 columns per step, two runs of four consecutive columns per lane, the next step's loads issued before this
     // step's values are looked at; steps are aligned to the row's first stored column
     constexpr uint32_t STEP = 512;
-    const uint32_t c_begin = base + ((c_from - base) & ~(STEP - 1));
+    const uint32_t c_begin = base + ((c_lo - base) & ~(STEP - 1));
     const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
     auto load4 = [&](uint32_t c) { return c < c_hi ? *reinterpret_cast<const float4*>(drow + (c - base)) : zero; };
     float4 cur0 = load4(c_begin + 4 * lane), cur1 = load4(c_begin + 256 + 4 * lane);
@@ -201,28 +239,25 @@ __global__ void __launch_bounds__(256) stream_select_keys_kernel(const float* __
         }
         const float dv[8] = {cur0.x, cur0.y, cur0.z, cur0.w, cur1.x, cur1.y, cur1.z, cur1.w};
         const bool interior = c0 >= c_from && c0 + STEP <= c_hi;  // wave-uniform
-        bool any = false;
         if (interior) {
+            bool any = false;
 #pragma unroll
             for (int e = 0; e < 8; ++e) any = any || dv[e] <= thr_d;
+            if (__ballot(any) != 0) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) offer(dv[e] <= thr_d, dv[e], c0 + (e >> 2) * 256 + 4 * lane + (e & 3));
+            }
         } else {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const uint32_t c = c0 + (e >> 2) * 256 + 4 * lane + (e & 3);
-                any = any || (c >= c_from && c < c_hi && dv[e] <= thr_d);
-            }
-        }
-        if (__ballot(any) != 0) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const uint32_t c = c0 + (e >> 2) * 256 + 4 * lane + (e & 3);
-                const bool in = c >= c_from && c < c_hi && dv[e] <= thr_d;
-                offer(in ? make_sel_key(dv[e], c) : kInvalidKey);
+                offer(c >= c_lo && c < c_hi && (dv[e] <= thr_d || (c < c_from && dv[e] != dv[e])), dv[e], c);
             }
         }
         cur0 = nxt0;
         cur1 = nxt1;
     }
+    if (nwait != 0) merge_waiting();
     if ((uint32_t)lane < kk) out_keys[(size_t)(row_query ? row_query[row] : row) * kk + lane] = mykey;
 }
 
@@ -504,7 +539,7 @@ int scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const Sc
     // selects inside the contraction: its thresholds start open for every row and tighten over the first hundreds of
     // admitted columns - most of a narrow interval, and again in every item that a long sweep is cut into, so sweeps are
     // cut only until every workgroup has an item and the longest one sets the time.  4999 queries with 1-4 of 64 buckets
-    // on 200k x 768 (mean sweep 23 column tiles, longest 128): 2.70 -> 0.35 ms of contraction, 0.16 ms of selection.  In
+    // on 200k x 768 (mean sweep 23 column tiles, longest 128): 2.70 -> 0.35 ms of contraction, 0.08 ms of selection.  In
     // passes of at most 128 row tiles whose distances fit a bound: for buckets what the buffers of the other way would take.
     const uint64_t dense_cap = rw.one_row_per_query ? 4ull << 30 : (uint64_t)target * TM * CAP * sizeof(uint64_t);
     constexpr uint64_t kTileBytes = (uint64_t)TM * TN * sizeof(float);

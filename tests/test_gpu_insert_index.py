@@ -46,6 +46,26 @@ def test_insert_large_call_uses_global_sort(oracle, grab):
     assert np.array_equal(d_graph.numpy(), exp)
 
 
+@pytest.mark.parametrize("deg,n_new,itopk", [
+    (64, 64, 128),     # an index-level step
+    (64, 1, 128),      # one run
+    (20, 33, 64),      # a row that does not fill its lanes, runs of 40 keys
+    (80, 100, 192),    # eight slots a lane, the longest copy that fits
+    (72, 130, 192),    # ... and one that does not: the general sort
+    (132, 30, 288),    # sixteen slots a lane
+    (4, 1500, 64),     # more short runs than are searched
+])
+def test_insert_step_shapes(oracle, grab, deg, n_new, itopk):
+    n0, dim = 900, 32
+    data = datasets.mixture(n0 + n_new, dim, 3, 52, 53)  # few clusters: several new rows ask for the same old one
+    graph = np.full((n0 + n_new, deg), 0xFFFFFFFF, np.uint32)
+    graph[:n0] = oracle.optimize(oracle.knn_graph(data[:n0], 2 * deg), deg)
+    exp, _ = oracle.insert_batch(data, n0, n_new, graph, itopk, 4, 50, 12, 9)
+    d_data, d_graph = grab.DeviceArray.from_numpy(data), grab.DeviceArray.from_numpy(graph)
+    grab.insert(d_data, dim, n0, n_new, d_data.ptr + n0 * dim * 4, d_graph, deg, grab.SearchParams(itopk, 4, 0, 50, 12), 9)
+    assert np.array_equal(d_graph.numpy(), exp)
+
+
 def _oracle_index_insert(oracle, data, n0, graph0, deg, seed_state, batches, flags=0):
     """CagraIndex::insert on the CPU: 64 rows per inner step (src/cagraIndex.cu:165-179)."""
     n = n0
