@@ -102,6 +102,27 @@ __device__ __forceinline__ void keys_to_column_list(const TileArgs& a, uint32_t 
         if (at + g < a.col_cap) a.col_list[(size_t)row * a.col_cap + at + g] = keys[g];
 }
 
+// Symmetric pass of the tile kernel: the next (row tile, slice) item, row tile * nsplit + slice; all-ones when none is
+// left.  Every XCD (workgroups go round the eight of them) has a queue of its own, in which eight row tiles follow each
+// other slice by slice: its 64 workgroups then sweep eight slices of the same eight row tiles, and rows and columns alike
+// come from its L2 for seven of eight workgroups.  An empty queue's workgroups go on with the next XCD's.  One row tile
+// after the other, each workgroup read rows of its own from beyond L2 again for every column tile: 100,003 x 768, inner
+// product: 28.5 -> 26.3 ms; 17,000 x 256, squared L2: kNN graph 3.8 -> 3.5 ms.
+constexpr uint32_t kXcds = 8, kSymGroup = 8;
+__device__ __forceinline__ uint32_t next_symmetric_item(const TileArgs& a) {
+    const uint32_t groups = (a.row_tiles + kSymGroup - 1) / kSymGroup, per_group = kSymGroup * a.nsplit;
+    for (uint32_t t = 0; t < kXcds; ++t) {
+        const uint32_t x = (blockIdx.x + t) % kXcds, items = groups > x ? (groups - x + kXcds - 1) / kXcds * per_group : 0u;
+        for (;;) {
+            const uint32_t i = atomicAdd(a.work_counter + x, 1u);
+            if (i >= items) break;
+            const uint32_t k = i / per_group, sp = (i - k * per_group) / kSymGroup, rt = (x + k * kXcds) * kSymGroup + i % kSymGroup;
+            if (rt + sp * a.tiles_per_split < a.col_tiles) return rt * a.nsplit + sp;  // not below the diagonal (nor past the last row)
+        }
+    }
+    return 0xFFFFFFFFu;
+}
+
 template <int METRIC, int FILTER, bool STORE, bool SPLIT = false>
 // two waves per SIMD: keeps the 64 accumulator registers plus the epilogue under 256 VGPRs
 __global__ void __launch_bounds__(256, 2) tile_topk_kernel(const TileArgs a) {
@@ -130,12 +151,11 @@ __global__ void __launch_bounds__(256, 2) tile_topk_kernel(const TileArgs a) {
     __shared__ uint32_t next_item;
     for (uint32_t base = 0; base < nwork; base += gridDim.x) {
         // With a counter the items are handed out in their order to whichever workgroup is free (the two workgroups of
-        // a CU do not run at the same pace: with equal shares the launch lasts as long as the slower ones).  Symmetric
-        // pass: row tile rt sweeps the column tiles from rt on, so the items shrink with rt - the longest go first.
+        // a CU do not run at the same pace: with equal shares the launch lasts as long as the slower ones).
         uint32_t work = base + blockIdx.x;
         if (a.work_counter != nullptr) {
             __syncthreads();  // the item before is fully drained
-            if (tid == 0) next_item = atomicAdd(a.work_counter, 1u);
+            if (tid == 0) next_item = FILTER == kFilterSymmetric ? next_symmetric_item(a) : atomicAdd(a.work_counter, 1u);
             __syncthreads();
             work = next_item;
             if (work >= nwork) break;  // workgroup-uniform
@@ -153,14 +173,8 @@ __global__ void __launch_bounds__(256, 2) tile_topk_kernel(const TileArgs a) {
             rt = lo_rt;
             sp = work - item_off[rt];
         } else {
-            if (FILTER == kFilterSymmetric) {  // slice by slice from the last columns down
-                sp = work / a.row_tiles;
-                rt = work - sp * a.row_tiles;
-                if (rt + sp * a.tiles_per_split >= a.col_tiles) continue;  // workgroup-uniform: the slice lies below the diagonal
-            } else {
-                rt = work / a.nsplit;
-                sp = work - rt * a.nsplit;
-            }
+            rt = work / a.nsplit;
+            sp = work - rt * a.nsplit;
         }
         const uint32_t row0 = rt * TM;
 
@@ -1638,9 +1652,15 @@ int exact_topk(const TopkProblem& p, hipStream_t stream, float* kernel_ms) {
             t.col_cap = kSymColCap;
             t.work_counter = next_counter();
             TileArgs ts = t;
-            ts.tiles_per_split = symmetric_slice(row_tiles, target);
+            if (bf16_bound) {
+                ts.tiles_per_split = symmetric_slice(row_tiles, target);
+            } else {
+                ts.tiles_per_split = std::max(4u, (row_tiles + 15u) / 16u);  // twice as many slices as an XCD has under way at a time
+                counters_used += kXcds - 1;  // a queue per XCD
+            }
             ts.nsplit = (row_tiles + ts.tiles_per_split - 1) / ts.tiles_per_split;
             const uint32_t sym_grid = std::min(row_tiles * ts.nsplit, target);
+            GRAB_REQUIRE(counters_used <= kCounters, "internal: work counters");
             if (bf16_bound) {
                 // where the bounds came from the bf16 pipe (squared L2, up to 128 dimensions) the pass runs there too,
                 // on the split rows the bounding pass left behind: three instructions a product, each at 16x the rate
