@@ -83,14 +83,6 @@ __device__ __forceinline__ void compact_row(Lds& s, uint64_t* rowbuf, int r, uin
     else compact_row_n<16>(s, rowbuf, r, kk, lane);
 }
 
-// STORE: instead of selecting, the distances of the visited tiles are written to a dense
-// matrix a.dense[tile-grid row][column] (row pitch a.dense_pitch); a streaming kernel selects later.
-// SPLIT: a.A and a.B hold rows made by split_rows_chunked_kernel - per chunk of 32 dimensions the 32 bf16 high halves,
-// then the 32 low halves (x = hi + lo + what is left, |left| <= 2^-16 |x|): 128 bytes a chunk like the fp32 row, so
-// the loads and the LDS tiles are the fp32 kernel's byte for byte.  The products come from v_mfma_f32_32x32x16_bf16 as
-// lo.hi + hi.lo + hi.hi with fp32 sums - 24 instructions a chunk where the fp32 path issues 64 that take twice as
-// long each - off the true dot product by at most 3 * 2^-16 |a||b|.  What such a pass returns are candidates; the
-// exact re-scoring and the check after it (refine_kernel, which is told the larger error) decide the result.
 // Symmetric pass with sweeps in slices: the slice that holds the diagonal leaves the row's own list, any other slice its
 // keys - all within the row's bound, like the keys that column walks leave - in the row's list in device memory.  One wave.
 __device__ __forceinline__ void keys_to_column_list(const TileArgs& a, uint32_t row, const uint64_t* keys, uint32_t n, int lane) {
@@ -123,6 +115,14 @@ __device__ __forceinline__ uint32_t next_symmetric_item(const TileArgs& a) {
     return 0xFFFFFFFFu;
 }
 
+// STORE: instead of selecting, the distances of the visited tiles are written to a dense
+// matrix a.dense[tile-grid row][column] (row pitch a.dense_pitch); a streaming kernel selects later.
+// SPLIT: a.A and a.B hold rows made by split_rows_chunked_kernel - per chunk of 32 dimensions the 32 bf16 high halves,
+// then the 32 low halves (x = hi + lo + what is left, |left| <= 2^-16 |x|): 128 bytes a chunk like the fp32 row, so
+// the loads and the LDS tiles are the fp32 kernel's byte for byte.  The products come from v_mfma_f32_32x32x16_bf16 as
+// lo.hi + hi.lo + hi.hi with fp32 sums - 24 instructions a chunk where the fp32 path issues 64 that take twice as
+// long each - off the true dot product by at most 3 * 2^-16 |a||b|.  What such a pass returns are candidates; the
+// exact re-scoring and the check after it (refine_kernel, which is told the larger error) decide the result.
 template <int METRIC, int FILTER, bool STORE, bool SPLIT = false>
 // two waves per SIMD: keeps the 64 accumulator registers plus the epilogue under 256 VGPRs
 __global__ void __launch_bounds__(256, 2) tile_topk_kernel(const TileArgs a) {
