@@ -289,12 +289,15 @@ void scan_rows(const uint64_t* h_bucket_offsets, uint32_t num_buckets, const uin
             r.pieces.push_back({(uint32_t)s0, (uint32_t)std::min<uint64_t>(s0 + kScanPiece, h_bucket_offsets[b + 1])});
     }
     first_piece[num_buckets] = (uint32_t)r.pieces.size();
+    // a query's set is walked along its set bits, not bucket by bucket (a branch that is rarely foretold, twice per query and
+    // bucket): the device waits for these tables.  4999 queries of 1-4 of 64 buckets: call 1.01 -> 0.67 ms
+    const uint64_t known = num_buckets == 64 ? ~0ull : (1ull << num_buckets) - 1ull;
     std::vector<uint32_t> piece_count(r.pieces.size() + 1, 0);
     r.list_off.assign(num_queries + 1, 0);
     for (size_t q = 0; q < num_queries; ++q) {
         uint32_t n = 0;
-        for (uint32_t b = 0; b < num_buckets; ++b) {
-            if (!((h_masks[q] >> b) & 1ull)) continue;
+        for (uint64_t m = h_masks[q] & known; m != 0; m &= m - 1) {
+            const uint32_t b = (uint32_t)__builtin_ctzll(m);
             for (uint32_t pc = first_piece[b]; pc < first_piece[b + 1]; ++pc) piece_count[pc + 1]++;
             n += first_piece[b + 1] - first_piece[b];
         }
@@ -309,8 +312,8 @@ void scan_rows(const uint64_t* h_bucket_offsets, uint32_t num_buckets, const uin
     r.lists.resize(r.list_off[num_queries]);
     std::vector<uint32_t> fill(r.piece_row0.begin(), r.piece_row0.end() - 1), at(r.list_off.begin(), r.list_off.end() - 1);
     for (size_t q = 0; q < num_queries; ++q)
-        for (uint32_t b = 0; b < num_buckets; ++b) {
-            if (!((h_masks[q] >> b) & 1ull)) continue;
+        for (uint64_t m = h_masks[q] & known; m != 0; m &= m - 1) {
+            const uint32_t b = (uint32_t)__builtin_ctzll(m);
             for (uint32_t pc = first_piece[b]; pc < first_piece[b + 1]; ++pc) {
                 const uint32_t row = fill[pc]++;
                 r.row_query[row] = (uint32_t)q;
