@@ -222,8 +222,9 @@ __global__ void __launch_bounds__(256) stream_select_keys_kernel(const float* __
         nwait += (uint32_t)__popcll(b);
         if (nwait >= 64u) merge_waiting();
     };
-    // of an interval of 512 columns and more the first 512 are all candidates, those without an order (NaN) among them
-    const uint32_t c_from = c_hi - c_lo >= 512u ? c_lo + 512u : c_lo;
+    // of an interval of 512 columns and more the first 512 are all candidates, those without an order (NaN) among them; a
+    // bucket's row takes none of these, like the selection inside the contraction that longer lists go through
+    const uint32_t c_from = row_query != nullptr && c_hi - c_lo >= 512u ? c_lo + 512u : c_lo;
     // 512 columns per step, two runs of four consecutive columns per lane, the next step's loads issued before this
     // step's values are looked at; steps are aligned to the row's first stored column
     constexpr uint32_t STEP = 512;

@@ -62,6 +62,32 @@ def test_bucket_scan_queries_that_the_candidates_cannot_prove(oracle, grab):
     assert sent_on > nq // 2, sent_on
 
 
+def test_bucket_scan_leaves_out_what_has_no_order(oracle, grab):
+    # columns whose |a|^2 + |b|^2 - 2ab is no number are no candidates, in buckets below and above 512 rows, whichever way
+    # the list is selected (stored distances up to k = 16, inside the contraction beyond)
+    n, dim = 4000, 32
+    offsets = np.array([0, 300, 1500, 4000], np.uint64)
+    data, q = datasets.mixture(n, dim, 12, 1, 2), datasets.mixture(4, dim, 12, 1, 3)
+    data[320:900:7, 5] = 0.0  # against an infinite query 0 * inf, beside distances that are infinite
+    q[1, 3], q[2, 5] = np.nan, -np.inf
+    bad = data.copy()
+    bad[100:700] = np.nan
+    bad[2000] = -np.float32(np.nan)
+    for rows, gone in ((data, []), (bad, [*range(100, 700), 2000])):
+        d_rows, d_q = grab.DeviceArray.from_numpy(rows), grab.DeviceArray.from_numpy(q)
+        for mask in (1, 2, 4, 7):
+            masks = np.full(4, mask, np.uint64)
+            long_ids, long_dist, _ = grab.bucket_scan_topk(d_rows, n, dim, offsets, d_q, 4, 17, masks)
+            labels = np.repeat(np.arange(3), np.diff(offsets.astype(np.int64))).astype(np.uint8)
+            labels[gone] = 63
+            eids, edist = oracle.bruteforce_topk(data, q[[0, 3]], 16, filter_kind=oracle.FILTER_MASK, labels=labels, masks=masks[:2])
+            for k in (10, 16):
+                ids, dist, _ = grab.bucket_scan_topk(d_rows, n, dim, offsets, d_q, 4, k, masks)
+                assert np.array_equal(ids, long_ids[:, :k]) and np.array_equal(dist.view(np.uint32), long_dist[:, :k].view(np.uint32)), (mask, k)
+                assert (ids[1] == -1).all()
+                assert np.array_equal(ids[[0, 3]], eids[:, :k]) and np.array_equal(dist[[0, 3]], edist[:, :k]), (mask, k)
+
+
 def test_bucket_scan_short_and_empty_buckets(oracle, grab):
     # buckets with fewer rows than k, empty buckets, queries whose buckets are all empty, a mask bit beyond the buckets
     n, dim, nb, nq, k = 900, 32, 16, 200, 20
