@@ -172,6 +172,7 @@ int search_ex_impl(const grab_search_desc* d, bool sync, bool static_tables) {
         use_small = bits <= 15 && bytes(bits) <= room;
         if (use_small && (1ull << bits) < 2 * most && bytes(bits + 1) <= room) ++bits;
         a.table_bitlen = bits;
+        a.set_may_fill = most == 1ull << a.hash_bitlen ? 1 : 0;
         if (use_small) lay.total = bytes(bits);
     }
     if (use_wave) {

@@ -45,6 +45,7 @@ struct SearchArgs {
     int per_query_window;
     uint32_t threads;       // small-batch kernel: threads of a workgroup
     uint32_t table_bitlen;  // small-batch kernel: slots of the visited set's table (2^hash_bitlen ids at most are in it)
+    int set_may_fill;       // small-batch kernel: 2^hash_bitlen ids can come between two rebuilds of the visited set
     uint32_t degree_shift;  // log2 of the degree where that is whole, else 32
     int fixed_shape;        // register-queue kernel: rows of 64 slots all followed, <= 4 parents, <= 64 seeds, filter first, cmax >= 256
     EntryWalk entry;

@@ -41,3 +41,27 @@ def test_small_batch_matches_oracle(oracle, grab, nq, itopk, width, iters, dim, 
     assert np.array_equal(ids, eids)
     assert np.array_equal(dist.view(np.uint32), edist.view(np.uint32))
     assert np.array_equal(ctr, ectr)
+
+
+@pytest.mark.parametrize("bitlen", [4, 6, 8, 10])
+@pytest.mark.parametrize("nq", [3, 300, 513])
+@pytest.mark.parametrize("how", ["all", "filter_first", "filter_after"])
+def test_visited_set_takes_its_size_and_no_more(grab, oracle, how, nq, bitlen):
+    # which ids a set that fills up refuses depends on their order, how many it takes does not, whatever kernel runs:
+    # up to the first rebuild (30 iterations) 2^bitlen ids are scored, and the others counted as refused
+    data, graph, d_data, d_graph = case(oracle, grab, 128, 32)
+    n, cap = data.shape[0], 1 << bitlen
+    d_q = grab.DeviceArray.from_numpy(datasets.mixture(nq, 128, 20, 10, 14))
+    seeds = np.stack([np.random.default_rng(i).permutation(n)[:128] for i in range(nq)]).astype(np.uint32)
+    dev = dict(d_seeds=grab.DeviceArray.from_numpy(seeds), n_provided=128)
+    if how != "all":  # a window that admits every row
+        dev.update(filter_kind=grab.FILTER_ID_RANGE, win=(0, n), flags=grab.FLAG_FILTER_FIRST if how == "filter_first" else 0)
+    for iters in (0, 30):
+        _, _, ctr, _ = grab.search_ex(d_data, d_graph, n, 128, 32, d_q, nq, 10, 128, 4, iters, bitlen, 128, 7, want_counters=True, **dev)
+        scored, refused = ctr[:, 1] + ctr[:, 4], ctr[:, 5]
+        assert (ctr[:, 1] == min(cap, 128)).all()
+        assert (scored[refused > 0] == cap).all() and (scored <= cap).all(), (iters, scored.min(), scored.max())
+        if iters == 0:
+            assert (refused == max(128 - cap, 0)).all()
+        else:
+            assert (refused > 0).any() or bitlen == 10
