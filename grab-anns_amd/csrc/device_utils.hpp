@@ -171,8 +171,11 @@ __device__ __forceinline__ float group8_distance(const float* q, const float* ro
 // taken (it counts the successful inserts); the answer is then -1 without a walk over the whole
 // table - present or not, the id is not expanded either way.
 // READ_FIRST: look at a slot before the compare-and-swap.  Tables in LDS go without: the swap answers what the read
-// would have, and each is a trip to LDS that the lanes of a wave wait for.
-template <bool READ_FIRST = false>
+// would have, and each is a trip to LDS that the lanes of a wave wait for.  Tables in device memory take it: a slot that
+// is taken - most often by the id itself - costs a read that the caches answer, not an atomic operation beyond them
+// (1000 queries, itopk 128, hash_bitlen 16, 100k x 128: 401 us against 535).  No default: every caller says where its
+// table is.
+template <bool READ_FIRST>
 __device__ __forceinline__ int hash_insert(uint32_t* table, uint32_t bitlen, uint32_t key, bool full = false) {
     if (full) return -1;
     const uint32_t size = 1u << bitlen, mask = size - 1;

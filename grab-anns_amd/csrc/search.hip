@@ -203,10 +203,11 @@ __device__ __forceinline__ void merge_candidates(const SearchArgs& a, const Lds&
 // insert into the visited set; successful inserts are counted per workgroup (one LDS add per
 // wave), and once the count says that every slot is taken the table is not walked any more.
 // Must be called by all lanes of a wave together; `active` = this lane has a key.
+template <bool GHASH>
 __device__ __forceinline__ int visited_insert(const Lds& l, uint32_t* table, uint32_t bitlen, bool active, uint32_t key, int lane) {
     const bool full = __atomic_load_n(&l.misc[M_USED], __ATOMIC_RELAXED) >> bitlen;
     int r = 0;
-    if (active) r = hash_insert(table, bitlen, key, full);
+    if (active) r = hash_insert<GHASH>(table, bitlen, key, full);
     const uint64_t b = __ballot(r == 1);
     if (b != 0 && lane == (int)__builtin_ctzll(b)) atomicAdd(&l.misc[M_USED], (uint32_t)__popcll(b));
     return r;
@@ -267,7 +268,7 @@ __global__ void __launch_bounds__(kBlock) search_kernel(const SearchArgs a) {
             if (FILTER != kFilterIdRange) my_f++;
             keep = filter_pass<FILTER>(a, flt, id);
         }
-        const int r = visited_insert(l, table, a.hash_bitlen, keep, id, lane);
+        const int r = visited_insert<GHASH>(l, table, a.hash_bitlen, keep, id, lane);
         if (r < 0) my_full++;
         if (!strict) {
             keep = keep && (r == 1);
@@ -298,7 +299,7 @@ __global__ void __launch_bounds__(kBlock) search_kernel(const SearchArgs a) {
                     const uint32_t i = base + tid;
                     const uint64_t k = i < itopk ? top[i] : kInvalidKey;
                     const bool have = (k != kInvalidKey) || (strict && i < itopk);
-                    const int r = visited_insert(l, table, a.hash_bitlen, have, k != kInvalidKey ? key_id(k) : 0x7FFFFFFFu, lane);
+                    const int r = visited_insert<GHASH>(l, table, a.hash_bitlen, have, k != kInvalidKey ? key_id(k) : 0x7FFFFFFFu, lane);
                     if (r < 0) my_full++;
                 }
                 __syncthreads();
@@ -349,7 +350,7 @@ __global__ void __launch_bounds__(kBlock) search_kernel(const SearchArgs a) {
                 if (FILTER != kFilterIdRange) my_f++;
                 keep = filter_pass<FILTER>(a, flt, nb);
             }
-            const int r = visited_insert(l, table, a.hash_bitlen, keep, nb, lane);
+            const int r = visited_insert<GHASH>(l, table, a.hash_bitlen, keep, nb, lane);
             if (r < 0) my_full++;
             keep = keep && (r == 1);
             if (keep && FILTER != kFilterNone && !filter_first) {

@@ -345,7 +345,7 @@ __global__ void __launch_bounds__(TB) search_small_kernel(const SearchArgs a) {
     auto enter = [&](bool active, uint32_t id, bool counted) {
         const bool full = FILL && (counted ? __atomic_load_n(&l.misc[M_USED], __ATOMIC_RELAXED) : used) >> a.hash_bitlen;
         int r = 0;
-        if (active) r = hash_insert(l.table, a.table_bitlen, id, full);
+        if (active) r = hash_insert<false>(l.table, a.table_bitlen, id, full);
         if (FILL && counted && r == 1 && lds_append(&l.misc[M_USED]) >> a.hash_bitlen) r = -1;
         if (FILL && r < 0) my_full++;
         return r == 1;

@@ -107,7 +107,7 @@ __device__ __forceinline__ void visit(const SearchArgs& a, const WLds& l, const 
         ok = wfilter_pass<FILTER>(a, flt, id);
     }
     if (ok) {
-        const int r = hash_insert(l.table, a.hash_bitlen, id, c.used >> a.hash_bitlen);
+        const int r = hash_insert<false>(l.table, a.hash_bitlen, id, c.used >> a.hash_bitlen);
         if (r < 0) c.full++;
         ok = (r == 1);
     }
@@ -326,7 +326,7 @@ __global__ void __launch_bounds__(64) search_wave_kernel(const SearchArgs a) {
         }
         if (strict) {  // the reference queues a seed whatever the insert returned, unfiltered
             int r = 0;
-            if (keep) r = hash_insert(l.table, a.hash_bitlen, id, cnt.used >> a.hash_bitlen);
+            if (keep) r = hash_insert<false>(l.table, a.hash_bitlen, id, cnt.used >> a.hash_bitlen);
             if (r < 0) cnt.full++;
             cnt.used += (uint32_t)__popcll(__ballot(r == 1));
             const uint64_t b = __ballot(keep);
@@ -354,8 +354,8 @@ __global__ void __launch_bounds__(64) search_wave_kernel(const SearchArgs a) {
                     const uint64_t k = i < itopk ? top[i] : kInvalidKey;
                     const bool full = cnt.used >> a.hash_bitlen;
                     int r = 0;
-                    if (k != kInvalidKey) r = hash_insert(l.table, a.hash_bitlen, key_id(k), full);
-                    else if (strict && i < itopk) r = hash_insert(l.table, a.hash_bitlen, 0x7FFFFFFFu, full);
+                    if (k != kInvalidKey) r = hash_insert<false>(l.table, a.hash_bitlen, key_id(k), full);
+                    else if (strict && i < itopk) r = hash_insert<false>(l.table, a.hash_bitlen, 0x7FFFFFFFu, full);
                     if (r < 0) cnt.full++;
                     cnt.used += (uint32_t)__popcll(__ballot(r == 1));
                 }
@@ -740,7 +740,7 @@ search_wave_reg_kernel(const SearchArgs a) {
             for (int s = 0; s < NQ; ++s) {
                 int r = 0;
                 if ((uint32_t)(lane + 64 * s) < itopk && qk[s] != kInvalidKey)
-                    r = hash_insert(l.table, a.hash_bitlen, key_id(qk[s]), cnt.used >> a.hash_bitlen);
+                    r = hash_insert<false>(l.table, a.hash_bitlen, key_id(qk[s]), cnt.used >> a.hash_bitlen);
                 if (r < 0) cnt.full++;
                 cnt.used += (uint32_t)__popcll(__ballot(r == 1));
             }
@@ -865,7 +865,7 @@ search_wave_reg_kernel(const SearchArgs a) {
                             const bool valid = base + lane < passing;
                             const uint32_t id = valid ? l.surv[first + base + lane] : 0u;
                             int r = 0;
-                            if (valid) r = hash_insert(l.table, a.hash_bitlen, id, cnt.used >> a.hash_bitlen);
+                            if (valid) r = hash_insert<false>(l.table, a.hash_bitlen, id, cnt.used >> a.hash_bitlen);
                             if (r < 0) cnt.full++;
                             const uint64_t b = __ballot(r == 1);
                             cnt.used += (uint32_t)__popcll(b);

@@ -40,7 +40,7 @@ __global__ void __launch_bounds__(256) hash_insert_kernel(uint32_t bitlen, uint3
     const uint32_t size = 1u << bitlen;
     for (uint32_t i = threadIdx.x; i < size; i += blockDim.x) table[i] = kInvalidId;
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) results[i] = hash_insert(table, bitlen, keys[i]) == 1 ? 1u : 0u;
+    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) results[i] = hash_insert<false>(table, bitlen, keys[i]) == 1 ? 1u : 0u;
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < size; i += blockDim.x) table_out[i] = table[i];
 }
