@@ -175,6 +175,22 @@ int search_ex_impl(const grab_search_desc* d, bool sync, bool static_tables) {
         a.set_may_fill = most == 1ull << a.hash_bitlen ? 1 : 0;
         if (use_small) lay.total = bytes(bits);
     }
+    // What that kernel refuses - the reference's literal behaviour, queues beyond 1024 entries, shapes beyond its LDS - gets
+    // 1024 threads of the general kernel in batches of up to 256 queries, and merges split over the waves when the
+    // partial counts fit LDS beside everything else; they never push the visited set to device memory or the queue out of
+    // LDS - such shapes take the plain merge.  Kernel times, us, 64 queries, 100k x 128, 1024 threads against 256:
+    // reference mode, itopk 128, width 6: 115 / 170; itopk 2048, width 4: 555 / 927; itopk 512, width 16, hash_bitlen 15:
+    // 319 / 606.
+    if (!use_wave && !use_small && a.nq <= kSmallBatchQueries) {
+        auto split_layout = [&](bool table) { return search_lds_layout(a.itopk, a.dim, a.cmax, a.search_width, table ? a.hash_bitlen : 0, table, true); };
+        const bool table_fits = a.hash_bitlen < 20 && lay.total <= kMaxLdsBytes;
+        if (a.hash_bitlen < 20 && split_layout(true).total <= kMaxLdsBytes) {
+            a.split_merge = 1;
+            lay = split_layout(true);
+        } else {
+            a.split_merge = !table_fits && split_layout(false).total <= kMaxLdsBytes;
+        }
+    }
     if (use_wave) {
         lay.total = wlay.total;
         a.cmax = wave_cmax;
@@ -183,7 +199,7 @@ int search_ex_impl(const grab_search_desc* d, bool sync, bool static_tables) {
         a.reg_queue = wave_reg ? 1 : 0;
         a.fixed_shape = wave_fixed ? 1 : 0;
     } else if (!use_small && (a.hash_bitlen >= 20 || lay.total > kMaxLdsBytes)) {
-        lay = search_lds_layout(a.itopk, a.dim, a.cmax, a.search_width, 0, false);
+        lay = search_lds_layout(a.itopk, a.dim, a.cmax, a.search_width, 0, false, a.split_merge != 0);
         GRAB_REQUIRE(lay.total <= kMaxLdsBytes, "queue does not fit LDS (itopk %u)", a.itopk);
         const size_t slots = (size_t)a.nq << a.hash_bitlen;
         if (static_tables) {

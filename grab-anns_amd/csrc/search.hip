@@ -1,4 +1,5 @@
-// Beam search over the CAGRA graph, one workgroup of 256 threads (4 waves) per query.
+// Beam search over the CAGRA graph, one workgroup per query: 256 threads (4 waves), or 1024 threads when the batch
+// is so small (<= 256 queries) that 256-thread workgroups would leave most of the device's SIMDs without a wave.
 //
 // Restates the loop of the reference's search_kernel / search_kernel_bucket /
 // search_kernel_range (src/index/search.cu:149-370, :375-586, :589-798) with the expansion
@@ -21,7 +22,8 @@ using namespace dev;
 
 namespace {
 
-constexpr int kBlock = 256;  // threads of a workgroup
+constexpr int kBlock = 256;       // threads of a workgroup, ordinary batches
+constexpr int kBlockSmall = 1024;  // small batches (kSmallBatchQueries queries at most)
 
 enum { M_NSURV = 0, M_NCAND, M_NPAR, M_F, M_FULL, M_USED, M_COUNT };
 
@@ -32,13 +34,14 @@ struct Lds {
     uint32_t* surv;
     uint32_t* parents;
     uint32_t* misc;
+    uint32_t* parts;
     uint32_t* table;
 };
 
 __device__ __forceinline__ Lds carve(uint8_t* smem, const SearchArgs& a) {
     Lds l;
     SearchLdsLayout lay = search_lds_layout(a.itopk, a.dim, a.cmax, a.search_width,
-                                            a.global_hash ? 0 : a.hash_bitlen, a.global_hash == nullptr);
+                                            a.global_hash ? 0 : a.hash_bitlen, a.global_hash == nullptr, a.split_merge != 0);
     l.query = reinterpret_cast<float*>(smem + lay.off_query);
     l.top[0] = reinterpret_cast<uint64_t*>(smem + lay.off_top0);
     l.top[1] = reinterpret_cast<uint64_t*>(smem + lay.off_top1);
@@ -46,6 +49,7 @@ __device__ __forceinline__ Lds carve(uint8_t* smem, const SearchArgs& a) {
     l.surv = reinterpret_cast<uint32_t*>(smem + lay.off_surv);
     l.parents = reinterpret_cast<uint32_t*>(smem + lay.off_parents);
     l.misc = reinterpret_cast<uint32_t*>(smem + lay.off_misc);
+    l.parts = reinterpret_cast<uint32_t*>(smem + lay.off_parts);
     l.table = reinterpret_cast<uint32_t*>(smem + lay.off_hash);
     return l;
 }
@@ -82,13 +86,18 @@ __device__ __forceinline__ void append_survivor(const Lds& l, bool keep, uint32_
 
 // Scores the survivors and appends those that beat `worst` to the candidate list.
 // Two rows per 8-lane group per round, so that 2*CPL row loads are in flight per lane.
-template <int CPL, int METRIC>
+//
+// Small batches (TB = 1024: fewer queries than CUs, every iteration a chain of two waits for HBM, graph rows then
+// vectors) also touch the graph row of every row that joins the list: whichever of them becomes a parent later has
+// its row in the second-level cache by then.  The words read stay in `touched` until the next round folds them
+// away: nothing depends on them before, so the wait for them falls a round or a whole iteration later.
+template <int TB, int CPL, int METRIC>
 __device__ __forceinline__ void score_survivors(const SearchArgs& a, const Lds& l, const float4 (&qreg)[CPL ? CPL : 1],
-                                                uint64_t worst, int grp, int j) {
+                                                uint64_t worst, int grp, int j, uint32_t (&touched)[3]) {
     const uint32_t ns = l.misc[M_NSURV];
     const uint32_t nchunks = a.dim >> 2;
     const float4* q4 = reinterpret_cast<const float4*>(l.query);
-    constexpr uint32_t kGroups = kBlock / 8;
+    constexpr uint32_t kGroups = TB / 8;
     const int lane = threadIdx.x & 63;
     const uint64_t lt = (1ull << lane) - 1ull;
     for (uint32_t sbase = 0; sbase < ns; sbase += 2 * kGroups) {  // same trip count for every wave
@@ -122,6 +131,13 @@ __device__ __forceinline__ void score_survivors(const SearchArgs& a, const Lds& 
             }
             k0 = make_key(s0, id0);
             if (two) k1 = make_key(s1, id1);
+        }
+        if (TB == kBlockSmall) {
+            const uint32_t line = (uint32_t)j * 32u;  // a lane per 128 bytes of the row
+            touched[2] ^= touched[0] ^ touched[1];  // the words of the round before
+            touched[0] = touched[1] = 0;
+            if (k0 < worst && line < a.degree) touched[0] = a.graph[(size_t)key_id(k0) * a.degree + line];
+            if (k1 < worst && line < a.degree) touched[1] = a.graph[(size_t)key_id(k1) * a.degree + line];
         }
         // one reservation in the candidate list per wave, not one per row
         const bool p0 = (j == 0) && k0 < worst, p1 = (j == 0) && k1 < worst;
@@ -170,11 +186,62 @@ __device__ __forceinline__ uint32_t count_before(const uint64_t* cand, uint32_t 
     return cnt;
 }
 
+// The merge of a small batch (1024 threads a query, LDS with room for partial counts).  A thread that counts a whole
+// list for its entry is what the workgroup waits for, so the counting is cut up: the list into kMergeChunks parts,
+// and every (64 entries, list part) pair is a task of its own, as is the search of the queue for 64 candidates; the
+// tasks go round the 16 waves, the counts to LDS, and after a barrier every entry adds up its counts and moves.
+__device__ __forceinline__ void merge_split(const SearchArgs& a, const Lds& l, const uint64_t* src, uint64_t* dst, uint32_t nc_any, int tid) {
+    const uint32_t nc = (uint32_t)__builtin_amdgcn_readfirstlane((int)nc_any);  // the same in every thread: the tasks below are picked per wave
+    constexpr uint32_t NW = kBlockSmall / 64, NB = kMergeChunks;
+    const uint32_t lane = (uint32_t)tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t itopk = a.itopk, cmax = a.cmax;
+    const bool ties = a.flags & GRAB_FLAG_STRICT_REFERENCE;  // two candidates of one list are only ever equal when this lets an id in twice
+    const uint32_t part_len = ((nc + 8u * NB - 1u) / (8u * NB)) * 8u;  // whole eights
+    const uint32_t c64 = (nc + 63u) >> 6, q64 = (itopk + 63u) >> 6;
+    uint32_t* cand_part = l.parts;                  // [NB][cmax]
+    uint32_t* cand_queue = l.parts + NB * cmax;     // [cmax]
+    uint32_t* queue_part = l.parts + (NB + 1u) * cmax;  // [NB][itopk]
+    const uint32_t n_tasks = c64 * NB + c64 + q64 * NB;
+    for (uint32_t task = wave; task < n_tasks; task += NW) {
+        if (task < c64 * NB) {  // candidates task / NB * 64 .. + 63 against list part task % NB
+            const uint32_t b = task % NB, x = (task / NB) * 64u + lane;
+            const uint32_t from = min(b * part_len, nc), len = min(part_len, nc - from);
+            if (x < nc) {
+                const uint64_t kx = l.cand[x];
+                const uint32_t self = x > from ? x - from : 0u;  // list places before x, counted from the part's start
+                cand_part[b * cmax + x] = ties ? count_before<true>(l.cand + from, len, kx, self) : count_before<false>(l.cand + from, len, kx, 0);
+            }
+        } else if (task < c64 * NB + c64) {  // the queue entries at or below 64 candidates
+            const uint32_t x = (task - c64 * NB) * 64u + lane;
+            if (x < nc) cand_queue[x] = upper_bound_u64(src, itopk, l.cand[x]);
+        } else {  // 64 queue entries against a list part; a queue entry goes ahead of an equal candidate
+            const uint32_t t = task - c64 * NB - c64;
+            const uint32_t b = t % NB, e = (t / NB) * 64u + lane;
+            const uint32_t from = min(b * part_len, nc), len = min(part_len, nc - from);
+            if (e < itopk) queue_part[b * itopk + e] = count_before<false>(l.cand + from, len, src[e] & ~1ull, 0);
+        }
+    }
+    __syncthreads();
+    for (uint32_t i = kBlockSmall - 1 - tid; i < itopk; i += kBlockSmall) {  // the last threads, as in the plain merge
+        uint32_t r = i;
+#pragma unroll
+        for (uint32_t b = 0; b < NB; ++b) r += queue_part[b * itopk + i];
+        if (r < itopk) dst[r] = src[i];
+    }
+    for (uint32_t x = tid; x < nc; x += kBlockSmall) {
+        uint32_t r = cand_queue[x];
+#pragma unroll
+        for (uint32_t b = 0; b < NB; ++b) r += cand_part[b * cmax + x];
+        if (r < itopk) dst[r] = l.cand[x];
+    }
+}
+
 // Rank-counting merge of the candidate list into the sorted queue.  An entry's new position
 // is the number of entries ordered before it by (distance,id); the expanded flag takes no part
 // in the order, queue entries go ahead of equal candidates and equal candidates go by list
 // index (equal entries only exist when GRAB_FLAG_STRICT_REFERENCE lets duplicates in).  On return `top` points to the merged queue
 // and `spare` to the other buffer.
+template <int TB>
 __device__ __forceinline__ void merge_candidates(const SearchArgs& a, const Lds& l, uint64_t*& top,
                                                  uint64_t*& spare, int tid) {
     const uint32_t nc = l.misc[M_NCAND];
@@ -182,15 +249,22 @@ __device__ __forceinline__ void merge_candidates(const SearchArgs& a, const Lds&
     const uint64_t* src = top;
     uint64_t* dst = spare;
     const uint32_t itopk = a.itopk;
+    if (TB == kBlockSmall && a.split_merge) {
+        merge_split(a, l, src, dst, nc, tid);
+        __syncthreads();
+        spare = top;
+        top = dst;
+        return;
+    }
     // the last threads take the queue entries, the first ones the candidates: different waves where there are several
-    for (uint32_t i = kBlock - 1 - tid; i < itopk; i += kBlock) {
+    for (uint32_t i = TB - 1 - tid; i < itopk; i += TB) {
         const uint64_t ki = src[i];
         const uint32_t r = i + count_before<false>(l.cand, nc, ki & ~1ull, 0);  // a queue entry goes ahead of an equal candidate
         if (r < itopk) dst[r] = ki;
     }
     // two candidates of one list are only ever equal when GRAB_FLAG_STRICT_REFERENCE lets an id in twice
     const bool ties = a.flags & GRAB_FLAG_STRICT_REFERENCE;
-    for (uint32_t x = tid; x < nc; x += kBlock) {
+    for (uint32_t x = tid; x < nc; x += TB) {
         const uint64_t kx = l.cand[x];
         const uint32_t cnt = upper_bound_u64(src, itopk, kx) + (ties ? count_before<true>(l.cand, nc, kx, x) : count_before<false>(l.cand, nc, kx, x));
         if (cnt < itopk) dst[cnt] = kx;
@@ -213,8 +287,8 @@ __device__ __forceinline__ int visited_insert(const Lds& l, uint32_t* table, uin
     return r;
 }
 
-template <int CPL, int METRIC, int FILTER, bool GHASH>
-__global__ void __launch_bounds__(kBlock) search_kernel(const SearchArgs a) {
+template <int TB, int CPL, int METRIC, int FILTER, bool GHASH>
+__global__ void __launch_bounds__(TB) search_kernel(const SearchArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
     Lds l = carve(smem, a);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -229,9 +303,9 @@ __global__ void __launch_bounds__(kBlock) search_kernel(const SearchArgs a) {
     // ---- set-up: query, empty queue, empty visited set (search.cu:217-227) ----
     {
         const float* gq = a.queries + (size_t)q * a.dim;
-        for (uint32_t i = tid; i < a.dim; i += kBlock) l.query[i] = gq[i];
-        for (uint32_t i = tid; i < itopk; i += kBlock) l.top[0][i] = kInvalidKey;
-        for (uint32_t i = tid; i < table_size; i += kBlock) table[i] = kInvalidId;
+        for (uint32_t i = tid; i < a.dim; i += TB) l.query[i] = gq[i];
+        for (uint32_t i = tid; i < itopk; i += TB) l.top[0][i] = kInvalidKey;
+        for (uint32_t i = tid; i < table_size; i += TB) table[i] = kInvalidId;
         if (tid < M_COUNT) l.misc[tid] = 0;
     }
     __syncthreads();
@@ -254,7 +328,7 @@ __global__ void __launch_bounds__(kBlock) search_kernel(const SearchArgs a) {
     uint32_t c_iters = 0, c_seed = 0, c_par = 0, c_child = 0;  // uniform counts
 
     // ---- seeds (compute_distance.cuh:144-202, :204-269) ----
-    for (uint32_t base = 0; base < a.n_seeds; base += kBlock) {
+    for (uint32_t base = 0; base < a.n_seeds; base += TB) {
         const uint32_t i = base + tid;
         bool keep = false;
         uint32_t id = kInvalidId;
@@ -281,7 +355,8 @@ __global__ void __launch_bounds__(kBlock) search_kernel(const SearchArgs a) {
     }
     __syncthreads();
     c_seed = l.misc[M_NSURV];
-    score_survivors<CPL, METRIC>(a, l, qreg, kInvalidKey, grp, j);
+    uint32_t touched[3] = {0, 0, 0};
+    score_survivors<TB, CPL, METRIC>(a, l, qreg, kInvalidKey, grp, j, touched);
     __syncthreads();
 
     uint64_t* top = l.top[0];
@@ -290,12 +365,12 @@ __global__ void __launch_bounds__(kBlock) search_kernel(const SearchArgs a) {
         // every 30 iterations the visited set is rebuilt from the queue (search.cu:265-283)
         const bool reset = iter > 0 && (iter % 30u == 0);
         for (int pass = 0; pass < 2; ++pass) {
-            if (pass == 1) merge_candidates(a, l, top, spare, tid);
+            if (pass == 1) merge_candidates<TB>(a, l, top, spare, tid);
             if (reset && ((pass == 0) == strict)) {
-                for (uint32_t i = tid; i < table_size; i += kBlock) table[i] = kInvalidId;
+                for (uint32_t i = tid; i < table_size; i += TB) table[i] = kInvalidId;
                 if (tid == 0) l.misc[M_USED] = 0;
                 __syncthreads();
-                for (uint32_t base = 0; base < itopk; base += kBlock) {  // hashmap.cuh:103-117
+                for (uint32_t base = 0; base < itopk; base += TB) {  // hashmap.cuh:103-117
                     const uint32_t i = base + tid;
                     const uint64_t k = i < itopk ? top[i] : kInvalidKey;
                     const bool have = (k != kInvalidKey) || (strict && i < itopk);
@@ -335,7 +410,7 @@ __global__ void __launch_bounds__(kBlock) search_kernel(const SearchArgs a) {
 
         // ---- expansion: ids, visited set, filter (compute_distance.cuh:274-380 etc.) ----
         const uint32_t total = np * a.degree;
-        for (uint32_t base = 0; base < total; base += kBlock) {
+        for (uint32_t base = 0; base < total; base += TB) {
             const uint32_t t = base + tid;
             bool keep = false;
             uint32_t nb = kInvalidId;
@@ -361,13 +436,14 @@ __global__ void __launch_bounds__(kBlock) search_kernel(const SearchArgs a) {
         }
         __syncthreads();
         c_child += l.misc[M_NSURV];
-        score_survivors<CPL, METRIC>(a, l, qreg, top[itopk - 1] & ~1ull, grp, j);
+        score_survivors<TB, CPL, METRIC>(a, l, qreg, top[itopk - 1] & ~1ull, grp, j, touched);
         __syncthreads();
     }
-    merge_candidates(a, l, top, spare, tid);
+    merge_candidates<TB>(a, l, top, spare, tid);
+    asm volatile("" ::"v"(touched[0] ^ touched[1] ^ touched[2]));  // the reads above are kept; nothing is done with the words
 
     // ---- results (search.cu:348-355; ids widened here instead of a second kernel) ----
-    for (uint32_t r = tid; r < a.k; r += kBlock) {
+    for (uint32_t r = tid; r < a.k; r += TB) {
         const uint64_t k = top[r];
         int64_t id = strict ? (int64_t)0x7FFFFFFF : -1;
         float d = kDistMax;
@@ -397,12 +473,13 @@ __global__ void __launch_bounds__(kBlock) search_kernel(const SearchArgs a) {
 
 template <int CPL, int METRIC, int FILTER, bool GHASH>
 int launch(const SearchArgs& a, size_t lds_bytes, hipStream_t stream) {
-    auto kern = search_kernel<CPL, METRIC, FILTER, GHASH>;
+    const bool small = a.nq <= kSmallBatchQueries;
+    auto kern = small ? search_kernel<kBlockSmall, CPL, METRIC, FILTER, GHASH> : search_kernel<kBlock, CPL, METRIC, FILTER, GHASH>;
     if (lds_bytes > 64 * 1024) {
         GRAB_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
     }
-    hipLaunchKernelGGL(kern, dim3(a.nq), dim3(kBlock), lds_bytes, stream, a);
+    hipLaunchKernelGGL(kern, dim3(a.nq), dim3(small ? kBlockSmall : kBlock), lds_bytes, stream, a);
     GRAB_HIP(hipGetLastError());
     return GRAB_OK;
 }

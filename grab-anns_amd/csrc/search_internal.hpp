@@ -43,6 +43,7 @@ struct SearchArgs {
     int single_queue;       // wave-per-query kernel: one queue buffer, merged in place (itopk <= 64, ccap <= 128)
     int reg_queue;          // wave-per-query kernel: the queue lives in registers, 1/2/4 entries per lane (itopk <= 256, not strict)
     int per_query_window;
+    int split_merge;        // workgroup-per-query kernel with 1024 threads: the merge is cut into tasks whose partial counts live in LDS
     uint32_t threads;       // small-batch kernel: threads of a workgroup
     uint32_t table_bitlen;  // small-batch kernel: slots of the visited set's table (2^hash_bitlen ids at most are in it)
     int set_may_fill;       // small-batch kernel: 2^hash_bitlen ids can come between two rebuilds of the visited set
@@ -52,13 +53,17 @@ struct SearchArgs {
 };
 
 struct SearchLdsLayout {
-    uint32_t off_query, off_top0, off_top1, off_cand, off_surv, off_parents, off_misc, off_hash, total;
+    uint32_t off_query, off_top0, off_top1, off_cand, off_surv, off_parents, off_misc, off_parts, off_hash, total;
 };
+
+// Batches of up to this many queries (CUs) get 1024 threads a query: what counts is how long one query takes
+constexpr uint32_t kSmallBatchQueries = 256;
+constexpr uint32_t kMergeChunks = 4;  // parts that the candidate list is cut into for a split merge
 
 // cmax = capacity of the survivor / candidate lists = max(search_width*degree, n_seeds)
 __host__ __device__ inline SearchLdsLayout search_lds_layout(uint32_t itopk, uint32_t dim, uint32_t cmax,
                                                             uint32_t search_width, uint32_t hash_bitlen,
-                                                            bool hash_in_lds) {
+                                                            bool hash_in_lds, bool split_merge = false) {
     SearchLdsLayout l;
     uint32_t off = 0;
     auto take = [&](uint32_t bytes) {
@@ -73,6 +78,8 @@ __host__ __device__ inline SearchLdsLayout search_lds_layout(uint32_t itopk, uin
     l.off_surv = take(cmax * 4);
     l.off_parents = take(search_width * 4);
     l.off_misc = take(16 * 4);
+    // split merge: per candidate one count per list part and one for the queue, per queue entry one count per list part
+    l.off_parts = take(split_merge ? ((kMergeChunks + 1u) * cmax + kMergeChunks * itopk) * 4u : 0u);
     l.off_hash = take(hash_in_lds ? (1u << hash_bitlen) * 4u : 0u);
     l.total = off;
     return l;
@@ -83,7 +90,6 @@ struct SearchSmallLdsLayout {
     uint32_t off_query, off_top, off_open, off_marked, off_ahead, off_cand, off_surv, off_parents, off_misc, off_hash, total;
 };
 constexpr uint32_t kSmallMaxItopk = 1024;
-constexpr uint32_t kSmallBatchQueries = 256;  // CUs
 // queue places: whole blocks of 64, and as many of them as the kernel's merge reads (1, 2, 4 or 16)
 __host__ __device__ inline uint32_t search_small_padded_queue(uint32_t itopk) {
     return itopk <= 64 ? 64u : itopk <= 128 ? 128u : itopk <= 256 ? 256u : 1024u;

@@ -1,5 +1,6 @@
 """Small batches: the kernel made for the time of one query, where its shapes change - 1024 / 512 threads, one to sixteen
-queue blocks, candidates merged beside the expansion or before it, rows that are no whole rounds of loads - against the oracle."""
+queue blocks, candidates merged beside the expansion or before it, rows that are no whole rounds of loads - and the general
+kernel for what that one refuses, against the oracle."""
 import numpy as np
 import pytest
 
@@ -22,7 +23,10 @@ def case(oracle, grab, dim, deg):
     (1, 64, 4, 50, 128, 32, 13, False), (3, 256, 6, 50, 128, 32, 13, False), (256, 65, 4, 40, 96, 32, 12, True),
     (257, 128, 4, 40, 96, 32, 12, True), (512, 64, 1, 35, 100, 32, 11, False), (513, 64, 4, 35, 100, 32, 12, False),
     (5, 300, 4, 62, 132, 24, 13, False), (7, 1000, 3, 31, 32, 24, 14, True), (9, 64, 20, 40, 32, 24, 17, False),
-    (4, 64, 32, 20, 128, 32, 13, True), (2, 64, 4, 0, 128, 32, 13, False), (2, 64, 4, 1, 128, 32, 13, False), (6, 10, 2, 45, 128, 32, 12, False)])
+    (4, 64, 32, 20, 128, 32, 13, True), (2, 64, 4, 0, 128, 32, 13, False), (2, 64, 4, 1, 128, 32, 13, False), (6, 10, 2, 45, 128, 32, 12, False),
+    # what that kernel refuses: 1024 threads of the general one, merges split over the waves or plain, tables in LDS or not
+    (3, 1100, 4, 40, 128, 32, 13, False), (256, 1030, 4, 33, 96, 32, 13, True), (257, 1100, 4, 20, 96, 32, 13, True),
+    (5, 64, 64, 12, 128, 32, 16, True), (2, 900, 100, 10, 128, 32, 15, False)])
 def test_small_batch_matches_oracle(oracle, grab, nq, itopk, width, iters, dim, deg, bitlen, filtered):
     data, graph, d_data, d_graph = case(oracle, grab, dim, deg)
     n, k = data.shape[0], 10
