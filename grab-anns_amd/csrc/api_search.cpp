@@ -155,7 +155,15 @@ int search_ex_impl(const grab_search_desc* d, bool sync, bool static_tables) {
     // itopk 128, width 4; workgroup kernel of 256 threads / 512 threads / 1024 threads): 1 query 115 / 86 / 80, 256: 167 /
     // 121 / 112, 300: 164 / 129 / 195, 512: 173 / 139 / 207, 600: 172 / 218 / 292; in the same order for other shapes
     // (itopk 64 and 256, 96 and 256 dimensions, 10 % windows).
-    bool use_small = !use_wave && a.nq <= 2 * kSmallBatchQueries && a.itopk <= kSmallMaxItopk && !(d->flags & GRAB_FLAG_STRICT_REFERENCE);
+    // Where a query can have a CU to itself, an iteration with many neighbours to look at is quicker in the general kernel
+    // (1024 threads, below): it reserves places in its lists for a wave at a time, not lane by lane, and its merge costs less
+    // for a candidate and more for a queue entry.  The two meet at 512 + itopk neighbours or 2 * itopk (100 queries, 100k x
+    // 128, us, general / this kernel; itopk 64: 512 neighbours 66 / 66, 640: 70 / 73, 2048: 185 / 301; 128: 640: 114 / 103,
+    // 768: 104 / 108; 256: 768: 188 / 166, 1536: 230 / 266; 512: 1024: 394 / 351; 1024: 2048: 17.5 / 14.3 ms).
+    const uint32_t neighbours = a.search_width * a.degree;
+    const bool few = neighbours <= std::max(512u + a.itopk, 2u * a.itopk);
+    bool use_small = !use_wave && a.nq <= 2 * kSmallBatchQueries && (few || a.nq > kSmallBatchQueries) && a.itopk <= kSmallMaxItopk &&
+                     !(d->flags & GRAB_FLAG_STRICT_REFERENCE);
     if (static_tables && (a.hash_bitlen >= 20 || lay.total > kMaxLdsBytes)) use_small = false;  // the static array's rules
     if (use_small) {
         const bool alone = a.nq <= kSmallBatchQueries;
@@ -175,12 +183,12 @@ int search_ex_impl(const grab_search_desc* d, bool sync, bool static_tables) {
         a.set_may_fill = most == 1ull << a.hash_bitlen ? 1 : 0;
         if (use_small) lay.total = bytes(bits);
     }
-    // What that kernel refuses - the reference's literal behaviour, queues beyond 1024 entries, shapes beyond its LDS - gets
-    // 1024 threads of the general kernel in batches of up to 256 queries, and merges split over the waves when the
-    // partial counts fit LDS beside everything else; they never push the visited set to device memory or the queue out of
-    // LDS - such shapes take the plain merge.  Kernel times, us, 64 queries, 100k x 128, 1024 threads against 256:
-    // reference mode, itopk 128, width 6: 115 / 170; itopk 2048, width 4: 555 / 927; itopk 512, width 16, hash_bitlen 15:
-    // 319 / 606.
+    // What that kernel does not take - the reference's literal behaviour, queues beyond 1024 entries, shapes beyond its LDS,
+    // many neighbours an iteration - gets 1024 threads of the general kernel in batches of up to 256 queries, and merges
+    // split over the waves when the partial counts fit LDS beside everything else; they never push the visited set to
+    // device memory or the queue out of LDS - such shapes take the plain merge.  Kernel times, us, 64 queries, 100k x 128,
+    // 1024 threads against 256: reference mode, itopk 128, width 6: 115 / 170; itopk 2048, width 4: 555 / 927; itopk 512,
+    // width 16, hash_bitlen 15: 319 / 606.
     if (!use_wave && !use_small && a.nq <= kSmallBatchQueries) {
         auto split_layout = [&](bool table) { return search_lds_layout(a.itopk, a.dim, a.cmax, a.search_width, table ? a.hash_bitlen : 0, table, true); };
         const bool table_fits = a.hash_bitlen < 20 && lay.total <= kMaxLdsBytes;

@@ -24,6 +24,8 @@ def case(oracle, grab, dim, deg):
     (257, 128, 4, 40, 96, 32, 12, True), (512, 64, 1, 35, 100, 32, 11, False), (513, 64, 4, 35, 100, 32, 12, False),
     (5, 300, 4, 62, 132, 24, 13, False), (7, 1000, 3, 31, 32, 24, 14, True), (9, 64, 20, 40, 32, 24, 17, False),
     (4, 64, 32, 20, 128, 32, 13, True), (2, 64, 4, 0, 128, 32, 13, False), (2, 64, 4, 1, 128, 32, 13, False), (6, 10, 2, 45, 128, 32, 12, False),
+    (300, 64, 32, 20, 128, 32, 13, True), (3, 1000, 40, 20, 96, 32, 14, False),  # more neighbours than threads
+    (2, 64, 18, 30, 128, 32, 13, False), (2, 64, 19, 30, 128, 32, 13, True),     # the last width it takes, and the first it does not
     # what that kernel refuses: 1024 threads of the general one, merges split over the waves or plain, tables in LDS or not
     (3, 1100, 4, 40, 128, 32, 13, False), (256, 1030, 4, 33, 96, 32, 13, True), (257, 1100, 4, 20, 96, 32, 13, True),
     (5, 64, 64, 12, 128, 32, 16, True), (2, 900, 100, 10, 128, 32, 15, False)])
