@@ -114,7 +114,7 @@ __device__ __forceinline__ float fold4(float s, const float4 a, const float4 b) 
 // Rows of any length (a multiple of four floats), query in LDS: lane j of a group of eight folds the chunks j, j + 8, ...
 // in that order.  Four chunks of each row are requested before the first is used, so that a wave keeps up to
 // 8 x 2 x 4 sixteen-byte loads in flight; the last ones too - a place past the end becomes the row's last chunk and is
-// folded as zeros, which leave a sum as it is - because a row costs one wait for memory per such round.
+// not folded (zeros in its place would turn a sum of -0 into +0) - because a row costs one wait for memory per such round.
 template <int METRIC, bool TWO>
 __device__ __forceinline__ void fold_rows_any(const float4* __restrict__ r0, const float4* __restrict__ r1, const float4* q4,
                                               uint32_t j, uint32_t nchunks, float& d0, float& d1) {
@@ -145,10 +145,13 @@ __device__ __forceinline__ void fold_rows_any(const float4* __restrict__ r0, con
 #pragma unroll
         for (int u = 0; u < 3; ++u) {
             const bool in = c + 8 * u < nchunks;
-            const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            const float4 qq = in ? q4[c + 8 * u] : zero;
-            d0 = fold4<METRIC>(d0, qq, in ? x0[u] : zero);
-            if (TWO) d1 = fold4<METRIC>(d1, qq, in ? x1[u] : zero);
+            const float4 qq = q4[min(c + 8 * u, nchunks - 1u)];
+            const float s0 = fold4<METRIC>(d0, qq, x0[u]);
+            d0 = in ? s0 : d0;
+            if (TWO) {
+                const float s1 = fold4<METRIC>(d1, qq, x1[u]);
+                d1 = in ? s1 : d1;
+            }
         }
     }
 }

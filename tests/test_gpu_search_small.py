@@ -71,3 +71,24 @@ def test_visited_set_takes_its_size_and_no_more(grab, oracle, how, nq, bitlen):
             assert (refused == max(128 - cap, 0)).all()
         else:
             assert (refused > 0).any() or bitlen == 10
+
+
+@pytest.mark.parametrize("nq", [2, 513])
+@pytest.mark.parametrize("dim", [36, 96, 104])
+def test_products_that_vanish_keep_their_sign(oracle, grab, dim, nq):
+    # every product underflows: a row's inner product is -0 or +0, which differ in the result and in the order
+    n, k = 300, 10
+    rng = np.random.default_rng(dim)
+    data = (np.float32(1e-30) * rng.choice(np.float32([-1, 1]), (n, 1))) * np.ones((1, dim), np.float32)
+    q = np.full((nq, dim), 1e-30, np.float32)
+    graph = rng.integers(0, n, (n, 32)).astype(np.uint32)
+    seeds = np.tile(np.arange(64, dtype=np.uint32), (nq, 1))
+    d_data, d_q = grab.DeviceArray.from_numpy(data), grab.DeviceArray.from_numpy(q)
+    eids, edist, _ = oracle.search(data, graph, q, k, 64, 2, 20, 13, 64, 5, metric=1, seeds=seeds)
+    ids, dist, _, _ = grab.search_ex(d_data, grab.DeviceArray.from_numpy(graph), n, dim, 32, d_q, nq, k, 64, 2, 20, 13, 64, 5, metric=1,
+                                     d_seeds=grab.DeviceArray.from_numpy(seeds), n_provided=64)
+    assert np.array_equal(dist.view(np.uint32), edist.view(np.uint32)) and np.array_equal(ids, eids)
+    # the exact scan re-scores its candidates in the same order of sums
+    bids, bdist, _ = grab.bruteforce_topk(d_data, n, dim, d_q, nq, k, metric=1)
+    xids, xdist = oracle.bruteforce_topk(data, q, k, metric=1)
+    assert np.array_equal(bdist.view(np.uint32), xdist.view(np.uint32)) and np.array_equal(bids, xids)
