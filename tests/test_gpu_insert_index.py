@@ -54,6 +54,8 @@ def test_insert_large_call_uses_global_sort(oracle, grab):
     (72, 130, 192),    # ... and one that does not: the general sort
     (132, 30, 288),    # sixteen slots a lane
     (4, 1500, 64),     # more short runs than are searched
+    (65, 20, 160), (128, 17, 256), (129, 9, 288), (256, 6, 512),  # either side of four, eight and sixteen slots a lane
+    (257, 5, 576), (400, 3, 800),                                 # thirty-two slots a lane, sixteen keys a lane sorted
 ])
 def test_insert_step_shapes(oracle, grab, deg, n_new, itopk):
     n0, dim = 900, 32
