@@ -1,5 +1,6 @@
-// Beam search over the CAGRA graph, one workgroup per query: 256 threads (4 waves), or 1024 threads when the batch
-// is so small (<= 256 queries) that 256-thread workgroups would leave most of the device's SIMDs without a wave.
+// Beam search over the CAGRA graph, one workgroup per query: 256 threads (4 waves), or 1024 threads in batches so small
+// (<= 256 queries) that 256-thread workgroups would leave most of the device's SIMDs without a wave - those of them that
+// search_small.hip does not take.
 //
 // Restates the loop of the reference's search_kernel / search_kernel_bucket /
 // search_kernel_range (src/index/search.cu:149-370, :375-586, :589-798) with the expansion

@@ -100,7 +100,8 @@ uint32_t grab_queue_capacity(uint32_t itopk, uint32_t search_width, uint32_t deg
 size_t grab_reference_smem_bytes(uint32_t itopk, uint32_t dim, uint32_t search_width,
                                  uint32_t degree, uint32_t hash_bitlen);
 /* LDS bytes that this library's workgroup-per-query search kernel uses for the same parameters on batches of more
- * than 512 queries (smaller batches use up to twice as much) */
+ * than 512 queries.  It says nothing about smaller batches: their queues are padded to whole blocks, their visited sets
+ * lie in LDS where this figure has them in device memory, and merges may keep counts beside them. */
 size_t grab_search_lds_bytes(uint32_t itopk, uint32_t dim, uint32_t search_width,
                              uint32_t degree, uint32_t n_seeds, uint32_t hash_bitlen);
 
