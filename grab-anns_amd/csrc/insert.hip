@@ -172,7 +172,7 @@ __global__ void __launch_bounds__(256) apply_updates_kernel(uint32_t* __restrict
             if (((__ballot(exists) >> group) & 0xFFFFull) != 0) continue;
             rng = rng * 6364136223846793005ull + 1;
             const uint32_t r1 = (uint32_t)(rng >> 32);
-            const bool upd_protected = (r1 % 10u == 0);
+            const bool upd_protected = (r1 % 10u == 0) && num_protected != 0;  // a row of one slot has no first half
             rng = rng * 6364136223846793005ull + 1;
             const uint32_t r2 = (uint32_t)(rng >> 32);
             const uint32_t slot = upd_protected ? (r2 % num_protected) : num_protected + (r2 % num_unprotected);

@@ -919,7 +919,7 @@ void orc_insert_batch(const float* data, uint32_t dim, size_t n_existing, size_t
             if (exists) continue;
             rng = rng * 6364136223846793005ull + 1;
             uint32_t r1 = (uint32_t)(rng >> 32);
-            bool upd_protected = (r1 % 10 == 0);
+            bool upd_protected = (r1 % 10 == 0) && num_protected != 0;  // a row of one slot has no first half
             rng = rng * 6364136223846793005ull + 1;
             uint32_t r2 = (uint32_t)(rng >> 32);
             uint32_t slot = upd_protected ? (r2 % num_protected) : num_protected + (r2 % num_unprotected);

@@ -55,6 +55,7 @@ def test_insert_large_call_uses_global_sort(oracle, grab):
     (132, 30, 288),    # sixteen slots a lane
     (4, 1500, 64),     # more short runs than are searched
     (65, 20, 160), (128, 17, 256), (129, 9, 288), (256, 6, 512),  # either side of four, eight and sixteen slots a lane
+    (1, 200, 64), (2, 200, 64),                                   # rows of one slot have no protected half
     (257, 5, 576), (400, 3, 800),                                 # thirty-two slots a lane, sixteen keys a lane sorted
 ])
 def test_insert_step_shapes(oracle, grab, deg, n_new, itopk):
