@@ -29,6 +29,9 @@ namespace {
 constexpr uint32_t kScanRowsTile = 128;
 constexpr uint32_t kScanListCap = 2048;  // entries of a row's list
 constexpr uint32_t kScanSortCap = 1024;  // ... of which a wave sorts the nearest
+constexpr float kScanLift = 0.5f;       // the longest base row comes to [2^11, 2^12): a query may be four times as long
+constexpr float kOpen = -9.0e8f;        // the threshold of a query that takes all its columns: below every value, above kNever
+constexpr uint32_t kSampleBlocks = 24;  // sampled blocks of an interval of the mean width
 // One block of so many is sampled at least.  (From one of 130, four values of 100,000 columns had to stand for 500 of them:
 // lists of 1024 overflowed for 673 of 10,000 queries, which went the plain way, 5.3 ms a call; 0.99 now, none redone.)
 constexpr uint32_t kMaxStride = 64;
