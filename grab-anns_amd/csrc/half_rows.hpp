@@ -215,6 +215,7 @@ __device__ __forceinline__ uint32_t share_of(float g, float t, float top, uint32
 // the wave goes over them, packs the pairs that passed and hands them on, 64 at a time.
 constexpr uint32_t kQueueAt = 16;             // entries that set a look at the queue off
 constexpr uint32_t kQueueCap = kQueueAt + 64;  // ... and what the block before that look can add
+constexpr uint32_t kQueueColumns = 1u << 26;   // a column shares a word with its row block, half and register: it must be less
 struct QueueLds {  // a wave's
     uint4 values[kQueueCap * 4];
     uint32_t where[kQueueCap];
@@ -272,7 +273,7 @@ struct PairQueue {
         queued = 0;
         __builtin_amdgcn_wave_barrier();
     }
-    // a block of 32 x 32: rows first + 32 rb .. of the tile, this lane's column j
+    // a block of 32 x 32: rows first + 32 rb .. of the tile, this lane's column j < kQueueColumns
     __device__ __forceinline__ void offer(const v16f& acc, uint32_t j, uint32_t rb) {
         int m = -1;
 #pragma unroll

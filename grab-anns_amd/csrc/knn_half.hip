@@ -833,6 +833,7 @@ int launch_sweep_long(const HalfKnn& h, uint32_t num_cu, hipStream_t st) {
 }  // namespace
 
 bool half_knn_applies(uint64_t n, uint32_t dim, int metric) {
+    static_assert((1u << 23) <= kQueueColumns, "columns of the sweep");
     return n >= 4096 && n <= (1u << 23) && ((metric == kMetricL2 && dim <= 128) || dim % 32 == 0);
 }
 

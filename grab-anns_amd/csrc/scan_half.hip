@@ -139,8 +139,9 @@ struct ScanSink {
     const ScanSweepArgs& a;
     const ScanTables& rows;
     ScanHits& hits;
-    uint32_t row0 = 0;
-    __device__ __forceinline__ void put(float value, uint32_t il, uint32_t j) {
+    uint32_t row0 = 0, col0 = 0;  // first row and column of the item
+    __device__ __forceinline__ void put(float value, uint32_t il, uint32_t col) {
+        const uint32_t j = col0 + col;
         if (j < rows.lo[il] || j >= rows.hi[il]) return;  // (what a row tile sweeps, not every row of it admits)
         const float t = rows.t[il];
         const uint32_t entry = j | share_of(value + t, t, rows.top[il], a.id_bits), slot = atomicAdd(&hits.fill, 1u);
@@ -199,6 +200,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
             s_rows.block_hi[tid >> 5] = hi;
         }
         queue.sink.row0 = row0;
+        queue.sink.col0 = first * 32;
         auto load = [&](v4u* to, uint32_t tile, uint32_t c) {
             const bool norms = c + 1 >= chunks;  // workgroup-uniform
             c = min(c, chunks - 1u);
@@ -282,7 +284,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
                         const uint32_t j0 = min(first + nth * stride, a.last_block) * 32;
 #pragma unroll
                         for (uint32_t rb = 0; rb < 2; ++rb)  // what passes here and no row admits would fall in put()
-                            if (j0 >= from[rb] && j0 < to[rb]) queue.offer(acc[rb][cb], j0 + l32, rb);
+                            if (j0 >= from[rb] && j0 < to[rb]) queue.offer(acc[rb][cb], j0 - first * 32 + l32, rb);  // (row numbers go up to 2^31)
                     }
                 }
                 if (++tile == tiles) break;  // workgroup-uniform
@@ -684,10 +686,12 @@ int half_base_async(const float* data, size_t n, uint32_t dim, int metric, void*
 
 void half_scan_plan(const HalfBase& b, uint32_t num_cu, const uint32_t* h_row_lo, const uint32_t* h_row_hi, HalfScan* s) {
     const uint32_t row_tiles = s->rows / kScanRowsTile;
-    // tiles of 8 blocks, 256 columns; an item is as many as leave every workgroup some four of them, thirty-two at most
+    // tiles of 8 blocks, 256 columns; an item is as many as leave every workgroup some four of them
+    constexpr uint32_t kItemTiles = 32;  // ... at most
+    static_assert(kItemTiles * 256 <= kQueueColumns, "columns of an item");
     uint64_t total = 0;
     for (uint32_t t = 0; t < row_tiles; ++t) total += (s->tile_hi[t] - s->tile_lo[t] + 1) / 2;
-    const uint32_t per = (uint32_t)std::min<uint64_t>(32, std::max<uint64_t>(1, total / (2ull * num_cu * 4)));
+    const uint32_t per = (uint32_t)std::min<uint64_t>(kItemTiles, std::max<uint64_t>(1, total / (2ull * num_cu * 4)));
     std::vector<uint32_t> stride(row_tiles);
     auto blocks_of = [&](uint32_t t) { return 4u * (s->tile_hi[t] - s->tile_lo[t]); };
     uint64_t sampled = 0;

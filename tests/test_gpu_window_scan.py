@@ -1,4 +1,6 @@
 """Exact top-k inside intervals of row ids (grab_window_scan_topk) against the CPU's exact range-filtered scan."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -267,3 +269,34 @@ def test_window_scan_of_wide_intervals(oracle, grab, widths, on_f16):
     eids, edist = oracle.bruteforce_topk(data, q, k, filter_kind=oracle.FILTER_RANGE, ts=np.arange(n, dtype=np.uint64), win_start=lo,
                                          win_end=np.minimum(hi, np.uint64(n)))
     assert np.array_equal(ids, eids) and np.array_equal(dist.view(np.uint32), edist.view(np.uint32))
+
+
+@pytest.mark.parametrize("k", [10, 40])
+def test_scans_beyond_67_million_rows(oracle, grab, k):
+    # 2^26 columns are what the queue's words once held of a row's number: intervals and buckets on either side of that row and
+    # across it, short ones (every column listed) and long ones
+    edge, dim, nq = 1 << 26, 32, 300
+    first, n = edge - 20000, edge + 30000
+    data, q = datasets.gaussian(n - first, dim, 4), datasets.gaussian(nq, dim, 7)
+    d_data, d_q = grab.DeviceArray((n, dim), np.float32), grab.DeviceArray.from_numpy(q)
+    d_data.fill_bytes(0)
+    grab.check(grab.lib.grab_copy_to_device(C.c_void_p(d_data.ptr + first * dim * 4), data.ctypes.data_as(C.c_void_p), C.c_size_t(data.nbytes)))
+    rng = np.random.default_rng(k)
+    width = np.where(np.arange(nq) % 3 == 0, rng.integers(1, 257, nq), rng.integers(12000, 20000, nq))
+    lo = np.where(np.arange(nq) % 2 == 0, rng.integers(edge, n - width), np.maximum(edge - rng.integers(0, width + 1), first)).astype(np.uint64)
+    hi = np.minimum(lo + width.astype(np.uint64), np.uint64(n))
+    base = grab.ScanBase(d_data, n, dim, 0)
+    ids, dist, _ = base.window_topk(d_q, nq, k, lo, hi)
+    own = np.arange(n - first, dtype=np.uint64)
+    eids, edist = oracle.bruteforce_topk(data, q, k, filter_kind=oracle.FILTER_RANGE, ts=own, win_start=lo - np.uint64(first), win_end=hi - np.uint64(first))
+    valid = eids >= 0
+    assert np.array_equal(ids, np.where(valid, eids + first, -1)) and np.array_equal(dist.view(np.uint32)[valid], edist.view(np.uint32)[valid])
+    offsets = np.array([first, edge - 9000, edge - 100, edge + 120, edge + 200, edge + 15000, n], np.uint64)
+    labels = (np.searchsorted(offsets, own + np.uint64(first), side="right") - 1).astype(np.uint8)
+    masks = rng.integers(1, 64, nq).astype(np.uint64)
+    masks[:30] = np.uint64(1 << 3)  # a bucket of 80 rows
+    ids, dist, _ = base.bucket_topk(offsets, d_q, nq, k, masks)
+    base.close()
+    eids, edist = oracle.bruteforce_topk(data, q, k, filter_kind=oracle.FILTER_MASK, labels=labels, masks=masks)
+    valid = eids >= 0
+    assert np.array_equal(ids, np.where(valid, eids + first, -1)) and np.array_equal(dist.view(np.uint32)[valid], edist.view(np.uint32)[valid])
