@@ -136,9 +136,9 @@ template <int WHICH>
 __global__ void __launch_bounds__(256) half_pack_kernel(const float* __restrict__ data, uint64_t n, uint32_t dim, uint32_t ks_count, uint32_t frags,
                                                         float norm_factor, float lift, const float* __restrict__ centre, const float* __restrict__ norm,
                                                         uint32_t* __restrict__ scal, const uint32_t* __restrict__ perm, uint32_t count,
-                                                        uint32_t places, uint4* __restrict__ blocks, float* __restrict__ hn,
+                                                        uint32_t first, uint32_t places, uint4* __restrict__ blocks, float* __restrict__ hn,
                                                         float* __restrict__ eps) {
-    const uint32_t p = (blockIdx.x * 256 + threadIdx.x) >> 4, j = threadIdx.x & 15;
+    const uint32_t p = first + ((blockIdx.x * 256 + threadIdx.x) >> 4), j = threadIdx.x & 15;
     if (p >= places) return;  // whole groups of 16 lanes; places is a multiple of 16
     const float scale = scale_of(__uint_as_float(scal[0])) * lift, unscale = 1.0f / scale;
     const bool live = p < count;
@@ -186,6 +186,15 @@ __global__ void __launch_bounds__(256) half_pack_kernel(const float* __restrict_
         note_largest(e, &scal[1]);
         if (live && !good && j == 0) scal[kScalBad] = 1u;
     }
+}
+// ... a launch has less than 2^32 threads: so many places each
+template <int WHICH>
+void launch_half_pack(const float* data, uint64_t n, uint32_t dim, uint32_t ks_count, uint32_t frags, float norm_factor, float lift, const float* centre, const float* norm,
+                      uint32_t* scal, const uint32_t* perm, uint32_t count, uint32_t places, uint4* blocks, float* hn, float* eps, hipStream_t st) {
+    constexpr uint32_t kPlaces = 1u << 27;
+    for (uint32_t first = 0; first < places; first += kPlaces)
+        hipLaunchKernelGGL(half_pack_kernel<WHICH>, dim3((places - first < kPlaces ? places - first : kPlaces) / 16), dim3(256), 0, st, data, n, dim, ks_count, frags,
+                           norm_factor, lift, centre, norm, scal, perm, count, first, places, blocks, hn, eps);
 }
 
 // the last fragment of a row as the sweeps want it: lane l32 of the lower half holds row l32's pieces of `h`

@@ -905,10 +905,9 @@ int half_knn_lists_async(const float* data, HalfKnn* h, void* workspace, uint32_
     GRAB_HIP(hipMemsetAsync(zeros, 0, ((size_t)places + ks * 16 + kOrderBins + 16) * 4, st));
     if (!h->ip) hipLaunchKernelGGL(half_centre_kernel, dim3(ks * 16), dim3(256), 0, st, data, (uint64_t)n, std::min(n, 8192u), dim, h->centre);
     hipLaunchKernelGGL(half_norms_kernel, dim3(std::min((n + 15) / 16, 2048u)), dim3(256), 0, st, data, n, dim, h->centre, h->cnorm, h->scal);
-    hipLaunchKernelGGL(half_pack_kernel<kSpaced>, dim3(h->sample_places / 16), dim3(256), 0, st, data, (uint64_t)n, dim, ks, h->frags, nf, 1.0f, h->centre, h->cnorm,
-                       h->scal, (const uint32_t*)nullptr, h->n_sample, h->sample_places, h->sample_blocks, sample_hn, (float*)nullptr);
-    hipLaunchKernelGGL(half_pack_kernel<kAll>, dim3(places / 16), dim3(256), 0, st, data, (uint64_t)n, dim, ks, h->frags, nf, 1.0f, h->centre, h->cnorm, h->scal,
-                       (const uint32_t*)nullptr, n, places, h->blocks, h->hn, h->eps);
+    launch_half_pack<kSpaced>(data, n, dim, ks, h->frags, nf, 1.0f, h->centre, h->cnorm, h->scal, nullptr, h->n_sample, h->sample_places, h->sample_blocks, sample_hn,
+                              nullptr, st);
+    launch_half_pack<kAll>(data, n, dim, ks, h->frags, nf, 1.0f, h->centre, h->cnorm, h->scal, nullptr, n, places, h->blocks, h->hn, h->eps, st);
     switch (dim <= 128 ? ks : 0u) {
         case 2: GRAB_TRY(launch_bounds_short<2>(*h, st)); break;
         case 4: GRAB_TRY(launch_bounds_short<4>(*h, st)); break;
@@ -925,8 +924,7 @@ int half_knn_lists_async(const float* data, HalfKnn* h, void* workspace, uint32_
     hipLaunchKernelGGL(order_count_kernel, dim3(order_grid), dim3(1024), bins_lds, st, h->bound, n, h->bins);
     hipLaunchKernelGGL(order_scan_kernel, dim3(1), dim3(1024), 0, st, h->bins);
     hipLaunchKernelGGL(order_place_kernel, dim3(order_grid), dim3(1024), bins_lds, st, h->bound, n, h->bins, h->perm);
-    hipLaunchKernelGGL(half_pack_kernel<kOrdered>, dim3(places / 16), dim3(256), 0, st, data, (uint64_t)n, dim, ks, h->frags, nf, 1.0f, h->centre, h->cnorm, h->scal,
-                       h->perm, n, places, h->blocks, h->hn, (float*)nullptr);
+    launch_half_pack<kOrdered>(data, n, dim, ks, h->frags, nf, 1.0f, h->centre, h->cnorm, h->scal, h->perm, n, places, h->blocks, h->hn, nullptr, st);
     hipLaunchKernelGGL(order_thresholds_kernel, dim3((places + 255) / 256), dim3(256), 0, st, h->bound, h->perm, h->scal, h->hn, n, places, (int)h->ip, h->t_own,
                        h->t_step, h->top);
     GRAB_HIP(hipGetLastError());

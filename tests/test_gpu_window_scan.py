@@ -271,11 +271,11 @@ def test_window_scan_of_wide_intervals(oracle, grab, widths, on_f16):
     assert np.array_equal(ids, eids) and np.array_equal(dist.view(np.uint32), edist.view(np.uint32))
 
 
-@pytest.mark.parametrize("k", [10, 40])
-def test_scans_beyond_67_million_rows(oracle, grab, k):
-    # 2^26 columns are what the queue's words once held of a row's number: intervals and buckets on either side of that row and
-    # across it, short ones (every column listed) and long ones
-    edge, dim, nq = 1 << 26, 32, 300
+@pytest.mark.parametrize("edge,k", [(1 << 26, 10), (1 << 26, 40), (1 << 28, 40)])
+def test_scans_beyond_67_million_rows(oracle, grab, edge, k):
+    # 2^26 columns are what the queue's words once held of a row's number, 2^28 the rows that one launch packs: intervals and
+    # buckets on either side of that row and across it, short ones (every column listed) and long ones
+    dim, nq = 32, 300
     first, n = edge - 20000, edge + 30000
     data, q = datasets.gaussian(n - first, dim, 4), datasets.gaussian(nq, dim, 7)
     d_data, d_q = grab.DeviceArray((n, dim), np.float32), grab.DeviceArray.from_numpy(q)
@@ -287,6 +287,7 @@ def test_scans_beyond_67_million_rows(oracle, grab, k):
     hi = np.minimum(lo + width.astype(np.uint64), np.uint64(n))
     base = grab.ScanBase(d_data, n, dim, 0)
     ids, dist, _ = base.window_topk(d_q, nq, k, lo, hi)
+    assert grab.last_knn_exact_rows() <= 3  # the candidates prove the answers
     own = np.arange(n - first, dtype=np.uint64)
     eids, edist = oracle.bruteforce_topk(data, q, k, filter_kind=oracle.FILTER_RANGE, ts=own, win_start=lo - np.uint64(first), win_end=hi - np.uint64(first))
     valid = eids >= 0
