@@ -1092,8 +1092,14 @@ int launch_refine_any(const RefineArgs& a, int metric, hipStream_t stream) {
     return metric == kMetricIP ? launch_refine<kMetricIP>(a, stream) : launch_refine<kMetricL2>(a, stream);
 }
 
+// Eight lanes a row, and a launch has less than 2^32 of them: so many rows each
+constexpr size_t kLaunchRows = (size_t)1 << 28;
+
 void launch_row_norms(const float* x, size_t n, uint32_t dim, float* out, hipStream_t stream) {
-    hipLaunchKernelGGL(row_norms_kernel, dim3((uint32_t)((n * 8 + 255) / 256)), dim3(256), 0, stream, x, (uint32_t)n, dim, out);
+    for (size_t from = 0; from < n; from += kLaunchRows) {
+        const size_t rows = std::min(n - from, kLaunchRows);
+        hipLaunchKernelGGL(row_norms_kernel, dim3((uint32_t)((rows * 8 + 255) / 256)), dim3(256), 0, stream, x + from * dim, (uint32_t)rows, dim, out + from);
+    }
 }
 
 void launch_max_float(const float* x, uint64_t n, uint32_t* out, hipStream_t stream) {
@@ -1106,7 +1112,11 @@ void launch_spaced_mean(const float* data, uint64_t n, uint32_t count, uint32_t 
 
 void launch_split_rows_chunked(const float* data, uint64_t n, uint32_t dim, const float* mean, uint16_t* out, float* norm,
                                hipStream_t stream) {
-    hipLaunchKernelGGL(split_rows_chunked_kernel, dim3((uint32_t)((n * 8 + 255) / 256)), dim3(256), 0, stream, data, n, dim, mean, out, norm);
+    for (size_t from = 0; from < n; from += kLaunchRows) {
+        const size_t rows = std::min<size_t>(n - from, kLaunchRows);
+        hipLaunchKernelGGL(split_rows_chunked_kernel, dim3((uint32_t)((rows * 8 + 255) / 256)), dim3(256), 0, stream, data + from * dim, (uint64_t)rows, dim, mean,
+                           out + from * dim * 2, norm ? norm + from : nullptr);
+    }
 }
 
 // Rows that the symmetric pass could not serve: the plain pass over them, in as many column slices as fill the machine, the
@@ -1370,12 +1380,10 @@ int exact_topk(const TopkProblem& p, hipStream_t stream, float* kernel_ms) {
     {   // the squared norms: terms of the L2 form, and for both metrics the scale of the rounding error that the
         // check after the re-scoring allows for.  doubt: [0] rows that fail it, [1..M] which, [M+1] max |b|^2
         GRAB_HIP(normB.alloc((size_t)p.N * 4));
-        hipLaunchKernelGGL(row_norms_kernel, dim3((uint32_t)((p.N * 8 + 255) / 256)), dim3(256), 0, stream, p.B,
-                           (uint32_t)p.N, p.dim, normB.as<float>());
+        launch_row_norms(p.B, p.N, p.dim, normB.as<float>(), stream);
         if (!same) {
             GRAB_HIP(normA.alloc((size_t)p.M * 4));
-            hipLaunchKernelGGL(row_norms_kernel, dim3((uint32_t)((p.M * 8 + 255) / 256)), dim3(256), 0, stream, p.A,
-                               (uint32_t)p.M, p.dim, normA.as<float>());
+            launch_row_norms(p.A, p.M, p.dim, normA.as<float>(), stream);
         }
         // [M+2]: max |b|^2 of the rows as split, where they are; then kCounters work counters, one a launch
         GRAB_HIP(doubt.alloc(((size_t)p.M + 3 + kCounters) * 4));

@@ -271,11 +271,12 @@ def test_window_scan_of_wide_intervals(oracle, grab, widths, on_f16):
     assert np.array_equal(ids, eids) and np.array_equal(dist.view(np.uint32), edist.view(np.uint32))
 
 
-@pytest.mark.parametrize("edge,k", [(1 << 26, 10), (1 << 26, 40), (1 << 28, 40)])
-def test_scans_beyond_67_million_rows(oracle, grab, edge, k):
-    # 2^26 columns are what the queue's words once held of a row's number, 2^28 the rows that one launch packs: intervals and
-    # buckets on either side of that row and across it, short ones (every column listed) and long ones
-    dim, nq = 32, 300
+@pytest.mark.parametrize("edge,dim,k", [(1 << 26, 32, 10), (1 << 26, 32, 40), (1 << 28, 32, 40), (1 << 29, 4, 10)])
+def test_scans_beyond_67_million_rows(oracle, grab, edge, dim, k):
+    # 2^26 columns are what the queue's words once held of a row's number, 2^28 the rows that one launch packs, 2^29 those whose
+    # norms one launch took (rows of 4: fp32 instructions): intervals and buckets on either side of that row and across it, short
+    # ones (every column listed) and long ones
+    nq = 300
     first, n = edge - 20000, edge + 30000
     data, q = datasets.gaussian(n - first, dim, 4), datasets.gaussian(nq, dim, 7)
     d_data, d_q = grab.DeviceArray((n, dim), np.float32), grab.DeviceArray.from_numpy(q)
