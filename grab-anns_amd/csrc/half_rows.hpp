@@ -128,10 +128,13 @@ __global__ void __launch_bounds__(256) half_norms_kernel(const float* __restrict
     note_largest(most_plain, scal + kScalPlain);
 }
 
-// Rows into blocks: place p of the output is row p (kAll), row p * n / count (kSpaced) or row perm[p] (kOrdered); places
-// from count on are padding.  hn[p]: squared norm of the rounded, scaled row, -1 for padding and rows that are not finite.
+// Rows into blocks: place p of the output is row p (kAll), row p * n / count (kSpaced), row perm[p] (kOrdered) or one of 2^count
+// rows (kOneOf); places from count (kOneOf: from the last row) on are padding.  hn[p]: squared norm of the rounded, scaled row, -1 for padding and rows that are not finite.
 // lift: a power of two on top of the scale.  kAll: eps[row], how far the row moved when it was rounded (unscaled), and the largest of them in scal[1].  16 lanes a row.
-enum { kAll = 0, kSpaced = 1, kOrdered = 2 };
+enum { kAll = 0, kSpaced = 1, kOrdered = 2, kOneOf = 3 };
+// The row that stands for the rows i << shift .. + 2^shift - 1: any of these, not always the first (rows may come in turns).  At
+// most 2^31 rows.
+__device__ __forceinline__ uint32_t one_of(uint32_t i, uint32_t shift, uint32_t n) { return min((i << shift) + ((i * 0x9E3779B1u) >> (32u - shift)), n - 1u); }
 template <int WHICH>
 __global__ void __launch_bounds__(256) half_pack_kernel(const float* __restrict__ data, uint64_t n, uint32_t dim, uint32_t ks_count, uint32_t frags,
                                                         float norm_factor, float lift, const float* __restrict__ centre, const float* __restrict__ norm,
@@ -141,8 +144,8 @@ __global__ void __launch_bounds__(256) half_pack_kernel(const float* __restrict_
     const uint32_t p = first + ((blockIdx.x * 256 + threadIdx.x) >> 4), j = threadIdx.x & 15;
     if (p >= places) return;  // whole groups of 16 lanes; places is a multiple of 16
     const float scale = scale_of(__uint_as_float(scal[0])) * lift, unscale = 1.0f / scale;
-    const bool live = p < count;
-    const uint32_t row = !live ? 0u : WHICH == kSpaced ? (uint32_t)((uint64_t)p * n / count) : WHICH == kOrdered ? perm[p] : p;
+    const bool live = WHICH == kOneOf ? ((uint64_t)p << count) < n : p < count;
+    const uint32_t row = !live ? 0u : WHICH == kSpaced ? (uint32_t)((uint64_t)p * n / count) : WHICH == kOrdered ? perm[p] : WHICH == kOneOf ? one_of(p, count, (uint32_t)n) : p;
     const bool good = live && norm[row] < 3.0e38f;
     const float* x = data + (size_t)row * dim;
     uint4* block = blocks + (size_t)(p >> 5) * frags * 64 + (p & 31);

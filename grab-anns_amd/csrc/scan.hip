@@ -600,7 +600,7 @@ int scan_topk_half(const float* d_dataset, size_t num_dataset, uint32_t dim, con
     s.k = k;
     s.tile_lo = rw.tile_lo.data();
     s.tile_hi = rw.tile_hi.data();
-    half_scan_plan(*b, num_cu, rw.row_lo.data(), rw.row_hi.data(), &s);
+    if (!half_scan_plan(*b, num_cu, rw.row_lo.data(), rw.row_hi.data(), &s)) return GRAB_OK;
     ScanUpload up;
     up.tab.reserve((size_t)rows * 3 + rw.list_off.size() + rw.lists.size() + s.words.size() + 96);
     const size_t at_rq = up.put(rw.row_query.data(), rows), at_lo = up.put(rw.row_lo.data(), rows), at_hi = up.put(rw.row_hi.data(), rows);

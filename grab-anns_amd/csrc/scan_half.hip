@@ -2,7 +2,7 @@
 // to f16 once (half_rows.hpp), scored and proven exactly like those of the kNN graph (knn_half.hip).
 //
 // A query is one row of the tile grid, or one per interval it admits.  Every row tile (128 rows) sweeps the union of its rows'
-// columns twice: once a few blocks of 32 columns, evenly spaced, whose values are stored and give the query a bound that a
+// columns twice: once a sample of them, one of 8 to 64 neighbours, whose values are stored and give the query a bound that a
 // few hundred of its columns lie within (scan_bound_kernel), then all of them with the bound as threshold - what passes goes
 // through the queue into the row's list, nothing else is ever written.  Writing the values of all columns and selecting from
 // them (lists of 64 keys, k up to 16), or selecting inside the contraction with thresholds that start open (beyond), from
@@ -31,10 +31,14 @@ constexpr uint32_t kScanListCap = 2048;  // entries of a row's list
 constexpr uint32_t kScanSortCap = 1024;  // ... of which a wave sorts the nearest
 constexpr float kScanLift = 0.5f;       // the longest base row comes to [2^11, 2^12): a query may be four times as long
 constexpr float kOpen = -9.0e8f;        // the threshold of a query that takes all its columns: below every value, above kNever
-constexpr uint32_t kSampleBlocks = 24;  // sampled blocks of an interval of the mean width
-// One block of so many is sampled at least.  (From one of 130, four values of 100,000 columns had to stand for 500 of them:
-// lists of 1024 overflowed for 673 of 10,000 queries, which went the plain way, 5.3 ms a call; 0.99 now, none redone.)
-constexpr uint32_t kMaxStride = 64;
+// A tile's queries are bounded by one of 2^shift columns each, kSampleShiftMin to kSampleShiftMax: the most that leaves a row of the
+// tile's mean width 1024 values, but one of 64 at least.  The sampled columns lie apart (one_of), in blocks of their own behind
+// the base's: rows that resemble their neighbours - frames of a scene, a document's passages - are sampled like any others.
+// (Whole blocks of 32 adjacent columns, as it was, stand for nothing but themselves there: 2000 queries in runs of 10, 40 and 200 rows
+// of 500,000 x 128, intervals of 50,000, k 10: 73, 340 and 456 queries not proven, calls of 4.2 - 4.4 ms; none and 0.24 - 0.27 now.
+// The same for intervals of 1500 among those of 100,000, of which every other had no sampled block: 4.46 -> 0.64.)
+constexpr uint32_t kSampleValues = 1024;
+constexpr uint64_t kScanSampleBytes = 4ull << 30;  // the sampled values of a call, at most
 constexpr uint32_t kBoundValues = 2048;  // sampled values that a query looks at, at most: 32 a lane
 
 // Tile-grid rows into blocks, and per query: squared norm of the rounded, scaled row (-1: not taken), what rounding moved it,
@@ -106,8 +110,8 @@ struct ScanSweepArgs {
     const uint4* row_blocks;
     const uint4* row_frags;
     const uint4* blocks;      // base rows
-    const uint32_t* items;    // [4 words]: row tile, first block, stride in blocks, tiles of 8 blocks << 20 | block of the sample
-    const uint32_t* tiles;    // [4 words] per row tile: its sample's place (of 4096 floats), blocks, first block, stride
+    const uint32_t* items;    // [4 words]: row tile, first block, tiles of 8 blocks, block of the sample
+    const uint32_t* tiles;    // [4 words] per row tile: its sample's place (of 4096 floats), blocks, first block among its shift's, shift
     const uint32_t* row_query;
     const uint32_t* row_lo;
     const uint32_t* row_hi;
@@ -179,8 +183,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
         const uint32_t work = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_item);
         if (work >= a.n_items) break;  // workgroup-uniform
         const uint32_t rt = (uint32_t)__builtin_amdgcn_readfirstlane((int)a.items[4 * work]), first = (uint32_t)__builtin_amdgcn_readfirstlane((int)a.items[4 * work + 1]);
-        const uint32_t stride = (uint32_t)__builtin_amdgcn_readfirstlane((int)a.items[4 * work + 2]), more = (uint32_t)__builtin_amdgcn_readfirstlane((int)a.items[4 * work + 3]);
-        const uint32_t tiles = more >> 20, row0 = rt * kScanRowsTile;
+        const uint32_t tiles = (uint32_t)__builtin_amdgcn_readfirstlane((int)a.items[4 * work + 2]), sampled = (uint32_t)__builtin_amdgcn_readfirstlane((int)a.items[4 * work + 3]);
+        const uint32_t row0 = rt * kScanRowsTile;
         if (!SAMPLE && tid < kScanRowsTile) {
             const uint32_t q = a.row_query[row0 + tid];
             s_hits.count[tid] = 0u;
@@ -214,7 +218,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
             const v4u* rb = reinterpret_cast<const v4u*>(a.blocks) + c * 128;
 #pragma unroll
             for (uint32_t i = 0; i < BF; ++i) {
-                const uint32_t at = tid + 256 * i, block = min(first + (8 * tile + (at >> 7)) * stride, a.last_block);  // (the last block is padding)
+                const uint32_t at = tid + 256 * i, block = min(first + 8 * tile + (at >> 7), a.last_block);  // (the base's last block is padding)
                 load_to_lds(rb + (size_t)block * a.frags * 64 + (at & 127u), to + kRowPart + wave * 64 + 256 * i);
             }
         };
@@ -274,14 +278,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
                     const uint32_t nth = 8 * tile + wc * 4 + cb;
                     if (SAMPLE) {
                         const uint32_t* t = a.tiles + 4 * rt;
-                        const uint32_t pitch = t[1] * 32, at = ((more & 0xFFFFFu) + nth) * 32 + l32;
+                        const uint32_t pitch = t[1] * 32, at = (sampled + nth) * 32 + l32;
                         float* out = a.sample + (size_t)t[0] * 4096 + at;
 #pragma unroll
                         for (uint32_t rb = 0; rb < 2; ++rb)
 #pragma unroll
                             for (uint32_t v = 0; v < 16; ++v) out[(size_t)(wr * 64 + rb * 32 + (v & 3) + 8 * (v >> 2) + 4 * half) * pitch] = acc[rb][cb][v];
                     } else {
-                        const uint32_t j0 = min(first + nth * stride, a.last_block) * 32;
+                        const uint32_t j0 = min(first + nth, a.last_block) * 32;
 #pragma unroll
                         for (uint32_t rb = 0; rb < 2; ++rb)  // what passes here and no row admits would fall in put()
                             if (j0 >= from[rb] && j0 < to[rb]) queue.offer(acc[rb][cb], j0 - first * 32 + l32, rb);  // (row numbers go up to 2^31)
@@ -306,11 +310,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
 }
 
-// A query's rows as scan_bound_kernel's lanes hold them, a row a lane: place of the row's sampled values, the interval, the tile's
-// first sampled block and the step between blocks, the first block that touches the interval; n values are looked at, as the
-// at-th and those after it of all that are.
+// A query's rows as scan_bound_kernel's lanes hold them, a row a lane: place of the row's sampled values, the interval, the shift,
+// the tile's first sampled value and the interval's; n values are looked at, as the at-th and those after it of all that are.
 struct SampledRow {
-    uint32_t row = 0, lo = 0, hi = 0, first = 0, stride = 1, b0 = 0, place = 0, pitch = 0, n = 0, at = 0;
+    uint32_t row = 0, lo = 0, hi = 0, shift = kSampleShiftMin, first = 0, s0 = 0, place = 0, pitch = 0, n = 0, at = 0;
 };
 __device__ __forceinline__ uint32_t lane_value(uint32_t v, uint32_t lane) {  // `lane` the same for the whole wave
     return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)lane);
@@ -320,7 +323,7 @@ __device__ __forceinline__ uint32_t lane_value(uint32_t v, uint32_t lane) {  // 
 // on values that are not there: 10,000 intervals 53 -> 33 us, 10,000 queries with 1 - 4 buckets of 1M x 768 152 -> 119.)
 template <int PER, bool ONE>
 __device__ __forceinline__ float scan_threshold(const float* __restrict__ sample, const SampledRow& mine, uint32_t lane, uint32_t nl, uint32_t every, uint32_t n_all,
-                                                uint32_t columns, uint32_t k) {
+                                                uint32_t columns, uint32_t k, uint32_t num_base) {
     const uint32_t rows = ONE ? 1u : nl;
     float v[PER], w[ONE ? 1 : PER];
     uint32_t of[ONE ? 1 : PER];  // the row, or none
@@ -334,16 +337,16 @@ __device__ __forceinline__ float scan_threshold(const float* __restrict__ sample
     }
     uint32_t inside_one = 0;
     for (uint32_t r = 0; r < rows; ++r) {
-        const uint32_t rr = lane_value(mine.row, r), rlo = lane_value(mine.lo, r), rhi = lane_value(mine.hi, r), rf = lane_value(mine.first, r), rs = lane_value(mine.stride, r);
-        const uint32_t rb0 = lane_value(mine.b0, r), rn = lane_value(mine.n, r), rat = lane_value(mine.at, r);
+        const uint32_t rr = lane_value(mine.row, r), rlo = lane_value(mine.lo, r), rhi = lane_value(mine.hi, r), shift = lane_value(mine.shift, r);
+        const uint32_t s0 = lane_value(mine.s0, r), from = s0 - lane_value(mine.first, r), rn = lane_value(mine.n, r), rat = lane_value(mine.at, r);
         const float* src = sample + (size_t)lane_value(mine.place, r) * 4096 + (size_t)(rr % kScanRowsTile) * lane_value(mine.pitch, r);
 #pragma unroll
         for (uint32_t i = 0; i < PER; ++i) {
             if (64 * i < rat + rn && 64 * i + 64 > rat) {  // wave-uniform
-                const uint32_t g = 64 * i + lane - rat, x = g * every, b = rb0 + x / 32, col = (rf + b * rs) * 32 + x % 32;
+                const uint32_t g = 64 * i + lane - rat, col = one_of(s0 + g * every, shift, num_base);
                 const bool in = g < rn && col >= rlo && col < rhi;  // (g wraps round before the row's first value)
                 if (in) {
-                    v[i] = src[b * 32 + x % 32];
+                    v[i] = src[from + g * every];
                     if (!ONE) of[i] = r;
                 }
                 if (ONE) inside_one += (uint32_t)__popcll(__ballot(in));
@@ -366,7 +369,7 @@ __device__ __forceinline__ float scan_threshold(const float* __restrict__ sample
         }
     }
     const float m = (float)k + 9.0f, want = fminf(m + 4.5f * sqrtf(m * weight_max) + 2.0f * weight_max, 800.0f);
-    if ((float)columns <= 1.3f * want) return kOpen;
+    if ((float)columns <= 1.3f * want && columns <= kScanSortCap) return kOpen;
     auto reach = [&](float t) {  // columns that reach t
         if (ONE) {
             uint32_t n = 0;
@@ -413,24 +416,23 @@ __device__ __forceinline__ float scan_threshold(const float* __restrict__ sample
 // column needs to be beyond the k-th by.  A query with few columns takes all.
 __global__ void __launch_bounds__(256) scan_bound_kernel(const float* __restrict__ sample, const uint32_t* __restrict__ tiles, const uint32_t* __restrict__ row_lo,
                                                          const uint32_t* __restrict__ row_hi, const uint32_t* __restrict__ list_off, const uint32_t* __restrict__ lists,
-                                                         const float* __restrict__ q_hn, uint32_t nq, uint32_t k, int ip, float* __restrict__ q_t, float* __restrict__ q_top,
-                                                         uint4* __restrict__ row_frags) {
+                                                         const float* __restrict__ q_hn, uint32_t nq, uint32_t k, int ip, uint32_t num_base, float* __restrict__ q_t,
+                                                         float* __restrict__ q_top, uint4* __restrict__ row_frags) {
     const uint32_t lane = threadIdx.x & 63, q = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (q >= nq) return;  // whole waves
     const uint32_t l0 = list_off[q], nl = list_off[q + 1] - l0;  // at most 64 rows
     if (nl == 0) return;
-    // lane r: row r's interval, and which of its tile's sampled blocks touch it
+    // lane r: row r's interval, and which of its tile's sampled columns stand for it
     SampledRow mine;
-    uint32_t b1 = 0;
+    uint32_t sampled = 0;
     if (lane < nl) {
         mine.row = lists[l0 + lane];
         mine.lo = row_lo[mine.row];
         mine.hi = row_hi[mine.row];
         const uint32_t* t = tiles + 4 * (mine.row / kScanRowsTile);
-        const uint32_t lo = mine.lo, hi = mine.hi, first = t[2], stride = t[3];
-        mine.place = t[0], mine.pitch = t[1] * 32, mine.first = first, mine.stride = stride;
-        mine.b0 = lo / 32 > first ? (lo / 32 - first + stride - 1) / stride : 0u;
-        b1 = max(mine.b0, min(t[1], hi > first * 32 ? ((hi - 1) / 32 - first) / stride + 1 : 0u));
+        mine.place = t[0], mine.pitch = t[1] * 32, mine.first = t[2] * 32, mine.shift = t[3];
+        mine.s0 = mine.lo >> mine.shift;
+        sampled = ((mine.hi - 1) >> mine.shift) + 1 - mine.s0;  // (no row of a list is empty)
     }
     auto wave_sum = [&](uint32_t v) {  // (zero in the lanes that hold no row)
         if (nl == 1) return lane_value(v, 0);
@@ -438,21 +440,21 @@ __global__ void __launch_bounds__(256) scan_bound_kernel(const float* __restrict
         for (int m = 1; m < 64; m <<= 1) v += __shfl_xor(v, m, 64);
         return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
     };
-    const uint32_t columns = wave_sum(mine.hi - mine.lo), all = wave_sum((b1 - mine.b0) * 32);
+    const uint32_t columns = wave_sum(mine.hi - mine.lo), all = wave_sum(sampled);
     const float hn = q_hn[q], top = ip ? sqrtf(fmaxf(hn, 0.0f)) * 4096.0f : 0.0f;
     float t_out = kOpen;
-    if (columns > 256 && all != 0) {
+    if (columns > 256) {
         const uint32_t every = (all + kBoundValues - 65 - 1) / (kBoundValues - 65);  // one value in so many is looked at
-        mine.n = ((b1 - mine.b0) * 32 + every - 1) / every;
+        mine.n = (sampled + every - 1) / every;
         for (uint32_t r = 0; r + 1 < nl; ++r) {
             const uint32_t n_r = lane_value(mine.n, r);
             if (lane > r) mine.at += n_r;
         }
         const uint32_t n_all = wave_sum(mine.n);
-        if (nl == 1 && n_all <= kBoundValues / 2) t_out = scan_threshold<kBoundValues / 128, true>(sample, mine, lane, nl, every, n_all, columns, k);
-        else if (nl == 1) t_out = scan_threshold<kBoundValues / 64, true>(sample, mine, lane, nl, every, n_all, columns, k);
-        else if (n_all <= kBoundValues / 2) t_out = scan_threshold<kBoundValues / 128, false>(sample, mine, lane, nl, every, n_all, columns, k);
-        else t_out = scan_threshold<kBoundValues / 64, false>(sample, mine, lane, nl, every, n_all, columns, k);
+        if (nl == 1 && n_all <= kBoundValues / 2) t_out = scan_threshold<kBoundValues / 128, true>(sample, mine, lane, nl, every, n_all, columns, k, num_base);
+        else if (nl == 1) t_out = scan_threshold<kBoundValues / 64, true>(sample, mine, lane, nl, every, n_all, columns, k, num_base);
+        else if (n_all <= kBoundValues / 2) t_out = scan_threshold<kBoundValues / 128, false>(sample, mine, lane, nl, every, n_all, columns, k, num_base);
+        else t_out = scan_threshold<kBoundValues / 64, false>(sample, mine, lane, nl, every, n_all, columns, k, num_base);
     }
     if (lane == 0) {
         q_t[q] = t_out;
@@ -647,10 +649,14 @@ size_t base_places(size_t n) { return (n + 255) / 256 * 256 + 256; }  // a block
 
 }  // namespace
 
-bool half_scan_takes(uint64_t widest) { return widest <= (uint64_t)(kBoundValues - 65) * kMaxStride; }
+bool half_scan_takes(uint64_t widest) { return widest <= (uint64_t)(kBoundValues - 65) << kSampleShiftMax; }
+
+size_t sample_places(size_t n, uint32_t shift) { return (((n - 1) >> shift) + 32) / 32 * 32; }
 
 size_t half_base_bytes(size_t n, uint32_t dim) {
-    return base_places(n) / 32 * (dim / 16 + 2) * 1024 + base_places(n) * 4 + n * 8 + (size_t)dim * 4 + 16 * 4 + 1024;
+    size_t places = base_places(n);
+    for (uint32_t shift = kSampleShiftMin; shift <= kSampleShiftMax; ++shift) places += sample_places(n, shift);
+    return places / 32 * (dim / 16 + 2) * 1024 + base_places(n) * 4 + n * 8 + (size_t)dim * 4 + 16 * 4 + 1024;
 }
 
 int half_base_async(const float* data, size_t n, uint32_t dim, int metric, void* mem, HalfBase* out, hipStream_t st) {
@@ -669,7 +675,13 @@ int half_base_async(const float* data, size_t n, uint32_t dim, int metric, void*
         m += (bytes + 255) & ~(size_t)255;
         return here;
     };
-    b.blocks = reinterpret_cast<uint4*>(take((size_t)places / 32 * b.frags * 1024));
+    uint32_t blocks = places / 32;
+    for (uint32_t shift = kSampleShiftMin; shift <= kSampleShiftMax; ++shift) {
+        b.sample_first[shift] = blocks;
+        blocks += (uint32_t)sample_places(n, shift) / 32;
+    }
+    b.last_sample_block = blocks - 1;
+    b.blocks = reinterpret_cast<uint4*>(take((size_t)blocks * b.frags * 1024));
     b.centre = reinterpret_cast<float*>(take((size_t)dim * 4 + 64));
     b.scal = reinterpret_cast<uint32_t*>(b.centre + dim);
     float* hn = reinterpret_cast<float*>(take((size_t)places * 4));
@@ -679,11 +691,14 @@ int half_base_async(const float* data, size_t n, uint32_t dim, int metric, void*
     if (!b.ip) hipLaunchKernelGGL(half_centre_kernel, dim3(dim), dim3(256), 0, st, data, (uint64_t)n, (uint32_t)std::min<size_t>(n, 8192), dim, b.centre);
     hipLaunchKernelGGL(half_norms_kernel, dim3((uint32_t)std::min<size_t>((n + 15) / 16, 2048)), dim3(256), 0, st, data, b.n, dim, b.centre, cnorm, b.scal);
     launch_half_pack<kAll>(data, n, dim, b.ks, b.frags, b.ip ? 0.0f : -0.5f, kScanLift, b.centre, cnorm, b.scal, nullptr, b.n, places, b.blocks, hn, eps, st);
+    for (uint32_t shift = kSampleShiftMin; shift <= kSampleShiftMax; ++shift)  // (their norms go where the rows' own were, which nothing reads)
+        launch_half_pack<kOneOf>(data, n, dim, b.ks, b.frags, b.ip ? 0.0f : -0.5f, kScanLift, b.centre, cnorm, b.scal, nullptr, shift, (uint32_t)sample_places(n, shift),
+                                 b.blocks + (size_t)b.sample_first[shift] * b.frags * 64, hn, nullptr, st);
     GRAB_HIP(hipGetLastError());
     return GRAB_OK;
 }
 
-void half_scan_plan(const HalfBase& b, uint32_t num_cu, const uint32_t* h_row_lo, const uint32_t* h_row_hi, HalfScan* s) {
+bool half_scan_plan(const HalfBase& b, uint32_t num_cu, const uint32_t* h_row_lo, const uint32_t* h_row_hi, HalfScan* s) {
     const uint32_t row_tiles = s->rows / kScanRowsTile;
     // tiles of 8 blocks, 256 columns; an item is as many as leave every workgroup some four of them
     constexpr uint32_t kItemTiles = 32;  // ... at most
@@ -691,10 +706,13 @@ void half_scan_plan(const HalfBase& b, uint32_t num_cu, const uint32_t* h_row_lo
     uint64_t total = 0;
     for (uint32_t t = 0; t < row_tiles; ++t) total += (s->tile_hi[t] - s->tile_lo[t] + 1) / 2;
     const uint32_t per = (uint32_t)std::min<uint64_t>(kItemTiles, std::max<uint64_t>(1, total / (2ull * num_cu * 4)));
-    std::vector<uint32_t> stride(row_tiles);
     auto blocks_of = [&](uint32_t t) { return 4u * (s->tile_hi[t] - s->tile_lo[t]); };
+    struct Sampled {
+        uint32_t shift, first, blocks;  // first block among the shift's, blocks in whole tiles
+    };
+    std::vector<Sampled> samples(row_tiles);
     uint64_t sampled = 0;
-    size_t n_sweep = 0, n_sample = 0;
+    size_t n_sweep = 0;
     for (uint32_t t = 0; t < row_tiles; ++t) {
         uint64_t width = 0;
         uint32_t live = 0;
@@ -702,15 +720,16 @@ void half_scan_plan(const HalfBase& b, uint32_t num_cu, const uint32_t* h_row_lo
             width += h_row_hi[r] - h_row_lo[r];  // (never the other way round)
             live += h_row_hi[r] > h_row_lo[r] ? 1u : 0u;
         }
-        stride[t] = std::max({1u, live ? std::min((uint32_t)(width / live / 32 / kSampleBlocks), kMaxStride) : 1u, blocks_of(t) / 4096});
-        sampled += ((blocks_of(t) + stride[t] - 1) / stride[t] + 7) / 8 * 8;
+        Sampled& x = samples[t];
+        x.shift = kSampleShiftMin;
+        while (x.shift < kSampleShiftMax && (width >> x.shift) > (uint64_t)live * kSampleValues) ++x.shift;
+        x.first = (s->tile_lo[t] * 128u >> x.shift) / 32;
+        x.blocks = (((s->tile_hi[t] * 128u - 1u) >> x.shift) / 32 - x.first + 8) / 8 * 8;
+        sampled += x.blocks;
         n_sweep += ((blocks_of(t) + 7) / 8 + per - 1) / per;
     }
-    const uint32_t thin = (uint32_t)std::max<uint64_t>(1, (sampled * 4096 * 4) >> 30);  // the sampled values take a GB at most
-    for (uint32_t t = 0; t < row_tiles; ++t) {
-        stride[t] *= thin;
-        n_sample += ((blocks_of(t) + stride[t] - 1) / stride[t] + 7) / 8;
-    }
+    if (sampled * 4096 * 4 > kScanSampleBytes) return false;
+    const size_t n_sample = sampled / 8;
     s->at_tiles = 0;
     s->at_sweep = (size_t)row_tiles * 4;
     s->at_sample = s->at_sweep + n_sweep * 4;
@@ -722,11 +741,12 @@ void half_scan_plan(const HalfBase& b, uint32_t num_cu, const uint32_t* h_row_lo
         to += 4;
     };
     for (uint32_t t = 0; t < row_tiles; ++t) {
-        const uint32_t first = 4 * s->tile_lo[t], blocks = blocks_of(t), st = stride[t], padded = ((blocks + st - 1) / st + 7) / 8 * 8;
-        for (uint32_t done = 0; done < blocks; done += 8 * per) put(sweep, t, first + done, 1u, std::min(per, (blocks - done + 7) / 8) << 20);
-        for (uint32_t i = 0; i < padded; i += 8) put(sample, t, first + i * st, st, 1u << 20 | i);
-        put(tile, at, padded, first, st);  // a row tile's sample: 128 rows of 32 floats a block
-        at += padded;
+        const uint32_t first = 4 * s->tile_lo[t], blocks = blocks_of(t);
+        const Sampled& x = samples[t];
+        for (uint32_t done = 0; done < blocks; done += 8 * per) put(sweep, t, first + done, std::min(per, (blocks - done + 7) / 8), 0u);
+        for (uint32_t i = 0; i < x.blocks; i += 8) put(sample, t, b.sample_first[x.shift] + x.first + i, 1u, i);
+        put(tile, at, x.blocks, x.first, x.shift);  // a row tile's sample: 128 rows of 32 floats a block
+        at += x.blocks;
     }
     s->sweep_items = (uint32_t)n_sweep;
     s->sample_items = (uint32_t)n_sample;
@@ -734,6 +754,7 @@ void half_scan_plan(const HalfBase& b, uint32_t num_cu, const uint32_t* h_row_lo
     auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
     s->workspace_bytes = up((size_t)s->rows / 32 * b.frags * 1024) + up((size_t)s->rows / 32 * 2048) + up(s->sample_floats * 4) + up((size_t)s->rows * kScanListCap * 4) +
                          up((size_t)s->nq * 28) + up((size_t)s->rows * 4 + 64 + (size_t)s->nq * 4);
+    return true;
 }
 
 int half_scan_async(const HalfBase& b, const HalfScan& s, const HalfScanArgs& given, void* workspace, uint32_t num_cu, uint32_t** left, hipStream_t st) {
@@ -770,15 +791,16 @@ int half_scan_async(const HalfBase& b, const HalfScan& s, const HalfScanArgs& gi
     w.q_t = q_t;
     w.q_top = q_top;
     w.frags = b.frags;
-    w.last_block = b.last_block;
+    w.last_block = b.last_sample_block;
     w.id_bits = 1;
     while ((1ull << w.id_bits) < b.n) ++w.id_bits;
     w.items = a.words + s.at_sample;
     w.n_items = s.sample_items;
     w.work_counter = counters;
     hipLaunchKernelGGL(scan_half_kernel<true>, dim3(std::min(s.sample_items, 2 * num_cu)), dim3(256), 0, st, w);
-    hipLaunchKernelGGL(scan_bound_kernel, dim3((nq + 3) / 4), dim3(256), 0, st, w.sample, w.tiles, a.row_lo, a.row_hi, a.list_off, a.lists, q_hn, nq, s.k, (int)b.ip, q_t, q_top,
+    hipLaunchKernelGGL(scan_bound_kernel, dim3((nq + 3) / 4), dim3(256), 0, st, w.sample, w.tiles, a.row_lo, a.row_hi, a.list_off, a.lists, q_hn, nq, s.k, (int)b.ip, b.n, q_t, q_top,
                        row_frags);
+    w.last_block = b.last_block;
     w.items = a.words + s.at_sweep;
     w.n_items = s.sweep_items;
     w.work_counter = counters + 1;

@@ -121,10 +121,13 @@ int half_knn_finish_async(const float* data, const HalfKnn& h, uint32_t k, const
 
 // Queries against intervals of a row set, on f16 products: scan_half.hip.  The base rows in blocks, made once (mem holds
 // half_base_bytes); whether a row is not finite can be read from scal[11] afterwards.
+constexpr uint32_t kSampleShiftMin = 3, kSampleShiftMax = 6;
 struct HalfBase {
     uint32_t n = 0, dim = 0, ks = 0, frags = 0, last_block = 0;
     bool ip = false;
-    uint4* blocks = nullptr;
+    uint4* blocks = nullptr;  // the rows; from block sample_first[s] on one row of 2^s
+    uint32_t sample_first[kSampleShiftMax + 1] = {};
+    uint32_t last_sample_block = 0;
     float* centre = nullptr;
     uint32_t* scal = nullptr;
 };
@@ -144,7 +147,8 @@ struct HalfScan {
     uint32_t sweep_items = 0, sample_items = 0;
     size_t sample_floats = 0, workspace_bytes = 0;
 };
-void half_scan_plan(const HalfBase& b, uint32_t num_cu, const uint32_t* h_row_lo, const uint32_t* h_row_hi, HalfScan* s);
+// false: the values that the bounds are taken from would need more memory than a call gets
+bool half_scan_plan(const HalfBase& b, uint32_t num_cu, const uint32_t* h_row_lo, const uint32_t* h_row_hi, HalfScan* s);
 // everything queued on `st`: results, and (*left)[0]: whether some query is one that this way does not take (nothing of the
 // results is to be used then), (*left)[1]: the number of queries not proven, from (*left)[2] on: which
 struct HalfScanArgs {

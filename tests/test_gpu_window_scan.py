@@ -302,3 +302,25 @@ def test_scans_beyond_67_million_rows(oracle, grab, edge, dim, k):
     eids, edist = oracle.bruteforce_topk(data, q, k, filter_kind=oracle.FILTER_MASK, labels=labels, masks=masks)
     valid = eids >= 0
     assert np.array_equal(ids, np.where(valid, eids + first, -1)) and np.array_equal(dist.view(np.uint32)[valid], edist.view(np.uint32)[valid])
+
+
+@pytest.mark.parametrize("run,k,widths", [(10, 10, (8000, 12000)), (40, 10, (40000, 60000)), (200, 40, (40000, 60000)), (1, 10, None)])
+def test_window_scan_of_rows_that_resemble_their_neighbours(oracle, grab, run, k, widths):
+    # rows in runs (frames of a scene), the query's run inside its interval; last, intervals of 1500 among long ones: what a query is
+    # bounded by is sampled from all of its interval, so that next to no query's candidates fail to prove the answer
+    n, dim, nq = 140000, 32, 1030
+    rng = np.random.default_rng(run)
+    scenes = datasets.gaussian((n + run - 1) // run, dim, 4) * np.float32(8.0)
+    data = np.repeat(scenes, run, axis=0)[:n] + datasets.gaussian(n, dim, 5)
+    own = rng.integers(0, n, nq)
+    q = data[own] + datasets.gaussian(nq, dim, 6)
+    width = rng.integers(widths[0], widths[1], nq) if widths else np.where(np.arange(nq) % 2, 1500, 90000)
+    lo = np.clip(own - (rng.random(nq) * width).astype(np.int64), 0, n - width).astype(np.uint64)
+    hi = lo + width.astype(np.uint64)
+    d_data, d_q = grab.DeviceArray.from_numpy(data), grab.DeviceArray.from_numpy(q)
+    base = grab.ScanBase(d_data, n, dim, 0)
+    ids, dist, _ = base.window_topk(d_q, nq, k, lo, hi)
+    assert grab.last_knn_exact_rows() <= 5
+    base.close()
+    eids, edist = oracle.bruteforce_topk(data, q, k, filter_kind=oracle.FILTER_RANGE, ts=np.arange(n, dtype=np.uint64), win_start=lo, win_end=hi)
+    assert np.array_equal(ids, eids) and np.array_equal(dist.view(np.uint32), edist.view(np.uint32))
