@@ -132,3 +132,25 @@ def test_bucket_scan_on_f16_rows_with_many_buckets_a_query(oracle, grab, n, dim,
     assert grab.last_knn_bf16_flop() > 0
     eids, edist = oracle.bruteforce_topk(data, q, k, metric=metric, filter_kind=oracle.FILTER_MASK, labels=labels.astype(np.uint8), masks=masks)
     assert np.array_equal(ids, eids) and np.array_equal(dist.view(np.uint32), edist.view(np.uint32))
+
+
+@pytest.mark.parametrize("k", [10, 128])
+def test_bucket_scan_of_large_buckets(oracle, grab, k):
+    # a query's sixty pieces list 900 columns give or take 600: as many as a wave scores, as it holds, and more, of which it takes
+    # the nearest
+    n, dim, nq = 1_000_000, 32, 300
+    data, q = datasets.gaussian(n, dim, 4), datasets.gaussian(nq, dim, 7)
+    offsets = np.array([0, 400_000, 400_050, 950_000, n], np.uint64)
+    masks = np.where(np.arange(nq) % 2, np.uint64(5), np.uint64(7)).astype(np.uint64)
+    d_data, d_q = grab.DeviceArray.from_numpy(data), grab.DeviceArray.from_numpy(q)
+    base = grab.ScanBase(d_data, n, dim, 0)
+    ids, dist, _ = base.bucket_topk(offsets, d_q, nq, k, masks)
+    if k == 10:
+        assert grab.last_knn_exact_rows() <= 5
+    base.close()
+    labels = np.repeat(np.arange(4, dtype=np.uint8), np.diff(offsets.astype(np.int64)))
+    gids, gdist, _ = grab.bruteforce_topk(d_data, n, dim, d_q, nq, k, filter_kind=grab.FILTER_MASK, d_labels=grab.DeviceArray.from_numpy(labels),
+                                          d_masks=grab.DeviceArray.from_numpy(masks))
+    assert np.array_equal(ids, gids) and np.array_equal(dist.view(np.uint32), gdist.view(np.uint32))
+    eids, _ = oracle.bruteforce_topk(data, q[:8], k, filter_kind=oracle.FILTER_MASK, labels=labels, masks=masks[:8])
+    assert np.array_equal(ids[:8], eids)
