@@ -288,6 +288,12 @@ def last_knn_bf16_flop():
     return float(lib.grab_last_knn_bf16_flop())
 
 
+def last_knn_f16_flop():
+    """grab_last_knn_f16_flop: matrix operations on f16 rows of the last kNN graph or scan (0 where none were taken)."""
+    lib.grab_last_knn_f16_flop.restype = C.c_double
+    return float(lib.grab_last_knn_f16_flop())
+
+
 def knn_allow_bf16(allow):
     """grab_knn_allow_bf16: may kNN graphs form their candidates on bf16 instructions (default yes); returns the previous setting."""
     return bool(lib.grab_knn_allow_bf16(1 if allow else 0))

@@ -568,11 +568,12 @@ int unproven_queries(const float* d_dataset, size_t num_dataset, uint32_t dim, c
     hipLaunchKernelGGL(gather_query_rows_kernel, dim3((uint32_t)(((size_t)n_doubt * 8 + 255) / 256)), dim3(256), 0, st, d_queries,
                        d_which.as<uint32_t>(), n_doubt, dim, sub_q.as<float>());
     GRAB_HIP(hipGetLastError());
-    const double flop_fp32 = knn_stats().flop, flop_bf16 = knn_stats().flop_bf16;
+    const double flop_fp32 = knn_stats().flop, flop_bf16 = knn_stats().flop_bf16, flop_f16 = knn_stats().flop_f16;
     GRAB_TRY(bucket_scan_by_rows(d_dataset, num_dataset, dim, sub, sub_q.as<float>(), n_doubt, k, metric, sub_ids.as<int64_t>(),
                                  sub_dist.as<float>(), st));
     knn_stats().flop = flop_fp32;  // the figures of the main pass
     knn_stats().flop_bf16 = flop_bf16;
+    knn_stats().flop_f16 = flop_f16;
     knn_stats().exact_rows = n_doubt;
     hipLaunchKernelGGL(scatter_results_kernel, dim3((n_doubt * k + 255) / 256), dim3(256), 0, st, sub_ids.as<int64_t>(), sub_dist.as<float>(),
                        d_which.as<uint32_t>(), n_doubt, k, d_out_indices, d_out_dists);
@@ -641,7 +642,8 @@ int scan_topk_half(const float* d_dataset, size_t num_dataset, uint32_t dim, con
     }
     if (left[0] != 0 || bad != 0) return GRAB_OK;
     *applied = true;
-    knn_stats().flop_bf16 = 3.0 * rw.tiles * 2.0 * TM * TN * dim;
+    knn_stats().flop_f16 = rw.tiles * 2.0 * TM * TN * dim;
+    knn_stats().flop_bf16 = 3.0 * knn_stats().flop_f16;
     knn_stats().exact_rows = left[1];
     if (left[1] == 0) return GRAB_OK;
     return unproven_queries(d_dataset, num_dataset, dim, sub_rows, d_queries, k, metric, w + 1, left[1], d_out_indices, d_out_dists, st);
@@ -655,7 +657,7 @@ int scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const Sc
               const float* d_queries, size_t num_queries, uint32_t k, int metric, int64_t* d_out_indices, float* d_out_dists,
               float* kernel_ms, hipStream_t st, const ScanBase* base = nullptr) {
     const uint32_t rows = rw.rows, nq = (uint32_t)num_queries;
-    knn_stats().flop = knn_stats().flop_bf16 = 0.0;
+    knn_stats().flop = knn_stats().flop_bf16 = knn_stats().flop_f16 = 0.0;
     knn_stats().redone_rows = knn_stats().exact_rows = 0;
     if (rows == 0) {  // no query admits a row
         std::vector<int64_t> ids(num_queries * (size_t)k, -1);

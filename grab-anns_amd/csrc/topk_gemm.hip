@@ -1242,7 +1242,8 @@ static int knn_graph_half(const TopkProblem& p, uint32_t kk, uint32_t num_cu, bo
     GRAB_HIP(hipGetLastError());
     const double tile_flop = 2.0 * TM * TN * (fp32_redo ? 128 : p.dim);
     knn_stats().flop = 0.0;
-    knn_stats().flop_bf16 = 3.0 * tile_flop * (0.5 * tiles * (tiles + 1.0) + (double)tiles * ((h.n_sample + TN - 1) / TN));
+    knn_stats().flop_f16 = tile_flop * (0.5 * tiles * (tiles + 1.0) + (double)tiles * ((h.n_sample + TN - 1) / TN));
+    knn_stats().flop_bf16 = 3.0 * knn_stats().flop_f16;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (kernel_ms) {
         GRAB_HIP(hipEventCreate(&e0));
@@ -1365,7 +1366,7 @@ int exact_topk(const TopkProblem& p, hipStream_t stream, float* kernel_ms) {
     const double tile_flop = 2.0 * TM * TN * p.dim;
     knn_stats().redone_rows = 0;
     knn_stats().exact_rows = 0;
-    knn_stats().flop_bf16 = 0.0;
+    knn_stats().flop_bf16 = knn_stats().flop_f16 = 0.0;
     knn_stats().flop = tile_flop * (sym ? 0.5 * row_tiles * (row_tiles + 1.0) : (double)row_tiles * col_tiles);
 
     DeviceScratch buf, cand, normA, normB, doubt;
@@ -1608,6 +1609,8 @@ int grab_last_knn_stats(double* flop, uint64_t* rows_redone) {
 uint64_t grab_last_knn_exact_rows(void) { return knn_stats().exact_rows; }
 
 double grab_last_knn_bf16_flop(void) { return knn_stats().flop_bf16; }
+
+double grab_last_knn_f16_flop(void) { return knn_stats().flop_f16; }
 
 int grab_knn_allow_bf16(int allow) { return g_knn_bf16.exchange(allow != 0 ? 1 : 0, std::memory_order_relaxed); }
 

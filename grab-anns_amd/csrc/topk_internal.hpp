@@ -172,6 +172,7 @@ int half_scan_async(const HalfBase& b, const HalfScan& s, const HalfScanArgs& a,
 struct KnnStats {
     double flop = 0.0;          // fp32 matrix instructions
     double flop_bf16 = 0.0;     // half-precision matrix instructions, counted as the three that a product of split rows takes
+    double flop_f16 = 0.0;      // ... those of f16 rows among them, as executed
     uint64_t redone_rows = 0;   // rows the symmetric pass handed to the plain pass
     uint64_t exact_rows = 0;    // rows (queries) that their candidates did not prove and an exact pass redid
 };

@@ -442,6 +442,8 @@ uint64_t grab_last_knn_exact_rows(void);
  * Returns the calling thread's last call's half-precision floating-point operations, which grab_last_knn_stats leaves out,
  * counted as the three bf16 instructions that a product of split rows takes (f16 rows execute a third of it). */
 double grab_last_knn_bf16_flop(void);
+/* ... those of them that ran on f16 rows, as executed; 0 where the last graph or scan of the calling thread took none. */
+double grab_last_knn_f16_flop(void);
 /* No counterpart in the reference.  Process-wide switch, on by default: with 0 every kNN graph forms its candidates
  * on fp32 matrix instructions (bounding pass and symmetric pass of tile_topk_kernel), whatever its metric and
  * dimension; the graphs are the same either way.  Returns the previous setting. */

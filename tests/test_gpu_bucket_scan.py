@@ -129,7 +129,7 @@ def test_bucket_scan_on_f16_rows_with_many_buckets_a_query(oracle, grab, n, dim,
     masks = np.array([np.bitwise_or.reduce(np.uint64(1) << rng.choice(nb, per_query, replace=False).astype(np.uint64)) for _ in range(nq)], np.uint64)
     d_data, d_q = grab.DeviceArray.from_numpy(data), grab.DeviceArray.from_numpy(q)
     ids, dist, _ = grab.bucket_scan_topk(d_data, n, dim, offsets, d_q, nq, k, masks, metric=metric)
-    assert grab.last_knn_bf16_flop() > 0
+    assert grab.last_knn_f16_flop() > 0
     eids, edist = oracle.bruteforce_topk(data, q, k, metric=metric, filter_kind=oracle.FILTER_MASK, labels=labels.astype(np.uint8), masks=masks)
     assert np.array_equal(ids, eids) and np.array_equal(dist.view(np.uint32), edist.view(np.uint32))
 
@@ -145,6 +145,7 @@ def test_bucket_scan_of_large_buckets(oracle, grab, k):
     d_data, d_q = grab.DeviceArray.from_numpy(data), grab.DeviceArray.from_numpy(q)
     base = grab.ScanBase(d_data, n, dim, 0)
     ids, dist, _ = base.bucket_topk(offsets, d_q, nq, k, masks)
+    assert grab.last_knn_f16_flop() > 0
     if k == 10:
         assert grab.last_knn_exact_rows() <= 5
     base.close()

@@ -243,7 +243,7 @@ def test_window_scan_on_f16_rows(oracle, grab, n, dim, nq, k, metric, widths, ki
     d_data, d_q = grab.DeviceArray.from_numpy(data), grab.DeviceArray.from_numpy(q)
     base = grab.ScanBase(d_data, len(data), dim, metric)
     ids, dist, _ = base.window_topk(d_q, nq, k, lo, hi)
-    assert grab.last_knn_bf16_flop() > 0
+    assert (grab.last_knn_f16_flop() > 0) == (kind != "far") and grab.last_knn_bf16_flop() > 0
     base.close()
     eids, edist = oracle.bruteforce_topk(data, q, k, metric=metric, filter_kind=oracle.FILTER_RANGE, ts=np.arange(len(data), dtype=np.uint64),
                                          win_start=lo, win_end=np.minimum(hi, np.uint64(len(data))))
@@ -263,6 +263,7 @@ def test_window_scan_of_wide_intervals(oracle, grab, widths, on_f16):
     d_data, d_q = grab.DeviceArray.from_numpy(data), grab.DeviceArray.from_numpy(q)
     base = grab.ScanBase(d_data, n, dim, 0)
     ids, dist, _ = base.window_topk(d_q, nq, k, lo, hi)
+    assert (grab.last_knn_f16_flop() > 0) == on_f16 and grab.last_knn_bf16_flop() > 0
     if on_f16:
         assert grab.last_knn_exact_rows() <= 5
     base.close()
@@ -288,7 +289,7 @@ def test_scans_beyond_67_million_rows(oracle, grab, edge, dim, k):
     hi = np.minimum(lo + width.astype(np.uint64), np.uint64(n))
     base = grab.ScanBase(d_data, n, dim, 0)
     ids, dist, _ = base.window_topk(d_q, nq, k, lo, hi)
-    assert grab.last_knn_exact_rows() <= 3  # the candidates prove the answers
+    assert grab.last_knn_exact_rows() <= 3 and (grab.last_knn_f16_flop() > 0) == (dim % 32 == 0)  # the candidates prove the answers
     own = np.arange(n - first, dtype=np.uint64)
     eids, edist = oracle.bruteforce_topk(data, q, k, filter_kind=oracle.FILTER_RANGE, ts=own, win_start=lo - np.uint64(first), win_end=hi - np.uint64(first))
     valid = eids >= 0
@@ -320,7 +321,7 @@ def test_window_scan_of_rows_that_resemble_their_neighbours(oracle, grab, run, k
     d_data, d_q = grab.DeviceArray.from_numpy(data), grab.DeviceArray.from_numpy(q)
     base = grab.ScanBase(d_data, n, dim, 0)
     ids, dist, _ = base.window_topk(d_q, nq, k, lo, hi)
-    assert grab.last_knn_exact_rows() <= 5
+    assert grab.last_knn_exact_rows() <= 5 and grab.last_knn_f16_flop() > 0
     base.close()
     eids, edist = oracle.bruteforce_topk(data, q, k, filter_kind=oracle.FILTER_RANGE, ts=np.arange(n, dtype=np.uint64), win_start=lo, win_end=hi)
     assert np.array_equal(ids, eids) and np.array_equal(dist.view(np.uint32), edist.view(np.uint32))
