@@ -675,11 +675,15 @@ int scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const Sc
     // a prepared base has paid for its split rows; otherwise splitting a million rows pays from a thousand query rows on
     const bool split = base ? base->split
                             : knn_bf16_allowed() && dim % KC == 0 && rows >= 1024 && num_dataset >= 4096;
-    // On f16 rows, except narrow intervals with short lists: there half of an interval's columns would be sampled and a fifth of
-    // them listed, and writing all values costs less.  A call over a prepared base, stored values against this way, k 10: 10,000
-    // intervals of 1000 of 1M x 128 384 against 582 us, of 6000 529 / 473, of 10,000 639 / 494; of 250 of 50,000 x 384 244 / 778.
-    // Longer lists, selection inside the contraction against this: k 40, 10,000 columns 2913 / 554, 250 of 50,000 x 384 2183 / 771.
-    const bool narrow = rw.one_row_per_query && kk <= 64 && rw.columns < 6000ull * rw.lists.size();
+    // On f16 rows, except narrow intervals with short lists: a tenth of an interval's columns would be listed, and writing all values
+    // costs less.  A call over a prepared base, stored values against this way in us, k 10, intervals of 1000, 4000, 6000 and 8000:
+    //   1M x 128, 100 queries     221 / 243, 230 / 223, 236 / 215, 241 / 212      150,000 x 768  197 / 198, 209 / 199, 213 / 193, 219 / 196
+    //   400,000 x 96, 100         119 / 145, 130 / 136, 134 / 134, 140 / 134      200,000 x 384  151 / 168, 161 / 157, 166 / 156, 172 / 157
+    // Where the lines cross moves with the batch: 3000 at 10,000 queries (430 / 406 of 1M x 128), 6000 from eight to a thousand, 10,000
+    // for one or two, which wait for this way's one launch more: one query, intervals of 6000, 8000 and 12,000 81 / 86, 86 / 88, 94 / 95
+    // of 1M x 128 and 114 / 127, 117 / 123, 125 / 130 of 150,000 x 768.
+    // Longer lists, selection inside the contraction against this: k 40, 10,000 queries, 1000 columns 1361 / 472, 20,000 3743 / 574.
+    const bool narrow = rw.one_row_per_query && kk <= 64 && rw.columns < (rw.lists.size() <= 2 ? 10000ull : 6000ull) * rw.lists.size();
     // Beyond 127,000 columns a sampled value stands for more than 64 columns, too few lie within a bound to set it by; by the same
     // reckoning as at 100,000 from one in 130 (scan_half.hip: 5.3 ms a call against 3.3 with stored values).
     if (split && !narrow && half_scan_takes(rw.widest) && (!base || base->half)) {

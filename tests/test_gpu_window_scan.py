@@ -325,3 +325,17 @@ def test_window_scan_of_rows_that_resemble_their_neighbours(oracle, grab, run, k
     base.close()
     eids, edist = oracle.bruteforce_topk(data, q, k, filter_kind=oracle.FILTER_RANGE, ts=np.arange(n, dtype=np.uint64), win_start=lo, win_end=hi)
     assert np.array_equal(ids, eids) and np.array_equal(dist.view(np.uint32), edist.view(np.uint32))
+
+
+@pytest.mark.parametrize("nq,width,k,on_f16", [(1, 9999, 10, False), (1, 10000, 16, True), (2, 9000, 10, False), (3, 6000, 10, True), (3, 5999, 16, False), (3, 300, 17, True)])
+def test_window_scan_of_few_queries(oracle, grab, nq, width, k, on_f16):
+    # narrow intervals with short lists keep the way of stored values, and narrower than ten thousand is narrow for one or two
+    n, dim = 30000, 64
+    data, q = datasets.gaussian(n, dim, 4), datasets.gaussian(nq, dim, 7)
+    lo, hi = _intervals(n, nq, width, width, nq)
+    base = grab.ScanBase(grab.DeviceArray.from_numpy(data), n, dim, 0)
+    ids, dist, _ = base.window_topk(grab.DeviceArray.from_numpy(q), nq, k, lo, hi)
+    assert (grab.last_knn_f16_flop() > 0) == on_f16 and grab.last_knn_bf16_flop() > 0
+    base.close()
+    eids, edist = oracle.bruteforce_topk(data, q, k, filter_kind=oracle.FILTER_RANGE, ts=np.arange(n, dtype=np.uint64), win_start=lo, win_end=hi)
+    assert np.array_equal(ids, eids) and np.array_equal(dist.view(np.uint32), edist.view(np.uint32))
