@@ -53,10 +53,11 @@ inline uint64_t splitmix64(uint64_t* state) {
 // A caller that runs the same allocating routine many times in a row (the buckets of the time-partitioned graph: a
 // dozen allocations and frees per bucket, each a wait for the device) can lend the calling thread one block of device
 // memory: while an arena is set, DeviceScratch takes its memory from it, bump-allocated, and gives nothing back; the
-// caller rewinds it between runs.  What does not fit is allocated as ever.  `wanted` adds up what was asked for.
+// caller rewinds it between runs.  What does not fit is allocated as ever.  `wanted` adds up what was asked for; who rewinds within
+// a run notes the most that was in `peak`.
 struct ScratchArena {
     char* base = nullptr;
-    size_t cap = 0, used = 0, wanted = 0;
+    size_t cap = 0, used = 0, wanted = 0, peak = 0;
 };
 ScratchArena*& scratch_arena();  // of the calling thread; null by default
 

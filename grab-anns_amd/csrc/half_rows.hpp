@@ -6,6 +6,7 @@
 #include <cstdint>
 
 #include "device_utils.hpp"
+#include "topk_internal.hpp"
 
 namespace grab {
 namespace {
@@ -95,7 +96,6 @@ __device__ __forceinline__ void note_largest(float v, uint32_t* out) {
     if ((threadIdx.x & 63) == 0 && __float_as_uint(v) > __atomic_load_n(out, __ATOMIC_RELAXED)) atomicMax(out, __float_as_uint(v));
 }
 
-constexpr uint32_t kScalBad = 11, kScalPlain = 12;  // scal[11]: whether some row is not finite (half_pack_kernel<kAll>)
 // squared norm of every centred row, and the largest finite one (scal[0], as bits); scal[kScalPlain]: the largest of the rows as
 // they are; 16 lanes a row
 __global__ void __launch_bounds__(256) half_norms_kernel(const float* __restrict__ data, uint32_t n, uint32_t dim,

@@ -582,33 +582,56 @@ int unproven_queries(const float* d_dataset, size_t num_dataset, uint32_t dim, c
     return GRAB_OK;
 }
 
-// The f16 way (scan_half.hip).  *applied = false: a query or a row that it does not take, and nothing is to be used of it.
-int scan_topk_half(const float* d_dataset, size_t num_dataset, uint32_t dim, const ScanRows& rw, const SubRows& sub_rows, const float* d_queries,
-                   size_t num_queries, uint32_t k, int metric, int64_t* d_out_indices, float* d_out_dists, float* kernel_ms, hipStream_t st,
-                   const ScanBase* base, uint32_t num_cu, bool* applied) {
-    const uint32_t rows = rw.rows, nq = (uint32_t)num_queries;
-    DeviceScratch base_mem, d_tab, ws;
-    HalfBase own;
-    const HalfBase* b = base ? base->half : &own;
+// One pass of the f16 way (scan_half.hip) over queries [first, first + nq) of the call, whose rows are `rw`; its kernels' time is added
+// to *kernel_ms.  *applied = false: a query or a row that this way does not take, or no room.
+constexpr size_t kHalfPassBytes = (size_t)4 << 30;  // device memory of a pass: what the other way's passes take
+constexpr uint32_t kHalfPassQueries = 128;          // ... which fewer queries than these are not split for
+int scan_half_pass(const HalfBase& b, const float* d_dataset, size_t num_dataset, const ScanRows& rw, const SubRows& sub_rows, const float* d_queries, uint32_t first,
+                   uint32_t nq, uint32_t k, int metric, int64_t* d_out_indices, float* d_out_dists, float* kernel_ms, hipStream_t st, const ScanBase* base,
+                   uint32_t num_cu, bool* applied) {
+    const uint32_t rows = rw.rows, dim = b.dim;
     *applied = false;
-    if (!base) {
-        GRAB_HIP(base_mem.alloc(half_base_bytes(num_dataset, dim)));
-        GRAB_TRY(half_base_async(d_dataset, num_dataset, dim, metric, base_mem.ptr, &own, st));
-    }
     HalfScan s;
     s.rows = rows;
     s.nq = nq;
     s.k = k;
     s.tile_lo = rw.tile_lo.data();
     s.tile_hi = rw.tile_hi.data();
-    if (!half_scan_plan(*b, num_cu, rw.row_lo.data(), rw.row_hi.data(), &s)) return GRAB_OK;
+    if (!half_scan_plan(b, num_cu, rw.row_lo.data(), rw.row_hi.data(), kHalfPassBytes, &s)) {
+        if (nq <= kHalfPassQueries) return GRAB_OK;
+        for (uint32_t part = 0; part < 2; ++part) {
+            const uint32_t from = part == 0 ? first : first + nq / 2, count = part == 0 ? nq / 2 : nq - nq / 2;
+            std::vector<uint32_t> which(count);
+            for (uint32_t i = 0; i < count; ++i) which[i] = from + i;
+            ScanRows half;
+            sub_rows(which, &half);
+            GRAB_TRY(scan_half_pass(b, d_dataset, num_dataset, half, sub_rows, d_queries, from, count, k, metric, d_out_indices, d_out_dists, kernel_ms, st, base, num_cu,
+                                    applied));
+            if (!*applied) return GRAB_OK;
+        }
+        return GRAB_OK;
+    }
+    struct Rewind {  // a pass is through with its scratch when it returns: the next one gets the same
+        ScratchArena* const arena = scratch_arena();
+        const size_t used = arena ? arena->used : 0, wanted = arena ? arena->wanted : 0;
+        ~Rewind() {
+            if (!arena) return;
+            arena->peak = std::max(arena->peak, arena->wanted);
+            arena->used = used;
+            arena->wanted = wanted;
+        }
+    } rewind;
+    DeviceScratch d_tab, ws;
     ScanUpload up;
     up.tab.reserve((size_t)rows * 3 + rw.list_off.size() + rw.lists.size() + s.words.size() + 96);
     const size_t at_rq = up.put(rw.row_query.data(), rows), at_lo = up.put(rw.row_lo.data(), rows), at_hi = up.put(rw.row_hi.data(), rows);
     const size_t at_loff = up.put(rw.list_off.data(), rw.list_off.size()), at_lists = up.put(rw.lists.data(), rw.lists.size());
     const size_t at_words = up.put(s.words.data(), s.words.size());
+    if (ws.alloc(s.workspace_bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return GRAB_OK;
+    }
     GRAB_TRY(up.upload(base, &d_tab, st));
-    GRAB_HIP(ws.alloc(s.workspace_bytes));
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (kernel_ms) {
         GRAB_HIP(hipEventCreate(&e0));
@@ -617,23 +640,24 @@ int scan_topk_half(const float* d_dataset, size_t num_dataset, uint32_t dim, con
     }
     HalfScanArgs a{};
     a.data = d_dataset;
-    a.queries = d_queries;
+    a.queries = d_queries + (size_t)first * dim;
     a.row_query = d_tab.as<uint32_t>() + at_rq;
     a.row_lo = d_tab.as<uint32_t>() + at_lo;
     a.row_hi = d_tab.as<uint32_t>() + at_hi;
     a.list_off = d_tab.as<uint32_t>() + at_loff;
     a.lists = d_tab.as<uint32_t>() + at_lists;
     a.words = d_tab.as<uint32_t>() + at_words;
-    a.out_ids = d_out_indices;
-    a.out_dist = d_out_dists;
+    a.out_ids = d_out_indices + (size_t)first * k;
+    a.out_dist = d_out_dists + (size_t)first * k;
     a.contraction_done = e1;
     uint32_t* w = nullptr;
-    int rc = half_scan_async(*b, s, a, ws.ptr, num_cu, &w, st);
+    float ms = 0.0f;
+    int rc = half_scan_async(b, s, a, ws.ptr, num_cu, &w, st);
     uint32_t left[2] = {0, 0}, bad = 0;
     if (rc == GRAB_OK && hipMemcpyAsync(left, w, 8, hipMemcpyDeviceToHost, st) != hipSuccess) rc = GRAB_ERR_HIP;
-    if (rc == GRAB_OK && !base && hipMemcpyAsync(&bad, own.scal + 11, 4, hipMemcpyDeviceToHost, st) != hipSuccess) rc = GRAB_ERR_HIP;
+    if (rc == GRAB_OK && !base && hipMemcpyAsync(&bad, b.scal + kScalBad, 4, hipMemcpyDeviceToHost, st) != hipSuccess) rc = GRAB_ERR_HIP;
     if (hipStreamSynchronize(st) != hipSuccess && rc == GRAB_OK) rc = GRAB_ERR_HIP;
-    if (rc == GRAB_OK && kernel_ms && hipEventElapsedTime(kernel_ms, e0, e1) != hipSuccess) rc = GRAB_ERR_HIP;
+    if (rc == GRAB_OK && kernel_ms && hipEventElapsedTime(&ms, e0, e1) != hipSuccess) rc = GRAB_ERR_HIP;
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
     if (rc != GRAB_OK) {
@@ -642,11 +666,43 @@ int scan_topk_half(const float* d_dataset, size_t num_dataset, uint32_t dim, con
     }
     if (left[0] != 0 || bad != 0) return GRAB_OK;
     *applied = true;
-    knn_stats().flop_f16 = rw.tiles * 2.0 * TM * TN * dim;
+    if (kernel_ms) *kernel_ms += ms;
+    knn_stats().flop_f16 += rw.tiles * 2.0 * TM * TN * dim;
     knn_stats().flop_bf16 = 3.0 * knn_stats().flop_f16;
-    knn_stats().exact_rows = left[1];
     if (left[1] == 0) return GRAB_OK;
-    return unproven_queries(d_dataset, num_dataset, dim, sub_rows, d_queries, k, metric, w + 1, left[1], d_out_indices, d_out_dists, st);
+    const uint64_t exact_before = knn_stats().exact_rows;
+    const SubRows own_rows = [&](const std::vector<uint32_t>& which, ScanRows* out) {
+        std::vector<uint32_t> of_call(which);
+        for (uint32_t& q : of_call) q += first;
+        sub_rows(of_call, out);
+    };
+    GRAB_TRY(unproven_queries(d_dataset, num_dataset, dim, own_rows, a.queries, k, metric, w + 1, left[1], a.out_ids, a.out_dist, st));
+    knn_stats().exact_rows += exact_before;
+    return GRAB_OK;
+}
+
+// The f16 way.  *applied = false: nothing is to be used of it.
+int scan_topk_half(const float* d_dataset, size_t num_dataset, uint32_t dim, const ScanRows& rw, const SubRows& sub_rows, const float* d_queries,
+                   size_t num_queries, uint32_t k, int metric, int64_t* d_out_indices, float* d_out_dists, float* kernel_ms, hipStream_t st,
+                   const ScanBase* base, uint32_t num_cu, bool* applied) {
+    DeviceScratch base_mem;
+    HalfBase own;
+    *applied = false;
+    if (!base) {
+        if (base_mem.alloc(half_base_bytes(num_dataset, dim)) != hipSuccess) {
+            (void)hipGetLastError();
+            return GRAB_OK;
+        }
+        GRAB_TRY(half_base_async(d_dataset, num_dataset, dim, metric, base_mem.ptr, &own, st));
+    }
+    GRAB_TRY(scan_half_pass(base ? *base->half : own, d_dataset, num_dataset, rw, sub_rows, d_queries, 0, (uint32_t)num_queries, k, metric, d_out_indices, d_out_dists,
+                            kernel_ms, st, base, num_cu, applied));
+    if (*applied) return GRAB_OK;
+    GRAB_HIP(hipStreamSynchronize(st));  // (the rows just made are freed)
+    if (kernel_ms) *kernel_ms = 0.0f;
+    knn_stats().flop_f16 = knn_stats().flop_bf16 = 0.0;
+    knn_stats().exact_rows = 0;
+    return GRAB_OK;
 }
 
 // The quick way.  One contraction over all tile-grid rows, which read their query's row in place; where there are
@@ -996,7 +1052,7 @@ int grab_scan_base_create(const float* d_dataset, size_t num_dataset, uint32_t d
         }
         const int rc = half_base_async(d_dataset, num_dataset, dim, metric, b->half_mem.ptr, &b->half, nullptr);
         if (rc != GRAB_OK) return fail(rc);
-        if (hipMemcpy(&bad, b->half.scal + 11, 4, hipMemcpyDeviceToHost) != hipSuccess) {
+        if (hipMemcpy(&bad, b->half.scal + kScalBad, 4, hipMemcpyDeviceToHost) != hipSuccess) {
             set_error("scan base: preparing the rows failed");
             return fail(GRAB_ERR_HIP);
         }
@@ -1068,8 +1124,8 @@ int scan_on_base(grab_scan_base* b, const std::function<int()>& run) {
         rc = run();  // returns with the stream drained: nothing of the block is in use any more
     }
     if (rc != GRAB_OK) (void)hipDeviceSynchronize();  // a call that gave up half way may have left kernels queued
-    const size_t want = std::min<size_t>(arena.wanted + arena.wanted / 8 + (1u << 20), 8ull << 30);
-    if (arena.wanted > b->block_bytes && want > b->block_bytes) {
+    const size_t most = std::max(arena.wanted, arena.peak), want = std::min<size_t>(most + most / 8 + (1u << 20), 8ull << 30);
+    if (most > b->block_bytes && want > b->block_bytes) {
         if (b->block) (void)hipFree(b->block);
         b->block = nullptr;
         b->block_bytes = 0;

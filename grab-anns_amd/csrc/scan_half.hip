@@ -39,7 +39,6 @@ constexpr float kOpen = -9.0e8f;        // the threshold of a query that takes a
 // of 500,000 x 128, intervals of 50,000, k 10: 73, 340 and 456 queries not proven, calls of 4.2 - 4.4 ms; none and 0.24 - 0.27 now.
 // The same for intervals of 1500 among those of 100,000, of which every other had no sampled block: 4.46 -> 0.64.)
 constexpr uint32_t kSampleValues = 1024;
-constexpr uint64_t kScanSampleBytes = 4ull << 30;  // the sampled values of a call, at most
 constexpr uint32_t kBoundValues = 2048;  // sampled values that a query looks at, at most: 32 a lane
 
 // Tile-grid rows into blocks, and per query: squared norm of the rounded, scaled row (-1: not taken), what rounding moved it,
@@ -729,7 +728,7 @@ int half_base_async(const float* data, size_t n, uint32_t dim, int metric, void*
     return GRAB_OK;
 }
 
-bool half_scan_plan(const HalfBase& b, uint32_t num_cu, const uint32_t* h_row_lo, const uint32_t* h_row_hi, HalfScan* s) {
+bool half_scan_plan(const HalfBase& b, uint32_t num_cu, const uint32_t* h_row_lo, const uint32_t* h_row_hi, size_t max_bytes, HalfScan* s) {
     const uint32_t row_tiles = s->rows / kScanRowsTile;
     // tiles of 8 blocks, 256 columns; an item is as many as leave every workgroup some four of them
     constexpr uint32_t kItemTiles = 32;  // ... at most
@@ -759,7 +758,7 @@ bool half_scan_plan(const HalfBase& b, uint32_t num_cu, const uint32_t* h_row_lo
         sampled += x.blocks;
         n_sweep += ((blocks_of(t) + 7) / 8 + per - 1) / per;
     }
-    if (sampled * 4096 * 4 > kScanSampleBytes) return false;
+    if (sampled * 4096 * 4 + (size_t)s->rows * kScanListCap * 4 > max_bytes) return false;
     const size_t n_sample = sampled / 8;
     s->at_tiles = 0;
     s->at_sweep = (size_t)row_tiles * 4;
@@ -785,7 +784,7 @@ bool half_scan_plan(const HalfBase& b, uint32_t num_cu, const uint32_t* h_row_lo
     auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
     s->workspace_bytes = up((size_t)s->rows / 32 * b.frags * 1024) + up((size_t)s->rows / 32 * 2048) + up(s->sample_floats * 4) + up((size_t)s->rows * kScanListCap * 4) +
                          up((size_t)s->nq * 28) + up((size_t)s->rows * 4 + 64 + (size_t)s->nq * 4);
-    return true;
+    return s->workspace_bytes <= max_bytes;
 }
 
 int half_scan_async(const HalfBase& b, const HalfScan& s, const HalfScanArgs& given, void* workspace, uint32_t num_cu, uint32_t** left, hipStream_t st) {

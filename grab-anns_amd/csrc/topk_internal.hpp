@@ -94,6 +94,7 @@ void launch_split_rows_chunked(const float* data, uint64_t n, uint32_t dim, cons
 
 // The candidates of a large kNN graph from f16 products: knn_half.hip.  Where it applies, a plan of the sizes, the lists, and
 // the neighbours that these prove.
+constexpr uint32_t kScalBad = 11, kScalPlain = 12;  // words of `scal`: whether some row is not finite; the largest squared norm of the rows as they are
 constexpr uint32_t kHalfListCap = 1024;  // keys of a row's list
 constexpr uint32_t kHalfSample = 49152;  // sample rows that the bounds are taken from, at most
 struct HalfKnn {
@@ -120,7 +121,7 @@ int half_knn_finish_async(const float* data, const HalfKnn& h, uint32_t k, const
                           uint32_t* redo_count, uint32_t* redo, uint32_t* doubt, hipStream_t st);
 
 // Queries against intervals of a row set, on f16 products: scan_half.hip.  The base rows in blocks, made once (mem holds
-// half_base_bytes); whether a row is not finite can be read from scal[11] afterwards.
+// half_base_bytes); whether a row is not finite can be read from scal[kScalBad] afterwards.
 constexpr uint32_t kSampleShiftMin = 3, kSampleShiftMax = 6;
 struct HalfBase {
     uint32_t n = 0, dim = 0, ks = 0, frags = 0, last_block = 0;
@@ -147,8 +148,8 @@ struct HalfScan {
     uint32_t sweep_items = 0, sample_items = 0;
     size_t sample_floats = 0, workspace_bytes = 0;
 };
-// false: the values that the bounds are taken from would need more memory than a call gets
-bool half_scan_plan(const HalfBase& b, uint32_t num_cu, const uint32_t* h_row_lo, const uint32_t* h_row_hi, HalfScan* s);
+// false: it would need more device memory than max_bytes
+bool half_scan_plan(const HalfBase& b, uint32_t num_cu, const uint32_t* h_row_lo, const uint32_t* h_row_hi, size_t max_bytes, HalfScan* s);
 // everything queued on `st`: results, and (*left)[0]: whether some query is one that this way does not take (nothing of the
 // results is to be used then), (*left)[1]: the number of queries not proven, from (*left)[2] on: which
 struct HalfScanArgs {

@@ -1,5 +1,6 @@
 """Exact top-k inside intervals of row ids (grab_window_scan_topk) against the CPU's exact range-filtered scan."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -338,4 +339,25 @@ def test_window_scan_of_few_queries(oracle, grab, nq, width, k, on_f16):
     assert (grab.last_knn_f16_flop() > 0) == on_f16 and grab.last_knn_bf16_flop() > 0
     base.close()
     eids, edist = oracle.bruteforce_topk(data, q, k, filter_kind=oracle.FILTER_RANGE, ts=np.arange(n, dtype=np.uint64), win_start=lo, win_end=hi)
+    assert np.array_equal(ids, eids) and np.array_equal(dist.view(np.uint32), edist.view(np.uint32))
+
+
+@pytest.mark.parametrize("nq,k,width", [(1_300_000, 17, 300), (70_000, 17, 60_000)])
+def test_window_scan_of_many_queries_takes_bounded_memory(oracle, grab, nq, k, width):
+    # lists of 8 KB a query, then some thousand sampled values a query: in passes of 4 GiB, whose scratch the base keeps
+    n, dim = 250_000, 32
+    data, q = datasets.gaussian(n, dim, 4), datasets.gaussian(nq, dim, 7)
+    lo, hi = _intervals(n, nq, width - 50, width, nq)
+    d_data, d_q = grab.DeviceArray.from_numpy(data), grab.DeviceArray.from_numpy(q)
+    out = (grab.DeviceArray((nq, k), np.int64), grab.DeviceArray((nq, k), np.float32))
+    base = grab.ScanBase(d_data, n, dim, 0)
+    free = grab.device_memory()[0]
+    base.window_topk(d_q, nq, k, lo, hi, d_out=out)
+    assert grab.last_knn_f16_flop() > 0 and grab.last_knn_exact_rows() <= 20
+    time.sleep(1.0)  # the first call's scratch is given back, which the driver takes its time over
+    assert free - grab.device_memory()[0] < 5 << 30
+    base.close()
+    pick = np.concatenate([[0, nq // 2 - 1, nq // 2, nq - 1], np.random.default_rng(1).integers(0, nq, 400)])
+    ids, dist = out[0].numpy()[pick], out[1].numpy()[pick]
+    eids, edist = oracle.bruteforce_topk(data, q[pick], k, filter_kind=oracle.FILTER_RANGE, ts=np.arange(n, dtype=np.uint64), win_start=lo[pick], win_end=hi[pick])
     assert np.array_equal(ids, eids) and np.array_equal(dist.view(np.uint32), edist.view(np.uint32))
