@@ -582,6 +582,16 @@ int unproven_queries(const float* d_dataset, size_t num_dataset, uint32_t dim, c
     return GRAB_OK;
 }
 
+// the results of queries of which none admits a row
+int no_row_admitted(size_t num_queries, uint32_t k, int64_t* d_out_indices, float* d_out_dists, hipStream_t st) {
+    std::vector<int64_t> ids(num_queries * (size_t)k, -1);
+    std::vector<float> dist(num_queries * (size_t)k, kDistMax);
+    GRAB_HIP(hipMemcpyAsync(d_out_indices, ids.data(), ids.size() * 8, hipMemcpyHostToDevice, st));
+    GRAB_HIP(hipMemcpyAsync(d_out_dists, dist.data(), dist.size() * 4, hipMemcpyHostToDevice, st));
+    GRAB_HIP(hipStreamSynchronize(st));
+    return GRAB_OK;
+}
+
 // One pass of the f16 way (scan_half.hip) over queries [first, first + nq) of the call, whose rows are `rw`; its kernels' time is added
 // to *kernel_ms.  *applied = false: a query or a row that this way does not take, or no room.
 constexpr size_t kHalfPassBytes = (size_t)4 << 30;  // device memory of a pass: what the other way's passes take
@@ -590,7 +600,8 @@ int scan_half_pass(const HalfBase& b, const float* d_dataset, size_t num_dataset
                    uint32_t nq, uint32_t k, int metric, int64_t* d_out_indices, float* d_out_dists, float* kernel_ms, hipStream_t st, const ScanBase* base,
                    uint32_t num_cu, bool* applied) {
     const uint32_t rows = rw.rows, dim = b.dim;
-    *applied = false;
+    *applied = rows == 0;  // (a part of a call may be without any)
+    if (rows == 0) return no_row_admitted(nq, k, d_out_indices + (size_t)first * k, d_out_dists + (size_t)first * k, st);
     HalfScan s;
     s.rows = rows;
     s.nq = nq;
@@ -715,14 +726,7 @@ int scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const Sc
     const uint32_t rows = rw.rows, nq = (uint32_t)num_queries;
     knn_stats().flop = knn_stats().flop_bf16 = knn_stats().flop_f16 = 0.0;
     knn_stats().redone_rows = knn_stats().exact_rows = 0;
-    if (rows == 0) {  // no query admits a row
-        std::vector<int64_t> ids(num_queries * (size_t)k, -1);
-        std::vector<float> dist(num_queries * (size_t)k, kDistMax);
-        GRAB_HIP(hipMemcpyAsync(d_out_indices, ids.data(), ids.size() * 8, hipMemcpyHostToDevice, st));
-        GRAB_HIP(hipMemcpyAsync(d_out_dists, dist.data(), dist.size() * 4, hipMemcpyHostToDevice, st));
-        GRAB_HIP(hipStreamSynchronize(st));
-        return GRAB_OK;
-    }
+    if (rows == 0) return no_row_admitted(num_queries, k, d_out_indices, d_out_dists, st);
     int dev = 0, num_cu = 0;
     GRAB_HIP(hipGetDevice(&dev));
     GRAB_HIP(hipDeviceGetAttribute(&num_cu, hipDeviceAttributeMultiprocessorCount, dev));

@@ -361,3 +361,22 @@ def test_window_scan_of_many_queries_takes_bounded_memory(oracle, grab, nq, k, w
     ids, dist = out[0].numpy()[pick], out[1].numpy()[pick]
     eids, edist = oracle.bruteforce_topk(data, q[pick], k, filter_kind=oracle.FILTER_RANGE, ts=np.arange(n, dtype=np.uint64), win_start=lo[pick], win_end=hi[pick])
     assert np.array_equal(ids, eids) and np.array_equal(dist.view(np.uint32), edist.view(np.uint32))
+
+
+def test_window_scan_of_many_queries_half_of_them_without_a_row(oracle, grab):
+    # lists of 560,000 queries are more than a pass takes; of the two that it is cut into one has no row at all
+    n, dim, nq, k = 20000, 32, 1_120_000, 17
+    data, q = datasets.gaussian(n, dim, 4), datasets.gaussian(nq, dim, 7)
+    lo, hi = _intervals(n, nq, 250, 300, 5)
+    hi[:nq // 2] = lo[:nq // 2]
+    d_data, d_q = grab.DeviceArray.from_numpy(data), grab.DeviceArray.from_numpy(q)
+    out = (grab.DeviceArray((nq, k), np.int64), grab.DeviceArray((nq, k), np.float32))
+    base = grab.ScanBase(d_data, n, dim, 0)
+    base.window_topk(d_q, nq, k, lo, hi, d_out=out)
+    assert grab.last_knn_f16_flop() > 0
+    base.close()
+    ids, dist = out[0].numpy(), out[1].numpy()
+    assert (ids[:nq // 2] == -1).all() and (dist[:nq // 2] == np.float32(3.40282e38)).all()
+    pick = np.concatenate([[nq // 2, nq - 1], np.random.default_rng(1).integers(nq // 2, nq, 400)])
+    eids, edist = oracle.bruteforce_topk(data, q[pick], k, filter_kind=oracle.FILTER_RANGE, ts=np.arange(n, dtype=np.uint64), win_start=lo[pick], win_end=hi[pick])
+    assert np.array_equal(ids[pick], eids) and np.array_equal(dist[pick].view(np.uint32), edist.view(np.uint32))
