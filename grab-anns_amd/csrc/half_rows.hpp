@@ -96,8 +96,8 @@ __device__ __forceinline__ void note_largest(float v, uint32_t* out) {
     if ((threadIdx.x & 63) == 0 && __float_as_uint(v) > __atomic_load_n(out, __ATOMIC_RELAXED)) atomicMax(out, __float_as_uint(v));
 }
 
-// squared norm of every centred row, and the largest finite one (scal[0], as bits); scal[kScalPlain]: the largest of the rows as
-// they are; 16 lanes a row
+// squared norm of every centred row, and the largest below 3e38, beyond which a row is not packed (scal[0], as bits); scal[kScalPlain]:
+// the largest of the rows as they are; 16 lanes a row
 __global__ void __launch_bounds__(256) half_norms_kernel(const float* __restrict__ data, uint32_t n, uint32_t dim,
                                                          const float* __restrict__ centre, float* __restrict__ norm, uint32_t* __restrict__ scal) {
     const uint32_t j = threadIdx.x & 15;
@@ -121,6 +121,7 @@ __global__ void __launch_bounds__(256) half_norms_kernel(const float* __restrict
             plain += __shfl_xor(plain, m, 64);
         }
         if (j == 0) norm[row] = s;
+        if (j == 0 && s >= 3.0e38f) scal[kScalLong] = 1u;
         if (s < 3.0e38f) most = fmaxf(most, s);
         most_plain = fmaxf(most_plain, plain);
     }

@@ -664,6 +664,7 @@ __global__ void __launch_bounds__(256) knn_finish_kernel(const FinishArgs a) {
         form = fmax((2.0 * dim + 96.0) * u * sqrt(cn * cn_max), 2.0 * (1.25 * dim + 16.0) * u * sqrt((double)a.norm[row] * (double)*a.max_norm));
         e_far = eps * sqrt(cn_max) + (sqrt(cn) + eps) * eps_max + form;
     }
+    if (a.scal[kScalLong] != 0) form = __builtin_inf();  // a row that is in no list, and may be near this one: nothing is proven
     // need + 1 columns' values lie in the parts up to `high`: their true distances lie within what the parts' lower edge, farthest
     // off, allows; a column whose value is beyond what follows from that is farther than all of them, also in the re-scored
     // order.  (A part's number was rounded: two parts more at either end.)

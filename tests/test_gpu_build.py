@@ -331,6 +331,22 @@ def test_knn_graph_of_rows_that_are_not_finite(grab):
         assert np.array_equal(got[finite], exp[finite])
 
 
+@pytest.mark.parametrize("metric", [0, 1])
+def test_knn_graph_with_a_row_too_long_to_be_packed(oracle, grab, metric):
+    # a squared norm between the 3e38 that the f16 pass takes and the largest float: the row is in no list, but among many rows'
+    # nearest by inner product, and with squared L2 the nearest of one that is almost as long
+    n, dim, k = 4200, 32, 8
+    data = datasets.unit_rows(n, dim, 3).astype(np.float64)
+    data *= 1.0e19 if metric else 1.0e18
+    data[7] *= 1.70e19 / np.linalg.norm(data[7])
+    data[1000] = data[7] * (1.76 / 1.70) if metric == 0 else data[1000] * 1.76
+    data = data.astype(np.float32)
+    got = grab.generate_knn_graph(grab.DeviceArray.from_numpy(data), n, dim, k, metric)[0].numpy()
+    assert (got[7, 0] == 1000) if metric == 0 else ((got == 1000).any(axis=1).sum() > 50)
+    own = np.arange(n) != 1000  # (its own go through the plain pass)
+    assert np.array_equal(got[own], oracle.knn_graph(data, k, metric)[own])
+
+
 @pytest.mark.parametrize("n,dim,k,kind", [(4096, 160, 20, "gauss"), (4353, 32, 16, "unit"), (5000, 224, 143, "unit"), (4607, 1024, 8, "gauss"),
                                           (8200, 128, 64, "unit"), (4500, 288, 31, "integers"), (4352, 256, 12, "negative")])
 def test_knn_graph_on_f16_products_inner_product_and_long_rows(oracle, grab, n, dim, k, kind):
