@@ -640,9 +640,13 @@ __global__ void __launch_bounds__(256) refine_kernel(const RefineArgs a) {
             if (a.split_normA != nullptr) err = fmax(err, 2.0 * cs * u * sqrt((double)a.split_normA[row] * (double)*a.split_max_normB));
             return err;
         }
-        double err = c * u * (na + nb);
-        if (a.split_normA != nullptr) err = fmax(err, cs * u * ((double)a.split_normA[row] + (double)*a.split_max_normB));
-        return err;
+        double most = na + nb, err = c * u * most;
+        if (a.split_normA != nullptr) {
+            const double split = (double)a.split_normA[row] + (double)*a.split_max_normB;
+            err = fmax(err, cs * u * split);
+            most = fmax(most, split);
+        }
+        return most < 3.4e38 ? err : __builtin_inf();  // |a|^2 + |b|^2 and 2ab overflow from there on: a near pair may have no value at all
     };
     // An ascending list need not be scored to its end: the first need + 1 candidates have true distances of at most
     // A + err (A = the GEMM-form value of the last of them), so a candidate whose GEMM-form value exceeds A + 2 err -

@@ -347,6 +347,22 @@ def test_knn_graph_with_a_row_too_long_to_be_packed(oracle, grab, metric):
     assert np.array_equal(got[own], oracle.knn_graph(data, k, metric)[own])
 
 
+@pytest.mark.parametrize("n,allow", [(4200, True), (4200, False), (600, False)])
+def test_knn_graph_where_the_sum_of_two_norms_overflows(oracle, grab, n, allow):
+    # |a|^2 + |b|^2 - 2ab of the two longest rows is infinity less infinity: no candidates of each other, nearest all the same
+    dim, k = 32, 8
+    data = datasets.unit_rows(n, dim, 3) * np.float32(1.0e18)
+    data[7] *= np.float32(14.0)
+    data[500] = data[7] * np.float32(1.1)
+    before = grab.knn_allow_bf16(allow)
+    try:
+        got = grab.generate_knn_graph(grab.DeviceArray.from_numpy(data), n, dim, k)[0].numpy()
+    finally:
+        grab.knn_allow_bf16(before)
+    assert got[7, 0] == 500 and got[500, 0] == 7
+    assert np.array_equal(got, oracle.knn_graph(data, k))
+
+
 @pytest.mark.parametrize("n,dim,k,kind", [(4096, 160, 20, "gauss"), (4353, 32, 16, "unit"), (5000, 224, 143, "unit"), (4607, 1024, 8, "gauss"),
                                           (8200, 128, 64, "unit"), (4500, 288, 31, "integers"), (4352, 256, 12, "negative")])
 def test_knn_graph_on_f16_products_inner_product_and_long_rows(oracle, grab, n, dim, k, kind):
