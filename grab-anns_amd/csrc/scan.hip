@@ -467,7 +467,7 @@ struct ScanBase {
     void** staging = nullptr;         // page-locked host memory for a call's tables, grown as needed (null: none kept)
     size_t* staging_bytes = nullptr;
     const HalfBase* half = nullptr;   // the rows rounded to f16, where these are what a call uses first
-    std::function<int(hipStream_t)> make_split;  // ... and rows_split is made when a call needs it after all
+    std::function<int(hipStream_t, bool* no_room)> make_split;  // ... and rows_split is made when a call needs it after all
 };
 
 // A call's tables, put together on the host and brought to the device in one upload
@@ -733,8 +733,7 @@ int scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const Sc
     const uint32_t kk = std::max<uint32_t>(2 * k + 32, 64);  // <= 288
     const uint32_t row_tiles = rows / TM, col_tiles = (uint32_t)((num_dataset + TN - 1) / TN), target = (uint32_t)num_cu * 2;
     // a prepared base has paid for its split rows; otherwise splitting a million rows pays from a thousand query rows on
-    const bool split = base ? base->split
-                            : knn_bf16_allowed() && dim % KC == 0 && rows >= 1024 && num_dataset >= 4096;
+    bool split = base ? base->split : knn_bf16_allowed() && dim % KC == 0 && rows >= 1024 && num_dataset >= 4096;
     // On f16 rows, except narrow intervals with short lists: a tenth of an interval's columns would be listed, and writing all values
     // costs less.  A call over a prepared base, stored values against this way in us, k 10, intervals of 1000, 4000, 6000 and 8000:
     //   1M x 128, 100 queries     221 / 243, 230 / 223, 236 / 215, 241 / 212      150,000 x 768  197 / 198, 209 / 199, 213 / 193, 219 / 196
@@ -746,17 +745,30 @@ int scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const Sc
     const bool narrow = rw.one_row_per_query && kk <= 64 && rw.columns < (rw.lists.size() <= 2 ? 10000ull : 6000ull) * rw.lists.size();
     // Beyond 127,000 columns a sampled value stands for more than 64 columns, too few lie within a bound to set it by; by the same
     // reckoning as at 100,000 from one in 130 (scan_half.hip: 5.3 ms a call against 3.3 with stored values).
-    if (split && !narrow && half_scan_takes(rw.widest) && (!base || base->half)) {
+    bool on_half = split && half_scan_takes(rw.widest) && (!base || base->half), applied = false;
+    if (on_half && !rw.one_row_per_query) {
         uint32_t most = 0;  // rows of a query; a wave's lanes hold them
-        for (size_t q = 0; q < num_queries && !rw.one_row_per_query; ++q) most = std::max(most, rw.list_off[q + 1] - rw.list_off[q]);
-        if (most <= 64) {
-            bool applied = false;
-            GRAB_TRY(scan_topk_half(d_dataset, num_dataset, dim, rw, sub_rows, d_queries, num_queries, k, metric, d_out_indices, d_out_dists, kernel_ms, st, base,
-                                    (uint32_t)num_cu, &applied));
+        for (size_t q = 0; q < num_queries; ++q) most = std::max(most, rw.list_off[q + 1] - rw.list_off[q]);
+        on_half = most <= 64;
+    }
+    auto run_half = [&] {
+        return scan_topk_half(d_dataset, num_dataset, dim, rw, sub_rows, d_queries, num_queries, k, metric, d_out_indices, d_out_dists, kernel_ms, st, base,
+                              (uint32_t)num_cu, &applied);
+    };
+    if (on_half && !narrow) {
+        GRAB_TRY(run_half());
+        if (applied) return GRAB_OK;
+    }
+    if (base && base->split && base->rows_split == nullptr) {
+        bool no_room = false;
+        GRAB_TRY(base->make_split(st, &no_room));
+        if (no_room) {  // the halves do not fit beside the f16 rows: these serve narrow intervals as well, the rows as they are what is left
+            if (on_half && narrow) GRAB_TRY(run_half());
             if (applied) return GRAB_OK;
+            base = nullptr;
+            split = false;
         }
     }
-    if (base && base->split && base->rows_split == nullptr) GRAB_TRY(base->make_split(st));
     DeviceScratch d_tab, buf, cand, merged, outside, norm_a, norm_b, split_a, split_b, mean, doubt;
     // Short candidate lists (k <= 16) go the dense way: the contraction writes the distances of the columns that a row tile
     // sweeps, in work items of equal length, and a streaming pass keeps the kk smallest of every row.  The other way
@@ -1063,26 +1075,25 @@ int grab_scan_base_create(const float* d_dataset, size_t num_dataset, uint32_t d
         if (bad == 0) b->view.half = &b->half;
     }
     // norms, and the rows as bf16 halves: now for a base that is scanned as it is, or when a call first needs them
-    auto prepare = [b](hipStream_t st) -> int {
+    auto prepare = [b](hipStream_t st, bool* no_room) -> int {
+        DeviceScratch norm, max_norm, mean, rows_split;  // the base's once all is queued
         ScratchArena* const lent = scratch_arena();
         scratch_arena() = nullptr;  // these stay: no part of a call's scratch
-        const bool room = b->norm.alloc(b->num_dataset * 4) == hipSuccess && b->max_norm.alloc(4) == hipSuccess &&
-                          (!b->view.split || b->rows_split.alloc(b->num_dataset * b->dim * 4) == hipSuccess);
+        *no_room = norm.alloc(b->num_dataset * 4) != hipSuccess || max_norm.alloc(4) != hipSuccess ||
+                   (b->view.split && rows_split.alloc(b->num_dataset * b->dim * 4) != hipSuccess);
         int rc = GRAB_OK;
-        if (!room) {
-            (void)hipGetLastError();
-            set_error("scan base: out of device memory");
-            rc = GRAB_ERR_HIP;
-        } else if (b->view.split) {
-            rc = split_base_rows(b->d_dataset, b->num_dataset, b->dim, b->metric, &b->mean, b->rows_split.as<uint16_t>(), b->norm.as<float>(), st);
-        } else {
-            launch_row_norms(b->d_dataset, b->num_dataset, b->dim, b->norm.as<float>(), st);
-        }
+        if (*no_room) (void)hipGetLastError();
+        else if (b->view.split) rc = split_base_rows(b->d_dataset, b->num_dataset, b->dim, b->metric, &mean, rows_split.as<uint16_t>(), norm.as<float>(), st);
+        else launch_row_norms(b->d_dataset, b->num_dataset, b->dim, norm.as<float>(), st);
         scratch_arena() = lent;
-        if (rc != GRAB_OK) return rc;
-        GRAB_HIP(hipMemsetAsync(b->max_norm.ptr, 0, 4, st));
-        launch_max_float(b->norm.as<float>(), b->num_dataset, b->max_norm.as<uint32_t>(), st);
+        if (rc != GRAB_OK || *no_room) return rc;
+        GRAB_HIP(hipMemsetAsync(max_norm.ptr, 0, 4, st));
+        launch_max_float(norm.as<float>(), b->num_dataset, max_norm.as<uint32_t>(), st);
         GRAB_HIP(hipGetLastError());
+        std::swap(b->norm.ptr, norm.ptr);
+        std::swap(b->max_norm.ptr, max_norm.ptr);
+        std::swap(b->mean.ptr, mean.ptr);
+        std::swap(b->rows_split.ptr, rows_split.ptr);
         b->view.rows_split = b->rows_split.as<uint16_t>();
         b->view.norm = b->norm.as<float>();
         b->view.mean = b->mean.as<float>();
@@ -1091,7 +1102,12 @@ int grab_scan_base_create(const float* d_dataset, size_t num_dataset, uint32_t d
     };
     b->view.make_split = prepare;
     if (b->view.half == nullptr) {
-        const int rc = prepare(nullptr);
+        bool no_room = false;
+        const int rc = prepare(nullptr, &no_room);
+        if (no_room) {
+            set_error("scan base: out of device memory");
+            return fail(GRAB_ERR_HIP);
+        }
         if (rc != GRAB_OK) return fail(rc);
     }
     if (hipDeviceSynchronize() != hipSuccess) {

@@ -380,3 +380,43 @@ def test_window_scan_of_many_queries_half_of_them_without_a_row(oracle, grab):
     pick = np.concatenate([[nq // 2, nq - 1], np.random.default_rng(1).integers(nq // 2, nq, 400)])
     eids, edist = oracle.bruteforce_topk(data, q[pick], k, filter_kind=oracle.FILTER_RANGE, ts=np.arange(n, dtype=np.uint64), win_start=lo[pick], win_end=hi[pick])
     assert np.array_equal(ids[pick], eids) and np.array_equal(dist[pick].view(np.uint32), edist.view(np.uint32))
+
+
+def test_scan_base_where_the_rows_as_bf16_halves_find_no_room(oracle, grab):
+    # narrow intervals would have the halves made: where the memory is not there they are scanned on f16 rows, those that f16 rows
+    # do not take on the rows as they are, nothing is left allocated, and with the memory back the halves are made
+    n, dim, nq, k = 2_000_000, 128, 60, 10
+    data, q = np.random.default_rng(4).standard_normal((n, dim), np.float32), datasets.gaussian(nq, dim, 7)
+    d_data, d_q = grab.DeviceArray.from_numpy(data), grab.DeviceArray.from_numpy(q)
+    base = grab.ScanBase(d_data, n, dim, 0)
+    taken = []
+    for size in (4 << 30, 256 << 20):
+        try:
+            while True:
+                taken.append(grab.DeviceArray((size,), np.uint8))
+        except grab.GrabError:
+            pass
+    for _ in range(2):  # 512 to 768 MB: the halves take 1024
+        taken.pop().free()
+
+    def scan(widths, f16, halves, seed=3):
+        lo, hi = _intervals(n, nq, widths[0], widths[1], seed)
+        lo, hi = lo % np.uint64(1000), hi - lo + lo % np.uint64(1000)
+        ids, dist, _ = base.window_topk(d_q, nq, k, lo, hi)
+        assert (grab.last_knn_f16_flop() > 0) == f16 and (grab.last_knn_bf16_flop() > 0) == (f16 or halves)
+        own = slice(0, int(hi.max()))
+        eids, edist = oracle.bruteforce_topk(data[own], q, k, filter_kind=oracle.FILTER_RANGE, ts=np.arange(own.stop, dtype=np.uint64), win_start=lo, win_end=hi)
+        assert np.array_equal(ids, eids) and np.array_equal(dist.view(np.uint32), edist.view(np.uint32))
+        return grab.device_memory()[0]
+
+    scan((2000, 3000), True, False)
+    free = scan((127500, 150000), False, False)  # (the base's block is as large as it gets)
+    for _ in range(3):
+        scan((2000, 3000), True, False)
+        now = scan((127500, 150000), False, False)
+    assert now > free - (16 << 20)  # norms of each of the six calls would be 48 MB
+    for t in taken:
+        t.free()
+    scan((2000, 3000), False, True)
+    scan((127500, 150000), False, True)
+    base.close()
