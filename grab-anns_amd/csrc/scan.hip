@@ -1072,7 +1072,12 @@ int grab_scan_base_create(const float* d_dataset, size_t num_dataset, uint32_t d
             set_error("scan base: preparing the rows failed");
             return fail(GRAB_ERR_HIP);
         }
-        if (bad == 0) b->view.half = &b->half;
+        if (bad == 0) {
+            b->view.half = &b->half;
+        } else {
+            (void)hipFree(b->half_mem.ptr);
+            b->half_mem.ptr = nullptr;
+        }
     }
     // norms, and the rows as bf16 halves: now for a base that is scanned as it is, or when a call first needs them
     auto prepare = [b](hipStream_t st, bool* no_room) -> int {

@@ -420,3 +420,20 @@ def test_scan_base_where_the_rows_as_bf16_halves_find_no_room(oracle, grab):
     scan((2000, 3000), False, True)
     scan((127500, 150000), False, True)
     base.close()
+
+
+def test_scan_base_of_rows_that_are_not_finite_keeps_no_f16_rows(grab):
+    n, dim = 4_000_000, 32
+    d_data = grab.DeviceArray((n, dim), np.float32)
+    d_data.fill_bytes(0)
+    free = grab.device_memory()[0]
+    base = grab.ScanBase(d_data, n, dim, 0)
+    kept = free - grab.device_memory()[0]
+    base.close()
+    nan = np.full(dim, np.nan, np.float32)
+    grab.check(grab.lib.grab_copy_to_device(C.c_void_p(d_data.ptr + 5 * dim * 4), nan.ctypes.data_as(C.c_void_p), C.c_size_t(nan.nbytes)))
+    free = grab.device_memory()[0]
+    base = grab.ScanBase(d_data, n, dim, 0)
+    halves = free - grab.device_memory()[0]
+    base.close()
+    assert kept > 0 and halves < n * (dim * 4 + 4) + (64 << 20)  # halves and norms, and no more
