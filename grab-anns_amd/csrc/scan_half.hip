@@ -402,7 +402,7 @@ __device__ __forceinline__ float scan_threshold(const float* __restrict__ sample
         const float mid = 0.5f * (low + high), c = reach(mid);
         if (c >= want) {
             low = mid;
-            if (c < 1.08f * want) break;
+            if (c < 1.08f * want || (ONE && c - weight_max < want)) break;  // (one value less would not do)
         } else {
             high = mid;
         }
@@ -550,7 +550,7 @@ __global__ void __launch_bounds__(256) scan_finish_kernel(const ScanFinishArgs f
         kept_part = (uint32_t)((((uint64_t)fit << shift) - 1u) >> f.id_bits);
         wave_sync();
     }
-    const uint32_t have = whole ? up_to((kept_part << f.id_bits) | id_mask) : 0u;
+    uint32_t have = whole ? up_to((kept_part << f.id_bits) | id_mask) : 0u;
     const float t = l1 > l0 ? f.q_t[q] : kOpen;
     const bool open = t <= kOpen;  // all columns are in the lists
     if (!whole || (!open && have <= need) || (open && kept_part != parts - 1u)) {
@@ -558,10 +558,13 @@ __global__ void __launch_bounds__(256) scan_finish_kernel(const ScanFinishArgs f
         return;
     }
     wave_sync();
-    constexpr int kEnts = kScanHave / 64;
+    // 1024 of them go to registers; more, which is rare, stay in LDS until it is known which few can matter (registers for 2048: 37 ->
+    // 44 us for 10,000 intervals of 10,000 rows of 1M x 128)
+    constexpr int kEnts = kScanSortCap / 64;
     uint32_t ent[kEnts];
+    const bool many = have > kScanSortCap;
 #pragma unroll
-    for (int i = 0; i < kEnts; ++i) ent[i] = (uint32_t)(i * 64 + lane) < have ? ents[i * 64 + lane] : kInvalidId;
+    for (int i = 0; i < kEnts; ++i) ent[i] = !many && (uint32_t)(i * 64 + lane) < have ? ents[i * 64 + lane] : kInvalidId;
     __builtin_amdgcn_wave_barrier();
     uint32_t last_part = parts - 1u;
     double bound = 0.0, form = 0.0, e_far = 0.0;
@@ -569,6 +572,10 @@ __global__ void __launch_bounds__(256) scan_finish_kernel(const ScanFinishArgs f
     auto within = [&](uint32_t part) {  // entries in the parts up to `part`
         uint32_t c = 0;
         const uint32_t last = (part << f.id_bits) | id_mask;
+        if (many) {
+            for (uint32_t g = 0; g < have; g += 64) c += (uint32_t)__popcll(__ballot(g + lane < have && ents[g + lane] <= last));
+            return c;
+        }
 #pragma unroll
         for (int i = 0; i < kEnts; ++i)
             if ((uint32_t)(i * 64) < have) c += (uint32_t)__popcll(__ballot((uint32_t)(i * 64 + lane) < have && ent[i] <= last));
@@ -607,9 +614,25 @@ __global__ void __launch_bounds__(256) scan_finish_kernel(const ScanFinishArgs f
         const double far_part = (top - cutoff / unit) / way * parts + 1.0;
         last_part = far_part < (double)(parts - 1u) ? (uint32_t)fmax(far_part, 0.0) : parts - 1u;  // (all of them where it is not a number)
     }
-    if (have > kScanSortCap && within(last_part) > kScanSortCap) {
-        if (lane == 0) f.a.doubt[1 + atomicAdd(f.a.doubt, 1u)] = q;
-        return;
+    if (many) {
+        if (within(last_part) > kScanSortCap) {
+            if (lane == 0) f.a.doubt[1 + atomicAdd(f.a.doubt, 1u)] = q;
+            return;
+        }
+        uint32_t kept = 0;  // those up to last_part to the front: a place is read before anything is written there
+        for (uint32_t g = 0; g < have; g += 64) {
+            const uint32_t e = g + lane < have ? ents[g + lane] : kInvalidId;
+            const bool in = g + lane < have && e <= ((last_part << f.id_bits) | id_mask);
+            const uint64_t b = __ballot(in);
+            wave_sync();
+            if (in) ents[kept + (uint32_t)__popcll(b & ((1ull << lane) - 1ull))] = e;
+            kept += (uint32_t)__popcll(b);
+        }
+        wave_sync();
+        have = kept;
+#pragma unroll
+        for (int i = 0; i < kEnts; ++i) ent[i] = (uint32_t)(i * 64 + lane) < have ? ents[i * 64 + lane] : kInvalidId;
+        __builtin_amdgcn_wave_barrier();
     }
     uint32_t n_score = 0;
     {
