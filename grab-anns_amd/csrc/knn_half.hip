@@ -791,9 +791,11 @@ int launch_sweep_short(const HalfKnn& h, uint32_t num_cu, hipStream_t st) {
     SymHalfArgs s = sweep_args(h);
     s.steps = (h.n + 31) / 32;
     const uint32_t grid = num_cu * half_groups(KS);
-    // sweeps in slices: sixteen items a workgroup at least, of 32 steps at least
-    const uint64_t total = (uint64_t)s.row_tiles * s.steps / 2;
-    s.steps_per_slice = (uint32_t)std::min<uint64_t>(s.steps, std::max<uint64_t>(32u, total / (16ull * grid)));
+    // sweeps in slices: sixteen items a workgroup at least, of 32 steps at least, and of fewer, down to two, where these leave workgroups
+    // without an item.  (4096 rows are 40 items of 32 steps for 768 workgroups: 4096 x 128 in clusters, k 128, 1137 us a call
+    // on two bf16 halves a value, 1349 in items of 32, 993 of 8, 762 of 4, 532 of two, 495 of one; 10,000 x 128, k 32: 529, 449, 439, 439, 435.)
+    const uint64_t total = (uint64_t)s.row_tiles * s.steps / 2, least = std::min<uint64_t>(32u, std::max<uint64_t>(2u, total / grid));
+    s.steps_per_slice = (uint32_t)std::min<uint64_t>(s.steps, std::max<uint64_t>(least, total / (16ull * grid)));
     s.slices = (s.steps + s.steps_per_slice - 1) / s.steps_per_slice;
     s.work_counter = h.scal + 2;
     static_assert(sizeof(SymHalfLds<KS>) <= 160 * 1024 / half_groups(KS), "so many workgroups per CU");

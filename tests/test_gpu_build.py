@@ -314,6 +314,15 @@ def test_knn_graph_on_f16_products_at_the_edges_of_its_tiles(oracle, grab, n, di
     assert np.array_equal(got.numpy(), oracle.knn_graph(data, k))
 
 
+@pytest.mark.parametrize("n", [4097, 6001, 11000, 19500])
+def test_knn_graph_on_f16_products_in_slices_of_few_steps(oracle, grab, n):
+    # from two steps of 32 columns a slice at the fewest rows to 32 at some 20,000; rows of a cluster, whose lists fill in few steps
+    data = np.sort(datasets.mixture(n, 32, 8, 3, n), axis=0)
+    got, _ = grab.generate_knn_graph(grab.DeviceArray.from_numpy(data), n, 32, 96)
+    assert grab.last_knn_f16_flop() > 0
+    assert np.array_equal(got.numpy(), oracle.knn_graph(data, 96))
+
+
 def test_knn_graph_of_rows_that_are_not_finite(grab):
     # rows with NaN or an overflowing norm get no list from the f16 pass and go the way they always went
     n, dim, k = 5000, 64, 32
