@@ -96,16 +96,16 @@ __device__ __forceinline__ void note_largest(float v, uint32_t* out) {
     if ((threadIdx.x & 63) == 0 && __float_as_uint(v) > __atomic_load_n(out, __ATOMIC_RELAXED)) atomicMax(out, __float_as_uint(v));
 }
 
-// squared norm of every centred row, and the largest below 3e38, beyond which a row is not packed (scal[0], as bits); scal[kScalPlain]:
-// the largest of the rows as they are; 16 lanes a row
+// squared norm of every centred row, and the largest below 3e38, beyond which a row is not packed (scal[0], as bits); scal[kScalLong]:
+// whether one is not; 16 lanes a row
 __global__ void __launch_bounds__(256) half_norms_kernel(const float* __restrict__ data, uint32_t n, uint32_t dim,
                                                          const float* __restrict__ centre, float* __restrict__ norm, uint32_t* __restrict__ scal) {
     const uint32_t j = threadIdx.x & 15;
     const float4* c4 = reinterpret_cast<const float4*>(centre);
-    float most = 0.0f, most_plain = 0.0f;
+    float most = 0.0f;
     for (uint32_t row = (blockIdx.x * 256 + threadIdx.x) >> 4; row < n; row += gridDim.x * 16) {
         const float4* r4 = reinterpret_cast<const float4*>(data + (size_t)row * dim);
-        float s = 0.0f, plain = 0.0f;
+        float s = 0.0f;
         for (uint32_t c = j; c < (dim >> 2); c += 16) {
             const float4 v = r4[c], m = c4[c];
             const float x = v.x - m.x, y = v.y - m.y, z = v.z - m.z, w = v.w - m.w;
@@ -113,20 +113,14 @@ __global__ void __launch_bounds__(256) half_norms_kernel(const float* __restrict
             s = __builtin_fmaf(y, y, s);
             s = __builtin_fmaf(z, z, s);
             s = __builtin_fmaf(w, w, s);
-            plain = __builtin_fmaf(v.x, v.x, __builtin_fmaf(v.y, v.y, __builtin_fmaf(v.z, v.z, __builtin_fmaf(v.w, v.w, plain))));
         }
 #pragma unroll
-        for (int m = 1; m < 16; m <<= 1) {
-            s += __shfl_xor(s, m, 64);
-            plain += __shfl_xor(plain, m, 64);
-        }
+        for (int m = 1; m < 16; m <<= 1) s += __shfl_xor(s, m, 64);
         if (j == 0) norm[row] = s;
         if (j == 0 && s >= 3.0e38f) scal[kScalLong] = 1u;
         if (s < 3.0e38f) most = fmaxf(most, s);
-        most_plain = fmaxf(most_plain, plain);
     }
     note_largest(most, scal);
-    note_largest(most_plain, scal + kScalPlain);
 }
 
 // Rows into blocks: place p of the output is row p (kAll), row p * n / count (kSpaced), row perm[p] (kOrdered) or one of 2^count

@@ -42,11 +42,11 @@ constexpr uint32_t kSampleValues = 1024;
 constexpr uint32_t kBoundValues = 2048;  // sampled values that a query looks at, at most: 32 a lane
 
 // Tile-grid rows into blocks, and per query: squared norm of the rounded, scaled row (-1: not taken), what rounding moved it,
-// its squared norm centred and as it is, its scale.  16 lanes a row.
+// its squared norm, its scale.  16 lanes a row.
 __global__ void __launch_bounds__(256) scan_pack_kernel(const float* __restrict__ queries, const uint32_t* __restrict__ row_query, const uint32_t* __restrict__ row_lo,
                                                         const uint32_t* __restrict__ row_hi, uint32_t rows, uint32_t dim, uint32_t ks_count, uint32_t frags, int ip,
                                                         const float* __restrict__ centre, const uint32_t* __restrict__ scal, uint4* __restrict__ blocks, uint4* __restrict__ row_frags,
-                                                        float* __restrict__ q_hn, float* __restrict__ q_eps, float* __restrict__ q_norm, float* __restrict__ q_plain, float* __restrict__ q_scale,
+                                                        float* __restrict__ q_hn, float* __restrict__ q_eps, float* __restrict__ q_norm, float* __restrict__ q_scale,
                                                         uint32_t* __restrict__ flag) {
     const uint32_t p = (blockIdx.x * 256 + threadIdx.x) >> 4, j = threadIdx.x & 15;
     if (p >= rows) return;  // whole groups of 16 lanes
@@ -54,18 +54,14 @@ __global__ void __launch_bounds__(256) scan_pack_kernel(const float* __restrict_
     const uint32_t q = row_query[p];
     const float4* x4 = reinterpret_cast<const float4*>(queries + (size_t)q * dim);
     const float4* c4 = reinterpret_cast<const float4*>(centre);
-    float s = 0.0f, plain = 0.0f;
+    float s = 0.0f;
     for (uint32_t c = j; c < (dim >> 2); c += 16) {
         const float4 v = x4[c], m = c4[c];
         const float x = v.x - m.x, y = v.y - m.y, z = v.z - m.z, w = v.w - m.w;
         s = __builtin_fmaf(x, x, __builtin_fmaf(y, y, __builtin_fmaf(z, z, __builtin_fmaf(w, w, s))));
-        plain = __builtin_fmaf(v.x, v.x, __builtin_fmaf(v.y, v.y, __builtin_fmaf(v.z, v.z, __builtin_fmaf(v.w, v.w, plain))));
     }
 #pragma unroll
-    for (int m = 1; m < 16; m <<= 1) {
-        s += __shfl_xor(s, m, 64);
-        plain += __shfl_xor(plain, m, 64);
-    }
+    for (int m = 1; m < 16; m <<= 1) s += __shfl_xor(s, m, 64);
     const float scale = (ip ? scale_of(s < 3.0e38f ? s : 0.0f) : scale_of(__uint_as_float(scal[0]))) * kScanLift;
     const bool good = s < 3.0e38f && s * scale * scale < 2.68e8f;  // 2^28
     uint4* block = blocks + (size_t)(p >> 5) * frags * 64 + (p & 31);
@@ -100,7 +96,6 @@ __global__ void __launch_bounds__(256) scan_pack_kernel(const float* __restrict_
         q_hn[q] = good ? sq : -1.0f;
         q_eps[q] = sqrtf(rem) / scale * 1.0001f + 1.3e-7f * sqrtf(s);
         q_norm[q] = s;
-        q_plain[q] = plain;
         q_scale[q] = scale;
         if (!good) *flag = 1u;
     }
@@ -473,7 +468,6 @@ struct ScanFinishArgs {
     const float* q_top;
     const float* q_eps;
     const float* q_norm;
-    const float* q_plain;
     const float* q_scale;
     const uint32_t* scal;
     uint32_t nq, k, dim, id_bits;
@@ -594,12 +588,14 @@ __global__ void __launch_bounds__(256) scan_finish_kernel(const ScanFinishArgs f
         }
         const double eps = f.q_eps[q], eps_max = __uint_as_float(f.scal[1]), cn = f.q_norm[q], cn_max = __uint_as_float(f.scal[0]);
         const double base_scale = (double)scale_of(__uint_as_float(f.scal[0])) * kScanLift, unit = (METRIC == kMetricL2 ? -2.0 : -1.0) / (base_scale * (double)f.q_scale[q]);
-        const double nq2 = f.q_plain[q], nb2 = __uint_as_float(f.scal[kScalPlain]);
+        // (the error of the products formed here, and none of a form on the rows as they are: with rows far from the origin, where that
+        // one tells nothing apart, these are centred.  100,000 x 128 about 100 in every coordinate, 300 windows of 20,000: 226 not proven
+        // and 3443 us a call with both, 155 with rows as two bf16 halves)
         if (METRIC == kMetricL2) {
-            form = fmax((3.25 * dim + 96.0) * u * (cn + cn_max), (1.25 * dim + 16.0) * u * (nq2 + nb2));
+            form = (3.25 * dim + 96.0) * u * (cn + cn_max);
             e_far = eps + eps_max;
         } else {
-            form = fmax((2.0 * dim + 96.0) * u * sqrt(cn * cn_max), 2.0 * (1.25 * dim + 16.0) * u * sqrt(nq2 * nb2));
+            form = (2.0 * dim + 96.0) * u * sqrt(cn * cn_max);
             e_far = eps * sqrt(cn_max) + (sqrt(cn) + eps) * eps_max + form;
         }
         const double top = f.q_top[q], way = top - (double)t, edge = (top - way * (high + 2.0) / parts) * unit;
@@ -806,7 +802,7 @@ bool half_scan_plan(const HalfBase& b, uint32_t num_cu, const uint32_t* h_row_lo
     s->sample_floats = (size_t)at * 4096;
     auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
     s->workspace_bytes = up((size_t)s->rows / 32 * b.frags * 1024) + up((size_t)s->rows / 32 * 2048) + up(s->sample_floats * 4) + up((size_t)s->rows * kScanListCap * 4) +
-                         up((size_t)s->nq * 28) + up((size_t)s->rows * 4 + 64 + (size_t)s->nq * 4);
+                         up((size_t)s->nq * 24) + up((size_t)s->rows * 4 + 64 + (size_t)s->nq * 4);
     return s->workspace_bytes <= max_bytes;
 }
 
@@ -824,8 +820,8 @@ int half_scan_async(const HalfBase& b, const HalfScan& s, const HalfScanArgs& gi
     uint4* row_frags = reinterpret_cast<uint4*>(take((size_t)rows / 32 * 2048));
     w.sample = reinterpret_cast<float*>(take(s.sample_floats * 4));
     w.list = reinterpret_cast<uint32_t*>(take((size_t)rows * kScanListCap * 4));
-    float* q_hn = reinterpret_cast<float*>(take((size_t)nq * 28));
-    float *q_eps = q_hn + nq, *q_norm = q_eps + nq, *q_plain = q_norm + nq, *q_scale = q_plain + nq, *q_t = q_scale + nq, *q_top = q_t + nq;
+    float* q_hn = reinterpret_cast<float*>(take((size_t)nq * 24));
+    float *q_eps = q_hn + nq, *q_norm = q_eps + nq, *q_scale = q_norm + nq, *q_t = q_scale + nq, *q_top = q_t + nq;
     // from zero: the lists' counts, two work counters, whether a query is not taken, the queries not proven; then which these are
     w.count = reinterpret_cast<uint32_t*>(take((size_t)rows * 4 + 64 + (size_t)nq * 4));
     uint32_t* counters = w.count + rows;
@@ -833,7 +829,7 @@ int half_scan_async(const HalfBase& b, const HalfScan& s, const HalfScanArgs& gi
     a.doubt = counters + 3;
     GRAB_HIP(hipMemsetAsync(w.count, 0, (size_t)rows * 4 + 64, st));
     hipLaunchKernelGGL(scan_pack_kernel, dim3(rows / 16), dim3(256), 0, st, a.queries, a.row_query, a.row_lo, a.row_hi, rows, b.dim, b.ks, b.frags, (int)b.ip, b.centre, b.scal,
-                       row_blocks, row_frags, q_hn, q_eps, q_norm, q_plain, q_scale, a.flag);
+                       row_blocks, row_frags, q_hn, q_eps, q_norm, q_scale, a.flag);
     w.row_blocks = row_blocks;
     w.row_frags = row_frags;
     w.blocks = b.blocks;
@@ -868,7 +864,6 @@ int half_scan_async(const HalfBase& b, const HalfScan& s, const HalfScanArgs& gi
     f.q_top = q_top;
     f.q_eps = q_eps;
     f.q_norm = q_norm;
-    f.q_plain = q_plain;
     f.q_scale = q_scale;
     f.scal = b.scal;
     f.nq = nq;

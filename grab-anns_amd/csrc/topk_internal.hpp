@@ -94,9 +94,7 @@ void launch_split_rows_chunked(const float* data, uint64_t n, uint32_t dim, cons
 
 // The candidates of a large kNN graph from f16 products: knn_half.hip.  Where it applies, a plan of the sizes, the lists, and
 // the neighbours that these prove.
-// words of `scal`: whether some row is not finite; the largest squared norm of the rows as they are; whether some row, not NaN, is too
-// long to be packed
-constexpr uint32_t kScalBad = 11, kScalPlain = 12, kScalLong = 13;
+constexpr uint32_t kScalBad = 11, kScalLong = 12;  // words of `scal`: whether some row is not finite; whether one, not NaN, is too long to be packed
 constexpr uint32_t kHalfListCap = 1024;  // keys of a row's list
 constexpr uint32_t kHalfSample = 49152;  // sample rows that the bounds are taken from, at most
 struct HalfKnn {

@@ -437,3 +437,25 @@ def test_scan_base_of_rows_that_are_not_finite_keeps_no_f16_rows(grab):
     halves = free - grab.device_memory()[0]
     base.close()
     assert kept > 0 and halves < n * (dim * 4 + 4) + (64 << 20)  # halves and norms, and no more
+
+
+@pytest.mark.parametrize("nq,k,widths", [(1, 10, (20000, 25000)), (300, 10, (9000, 25000)), (1100, 40, (100, 25000))])
+def test_scans_of_rows_far_from_the_origin(oracle, grab, nq, k, widths):
+    # a hundred standard deviations in every coordinate: the rows are centred, and so is what the proof allows for
+    n, dim = 25000, 128
+    data, q = datasets.gaussian(n, dim, 4) + np.float32(100.0), datasets.gaussian(nq, dim, 7) + np.float32(100.0)
+    lo, hi = _intervals(n, nq, widths[0], widths[1], nq)
+    d_data, d_q = grab.DeviceArray.from_numpy(data), grab.DeviceArray.from_numpy(q)
+    base = grab.ScanBase(d_data, n, dim, 0)
+    ids, dist, _ = base.window_topk(d_q, nq, k, lo, hi)
+    assert grab.last_knn_f16_flop() > 0 and grab.last_knn_exact_rows() <= 3
+    eids, edist = oracle.bruteforce_topk(data, q, k, filter_kind=oracle.FILTER_RANGE, ts=np.arange(n, dtype=np.uint64), win_start=lo, win_end=hi)
+    assert np.array_equal(ids, eids) and np.array_equal(dist.view(np.uint32), edist.view(np.uint32))
+    offsets = np.array([0, 3000, 3100, 15000, n], np.uint64)
+    masks = np.random.default_rng(nq).integers(1, 16, nq).astype(np.uint64)
+    ids, dist, _ = base.bucket_topk(offsets, d_q, nq, k, masks)
+    assert grab.last_knn_f16_flop() > 0 and grab.last_knn_exact_rows() <= 3
+    base.close()
+    labels = np.repeat(np.arange(4, dtype=np.uint8), np.diff(offsets.astype(np.int64)))
+    eids, edist = oracle.bruteforce_topk(data, q, k, filter_kind=oracle.FILTER_MASK, labels=labels, masks=masks)
+    assert np.array_equal(ids, eids) and np.array_equal(dist.view(np.uint32), edist.view(np.uint32))
