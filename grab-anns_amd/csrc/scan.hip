@@ -551,9 +551,15 @@ void dense_sched(const uint32_t* tile_lo, const uint32_t* tile_hi, uint32_t row_
 // What the quick way needs beyond the rows: the rows of a subset of the queries (ascending query numbers), for the plain way.
 using SubRows = std::function<void(const std::vector<uint32_t>& which, ScanRows* out)>;
 
-// Queries whose candidates prove nothing (distances far below the rounding error of the GEMM form), doubt[1 .. n_doubt]: the plain way
+enum RowsAs { kOnF16, kAsHalves, kAsTheyAre };  // on f16 rows wherever these serve; as two bf16 halves where the base has or makes them, or at once
+int scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const ScanRows& rw, const SubRows& sub_rows, const float* d_queries, size_t num_queries,
+              uint32_t k, int metric, int64_t* d_out_indices, float* d_out_dists, float* kernel_ms, hipStream_t st, const ScanBase* base, RowsAs rows_as);
+
+// Queries that a pass could not prove, doubt[1 .. n_doubt]: all those of a pass on f16 rows once more (rows_as other than kOnF16; base: the
+// call's), the plain way after any other pass.
 int unproven_queries(const float* d_dataset, size_t num_dataset, uint32_t dim, const SubRows& sub_rows, const float* d_queries, uint32_t k, int metric,
-                     const uint32_t* doubt, uint32_t n_doubt, int64_t* d_out_indices, float* d_out_dists, hipStream_t st) {
+                     const uint32_t* doubt, uint32_t n_doubt, int64_t* d_out_indices, float* d_out_dists, hipStream_t st, RowsAs rows_as = kOnF16,
+                     const ScanBase* base = nullptr) {
     std::vector<uint32_t> which(n_doubt);
     GRAB_HIP(hipMemcpy(which.data(), doubt + 1, (size_t)n_doubt * 4, hipMemcpyDeviceToHost));
     std::sort(which.begin(), which.end());
@@ -568,13 +574,24 @@ int unproven_queries(const float* d_dataset, size_t num_dataset, uint32_t dim, c
     hipLaunchKernelGGL(gather_query_rows_kernel, dim3((uint32_t)(((size_t)n_doubt * 8 + 255) / 256)), dim3(256), 0, st, d_queries,
                        d_which.as<uint32_t>(), n_doubt, dim, sub_q.as<float>());
     GRAB_HIP(hipGetLastError());
-    const double flop_fp32 = knn_stats().flop, flop_bf16 = knn_stats().flop_bf16, flop_f16 = knn_stats().flop_f16;
-    GRAB_TRY(bucket_scan_by_rows(d_dataset, num_dataset, dim, sub, sub_q.as<float>(), n_doubt, k, metric, sub_ids.as<int64_t>(),
-                                 sub_dist.as<float>(), st));
-    knn_stats().flop = flop_fp32;  // the figures of the main pass
-    knn_stats().flop_bf16 = flop_bf16;
-    knn_stats().flop_f16 = flop_f16;
-    knn_stats().exact_rows = n_doubt;
+    const KnnStats main_pass = knn_stats();
+    const bool again = rows_as != kOnF16;
+    if (again) {
+        const SubRows of_these = [&](const std::vector<uint32_t>& some, ScanRows* out) {
+            std::vector<uint32_t> of_call(some);
+            for (uint32_t& q : of_call) q = which[q];
+            sub_rows(of_call, out);
+        };
+        GRAB_TRY(scan_topk(d_dataset, num_dataset, dim, sub, of_these, sub_q.as<float>(), n_doubt, k, metric, sub_ids.as<int64_t>(), sub_dist.as<float>(), nullptr,
+                           st, base, rows_as));
+    } else {
+        GRAB_TRY(bucket_scan_by_rows(d_dataset, num_dataset, dim, sub, sub_q.as<float>(), n_doubt, k, metric, sub_ids.as<int64_t>(),
+                                     sub_dist.as<float>(), st));
+    }
+    const uint64_t exact = again ? knn_stats().exact_rows : n_doubt;
+    knn_stats() = main_pass;  // the figures of the main pass
+    knn_stats().exact_rows = main_pass.exact_rows + exact;
+    if (again) knn_stats().redone_rows += n_doubt;
     hipLaunchKernelGGL(scatter_results_kernel, dim3((n_doubt * k + 255) / 256), dim3(256), 0, st, sub_ids.as<int64_t>(), sub_dist.as<float>(),
                        d_which.as<uint32_t>(), n_doubt, k, d_out_indices, d_out_dists);
     GRAB_HIP(hipGetLastError());
@@ -681,15 +698,15 @@ int scan_half_pass(const HalfBase& b, const float* d_dataset, size_t num_dataset
     knn_stats().flop_f16 += rw.tiles * 2.0 * TM * TN * dim;
     knn_stats().flop_bf16 = 3.0 * knn_stats().flop_f16;
     if (left[1] == 0) return GRAB_OK;
-    const uint64_t exact_before = knn_stats().exact_rows;
     const SubRows own_rows = [&](const std::vector<uint32_t>& which, ScanRows* out) {
         std::vector<uint32_t> of_call(which);
         for (uint32_t& q : of_call) q += first;
         sub_rows(of_call, out);
     };
-    GRAB_TRY(unproven_queries(d_dataset, num_dataset, dim, own_rows, a.queries, k, metric, w + 1, left[1], a.out_ids, a.out_dist, st));
-    knn_stats().exact_rows += exact_before;
-    return GRAB_OK;
+    // These are few as a rule, and the fp32 instructions' error is the smallest; halves of all rows are made for many
+    const bool halves = left[1] >= kHalfPassQueries || (base && base->rows_split);
+    return unproven_queries(d_dataset, num_dataset, dim, own_rows, a.queries, k, metric, w + 1, left[1], a.out_ids, a.out_dist, st, halves ? kAsHalves : kAsTheyAre,
+                            halves ? base : nullptr);
 }
 
 // The f16 way.  *applied = false: nothing is to be used of it.
@@ -722,7 +739,7 @@ int scan_topk_half(const float* d_dataset, size_t num_dataset, uint32_t dim, con
 // check run once per query, not once per tile-grid row.  Queries that the check cannot prove go the plain way.
 int scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const ScanRows& rw, const SubRows& sub_rows,
               const float* d_queries, size_t num_queries, uint32_t k, int metric, int64_t* d_out_indices, float* d_out_dists,
-              float* kernel_ms, hipStream_t st, const ScanBase* base = nullptr) {
+              float* kernel_ms, hipStream_t st, const ScanBase* base, RowsAs rows_as) {
     const uint32_t rows = rw.rows, nq = (uint32_t)num_queries;
     knn_stats().flop = knn_stats().flop_bf16 = knn_stats().flop_f16 = 0.0;
     knn_stats().redone_rows = knn_stats().exact_rows = 0;
@@ -733,7 +750,7 @@ int scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const Sc
     const uint32_t kk = std::max<uint32_t>(2 * k + 32, 64);  // <= 288
     const uint32_t row_tiles = rows / TM, col_tiles = (uint32_t)((num_dataset + TN - 1) / TN), target = (uint32_t)num_cu * 2;
     // a prepared base has paid for its split rows; otherwise splitting a million rows pays from a thousand query rows on
-    bool split = base ? base->split : knn_bf16_allowed() && dim % KC == 0 && rows >= 1024 && num_dataset >= 4096;
+    bool split = base ? base->split : rows_as != kAsTheyAre && knn_bf16_allowed() && dim % KC == 0 && rows >= 1024 && num_dataset >= 4096;
     // On f16 rows, except narrow intervals with short lists: a tenth of an interval's columns would be listed, and writing all values
     // costs less.  A call over a prepared base, stored values against this way in us, k 10, intervals of 1000, 4000, 6000 and 8000:
     //   1M x 128, 100 queries     221 / 243, 230 / 223, 236 / 215, 241 / 212      150,000 x 768  197 / 198, 209 / 199, 213 / 193, 219 / 196
@@ -745,7 +762,7 @@ int scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const Sc
     const bool narrow = rw.one_row_per_query && kk <= 64 && rw.columns < (rw.lists.size() <= 2 ? 10000ull : 6000ull) * rw.lists.size();
     // Beyond 127,000 columns a sampled value stands for more than 64 columns, too few lie within a bound to set it by; by the same
     // reckoning as at 100,000 from one in 130 (scan_half.hip: 5.3 ms a call against 3.3 with stored values).
-    bool on_half = split && half_scan_takes(rw.widest) && (!base || base->half), applied = false;
+    bool on_half = rows_as == kOnF16 && split && half_scan_takes(rw.widest) && (!base || base->half), applied = false;
     if (on_half && !rw.one_row_per_query) {
         uint32_t most = 0;  // rows of a query; a wave's lanes hold them
         for (size_t q = 0; q < num_queries; ++q) most = std::max(most, rw.list_off[q + 1] - rw.list_off[q]);
@@ -971,7 +988,6 @@ int scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const Sc
         set_error("scan: re-scoring failed");
         return rc;
     }
-    knn_stats().exact_rows = n_doubt;
     if (n_doubt == 0) return GRAB_OK;
     return unproven_queries(d_dataset, num_dataset, dim, sub_rows, d_queries, k, metric, doubt.as<uint32_t>(), n_doubt, d_out_indices, d_out_dists, st);
 }
@@ -1005,7 +1021,7 @@ int grab_bucket_scan_topk(const float* d_dataset, size_t num_dataset, uint32_t d
         for (size_t i = 0; i < which.size(); ++i) sub_masks[i] = h_masks[which[i]];
         scan_rows(h_bucket_offsets, num_buckets, sub_masks.data(), which.size(), out);
     };
-    return scan_topk(d_dataset, num_dataset, dim, rw, sub_rows, d_queries, num_queries, k, metric, d_out_indices, d_out_dists, kernel_ms, st);
+    return scan_topk(d_dataset, num_dataset, dim, rw, sub_rows, d_queries, num_queries, k, metric, d_out_indices, d_out_dists, kernel_ms, st, nullptr, kOnF16);
 }
 
 int grab_window_scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const float* d_queries, size_t num_queries,
@@ -1024,7 +1040,7 @@ int grab_window_scan_topk(const float* d_dataset, size_t num_dataset, uint32_t d
         window_rows(h_id_lo, h_id_hi, which.data(), which.size(), num_dataset, out);
     };
     return scan_topk(d_dataset, num_dataset, dim, rw, sub_rows, d_queries, num_queries, k, metric, d_out_indices, d_out_dists, kernel_ms,
-                     static_cast<hipStream_t>(stream));
+                     static_cast<hipStream_t>(stream), nullptr, kOnF16);
 }
 
 // A base prepared for the two scans: what a call would otherwise make of the base rows every time, and a block of
@@ -1175,7 +1191,7 @@ int grab_scan_base_window_topk(grab_scan_base* b, const float* d_queries, size_t
     };
     return scan_on_base(b, [&]() {
         return scan_topk(b->d_dataset, b->num_dataset, b->dim, rw, sub_rows, d_queries, num_queries, k, b->metric, d_out_indices,
-                         d_out_dists, kernel_ms, static_cast<hipStream_t>(stream), &b->view);
+                         d_out_dists, kernel_ms, static_cast<hipStream_t>(stream), &b->view, kOnF16);
     });
 }
 
@@ -1200,7 +1216,7 @@ int grab_scan_base_bucket_topk(grab_scan_base* b, const uint64_t* h_bucket_offse
     };
     return scan_on_base(b, [&]() {
         return scan_topk(b->d_dataset, b->num_dataset, b->dim, rw, sub_rows, d_queries, num_queries, k, b->metric, d_out_indices,
-                         d_out_dists, kernel_ms, static_cast<hipStream_t>(stream), &b->view);
+                         d_out_dists, kernel_ms, static_cast<hipStream_t>(stream), &b->view, kOnF16);
     });
 }
 

@@ -423,7 +423,8 @@ int grab_generate_knn_graph(const float* d_dataset, size_t num_dataset, uint32_t
  * of 16384 rows or more (4096 where grab_last_knn_bf16_flop applies), the rows that its symmetric pass handed back to
  * the plain pass.  From that size on the graph's contraction computes only the tiles on and above the diagonal - about
  * half of 2 N^2 dim - plus every row against a sample of the rows, which bounds what a tile contributes to the rows
- * behind its columns. */
+ * behind its columns.  After a scan: the queries that its pass on f16 rows did not prove and a second pass, on bf16 halves or the
+ * rows as they are, took over. */
 int grab_last_knn_stats(double* flop, uint64_t* rows_redone);
 /* The candidates of a row are picked by |a|^2+|b|^2-2ab (or -ab) on the matrix cores and only then scored exactly.
  * After the exact scoring every row is checked: its k-th exact distance must lie below the smallest GEMM-form
