@@ -274,11 +274,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
                     if (SAMPLE) {
                         const uint32_t* t = a.tiles + 4 * rt;
                         const uint32_t pitch = t[1] * 32, at = (sampled + nth) * 32 + l32;
-                        float* out = a.sample + (size_t)t[0] * 4096 + at;
+                        float* out = a.sample + (size_t)t[0] * 4096 + (size_t)(wr * 64 + 4 * half) * pitch + at;
 #pragma unroll
-                        for (uint32_t rb = 0; rb < 2; ++rb)
+                        for (uint32_t rb = 0; rb < 2; ++rb)  // (the rows one after the other: 32 addresses at once do not fit the registers)
 #pragma unroll
-                            for (uint32_t v = 0; v < 16; ++v) out[(size_t)(wr * 64 + rb * 32 + (v & 3) + 8 * (v >> 2) + 4 * half) * pitch] = acc[rb][cb][v];
+                            for (uint32_t v = 0; v < 16; ++v) {
+                                *out = acc[rb][cb][v];
+                                out += (size_t)pitch * (v % 4 == 3 ? 5 : 1);
+                            }
                     } else {
                         const uint32_t j0 = min(first + nth, a.last_block) * 32;
 #pragma unroll
