@@ -751,15 +751,22 @@ int scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const Sc
     const uint32_t row_tiles = rows / TM, col_tiles = (uint32_t)((num_dataset + TN - 1) / TN), target = (uint32_t)num_cu * 2;
     // a prepared base has paid for its split rows; otherwise splitting a million rows pays from a thousand query rows on
     bool split = base ? base->split : rows_as != kAsTheyAre && knn_bf16_allowed() && dim % KC == 0 && rows >= 1024 && num_dataset >= 4096;
-    // On f16 rows, except narrow intervals with short lists: a tenth of an interval's columns would be listed, and writing all values
-    // costs less.  A call over a prepared base, stored values against this way in us, k 10, intervals of 1000, 4000, 6000 and 8000:
-    //   1M x 128, 100 queries     221 / 243, 230 / 223, 236 / 215, 241 / 212      150,000 x 768  197 / 198, 209 / 199, 213 / 193, 219 / 196
-    //   400,000 x 96, 100         119 / 145, 130 / 136, 134 / 134, 140 / 134      200,000 x 384  151 / 168, 161 / 157, 166 / 156, 172 / 157
-    // Where the lines cross moves with the batch: 3000 at 10,000 queries (430 / 406 of 1M x 128), 6000 from eight to a thousand, 10,000
-    // for one or two, which wait for this way's one launch more: one query, intervals of 6000, 8000 and 12,000 81 / 86, 86 / 88, 94 / 95
-    // of 1M x 128 and 114 / 127, 117 / 123, 125 / 130 of 150,000 x 768.
-    // Longer lists, selection inside the contraction against this: k 40, 10,000 queries, 1000 columns 1361 / 472, 20,000 3743 / 574.
-    const bool narrow = rw.one_row_per_query && kk <= 64 && rw.columns < (rw.lists.size() <= 2 ? 10000ull : 6000ull) * rw.lists.size();
+    // On f16 rows, except narrow intervals with short lists: a tenth of an interval's columns would be listed, and writing all values costs
+    // less.  What this way saves goes with the products of the sweep, of which it takes one of three, with the queries, and with the
+    // columns that one query's wave selects from; against that stand some 25 us of launches and of sampling.  Seven row sets from 300,000 x 32 to
+    // 150,000 x 768, 1 to 10,000 queries, intervals of 3000 to 15,000, k 10 and 16, a call over a prepared base: the rule's choice takes
+    // 0.3 % more than the better one in the mean, 4 % more than stored values at worst (a line at 6000 columns: 2 %, and 19 %).  Intervals of
+    // 3000, 6000 and 11,000, k 10, stored values against this way in us:
+    //   300,000 x 32   1 query 69 / 84, 76 / 85, 86 / 86;         300 106 / 131, 113 / 132, 126 / 131;   10,000 273 / 285, 343 / 300, 458 / 320
+    //   1M x 128       1       73 / 93, 81 / 87, 92 / 92;         300 240 / 230, 250 / 221, 265 / 213;   10,000 443 / 398, 529 / 409, 666 / 428
+    //   150,000 x 768  1       101 / 111, 115 / 110, 128 / 114;   300 216 / 207, 228 / 195, 242 / 191;   10,000 579 / 437, 735 / 494, 1027 / 585
+    // Below 3000 none was measured to gain (1000, 10,000 queries of 1M x 128: 384 / 582).  Longer lists, selection inside the contraction against
+    // this: k 40, 10,000 queries, 1000 columns 1361 / 472, 20,000 3743 / 574.
+    bool narrow = false;
+    if (rw.one_row_per_query && kk <= 64) {
+        const double queries = (double)rw.lists.size(), mean = (double)rw.columns / queries;
+        narrow = mean < 3000.0 || rw.tiles * dim / 30000.0 + queries / 800.0 + mean / 430.0 < 26.0;
+    }
     // Beyond 127,000 columns a sampled value stands for more than 64 columns, too few lie within a bound to set it by; by the same
     // reckoning as at 100,000 from one in 130 (scan_half.hip: 5.3 ms a call against 3.3 with stored values).
     bool on_half = rows_as == kOnF16 && split && half_scan_takes(rw.widest) && (!base || base->half), applied = false;

@@ -223,7 +223,8 @@ def test_window_scan_in_several_passes(oracle, grab):
 
 
 @pytest.mark.parametrize("n,dim,nq,k,metric,widths,kind", [
-    (30000, 96, 1200, 10, 0, (5900, 9000), "mix"),     # ties between integer rows, intervals wide enough for short lists
+    (30000, 96, 1200, 10, 0, (5900, 9000), "mix"),     # ties between integer rows; narrow for short lists
+    (30000, 96, 1200, 10, 0, (11000, 14000), "mix"),   # ... and wide enough
     (12001, 32, 1030, 128, 0, (1, 12001), "gauss"),    # the longest lists, intervals from one row to all
     (20000, 288, 1100, 16, 1, (6100, 15000), "unit"),  # an odd number of chunks of 32 dimensions
     (40000, 128, 1500, 40, 1, (200, 300), "unit"),     # narrow intervals, lists too long for stored values
@@ -244,7 +245,7 @@ def test_window_scan_on_f16_rows(oracle, grab, n, dim, nq, k, metric, widths, ki
     d_data, d_q = grab.DeviceArray.from_numpy(data), grab.DeviceArray.from_numpy(q)
     base = grab.ScanBase(d_data, len(data), dim, metric)
     ids, dist, _ = base.window_topk(d_q, nq, k, lo, hi)
-    assert (grab.last_knn_f16_flop() > 0) == (kind != "far") and grab.last_knn_bf16_flop() > 0
+    assert (grab.last_knn_f16_flop() > 0) == (kind != "far" and widths != (5900, 9000)) and grab.last_knn_bf16_flop() > 0
     base.close()
     eids, edist = oracle.bruteforce_topk(data, q, k, metric=metric, filter_kind=oracle.FILTER_RANGE, ts=np.arange(len(data), dtype=np.uint64),
                                          win_start=lo, win_end=np.minimum(hi, np.uint64(len(data))))
@@ -285,7 +286,7 @@ def test_scans_beyond_67_million_rows(oracle, grab, edge, dim, k):
     d_data.fill_bytes(0)
     grab.check(grab.lib.grab_copy_to_device(C.c_void_p(d_data.ptr + first * dim * 4), data.ctypes.data_as(C.c_void_p), C.c_size_t(data.nbytes)))
     rng = np.random.default_rng(k)
-    width = np.where(np.arange(nq) % 3 == 0, rng.integers(1, 257, nq), rng.integers(12000, 20000, nq))
+    width = np.where(np.arange(nq) % 3 == 0, rng.integers(1, 257, nq), rng.integers(18000, 20000, nq))
     lo = np.where(np.arange(nq) % 2 == 0, rng.integers(edge, n - width), np.maximum(edge - rng.integers(0, width + 1), first)).astype(np.uint64)
     hi = np.minimum(lo + width.astype(np.uint64), np.uint64(n))
     base = grab.ScanBase(d_data, n, dim, 0)
@@ -328,9 +329,10 @@ def test_window_scan_of_rows_that_resemble_their_neighbours(oracle, grab, run, k
     assert np.array_equal(ids, eids) and np.array_equal(dist.view(np.uint32), edist.view(np.uint32))
 
 
-@pytest.mark.parametrize("nq,width,k,on_f16", [(1, 9999, 10, False), (1, 10000, 16, True), (2, 9000, 10, False), (3, 6000, 10, True), (3, 5999, 16, False), (3, 300, 17, True)])
+@pytest.mark.parametrize("nq,width,k,on_f16", [(1, 11000, 10, False), (1, 11400, 16, True), (2, 10500, 10, False), (2, 11300, 10, True), (300, 9000, 16, False),
+                                               (300, 11000, 10, True), (3000, 2999, 16, False), (3, 300, 17, True)])
 def test_window_scan_of_few_queries(oracle, grab, nq, width, k, on_f16):
-    # narrow intervals with short lists keep the way of stored values, and narrower than ten thousand is narrow for one or two
+    # narrow intervals with short lists keep the way of stored values, the longer the fewer the queries and the shorter the rows
     n, dim = 30000, 64
     data, q = datasets.gaussian(n, dim, 4), datasets.gaussian(nq, dim, 7)
     lo, hi = _intervals(n, nq, width, width, nq)
