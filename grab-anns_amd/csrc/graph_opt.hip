@@ -190,12 +190,11 @@ __global__ void __launch_bounds__(256) prune_map_kernel(const uint32_t* __restri
     // every id writes its place; who finds another's there shares the byte with it, or is the same id once more
     for (uint32_t p = lane; p < deg; p += 64) map[slot_of(row[p])] = (uint8_t)p;
     wave_sync();
-    bool lost[(MAXDEG + 63) / 64], again = false;
+    bool lost[(MAXDEG + 63) / 64];
 #pragma unroll
     for (uint32_t i = 0; i < (MAXDEG + 63) / 64; ++i) {
         const uint32_t p = 64 * i + lane, at = p < deg ? map[slot_of(row[p])] : p;
         lost[i] = at != p;
-        again = again || (at != p && row[at] == row[p]);
     }
     wave_sync();
     for (uint32_t i = 0; i < (MAXDEG + 63) / 64; ++i)
@@ -205,10 +204,6 @@ __global__ void __launch_bounds__(256) prune_map_kernel(const uint32_t* __restri
         if (map[slot_of(row[p])] == kShared) shared[atomicAdd(&s.shared_count[wave], 1u)] = p;
     wave_sync();
     const uint32_t n_shared = s.shared_count[wave];
-    // the same id twice in a row (padding included) may also hide behind a shared byte
-    for (uint32_t i = lane; i < n_shared; i += 64)
-        for (uint32_t x = 0; x < n_shared; ++x) again = again || (x != i && row[shared[x]] == row[shared[i]]);
-    const bool duplicates = __ballot(again) != 0;
 
     // eight D rows per round: their reads are in flight together, and so are the eight reads of the map
     constexpr int U = 8;
@@ -226,29 +221,22 @@ __global__ void __launch_bounds__(256) prune_map_kernel(const uint32_t* __restri
             for (int u = 0; u < U; ++u) bc[u] = dnode[u] != kInvalidId ? knn[(size_t)dnode[u] * deg + kDB] : 0u;
 #pragma unroll
             for (int u = 0; u < U; ++u) at[u] = map[slot_of(bc[u])];
-            if (!duplicates) {
-                uint32_t there[U];
+            uint32_t there[U];
 #pragma unroll
-                for (int u = 0; u < U; ++u) there[u] = row[at[u] < kShared ? at[u] : 0u];
+            for (int u = 0; u < U; ++u) there[u] = row[at[u] < kShared ? at[u] : 0u];
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const uint32_t kAD = k0 + u;
-                    uint32_t p = there[u] == bc[u] && at[u] < kShared ? at[u] : 0u;  // place 0 is behind no kAD
-                    if (at[u] == kShared)
-                        for (uint32_t x = 0; x < n_shared; ++x) p = row[shared[x]] == bc[u] ? shared[x] : p;
-                    if (dnode[u] != kInvalidId && p > kAD) atomicAdd(&cnt[p], 1u);
-                }
-                continue;
-            }
-#pragma unroll 1
-            for (int u = 0; u < U; ++u) {  // cagra.cu:262-271 as written
+            for (int u = 0; u < U; ++u) {
                 const uint32_t kAD = k0 + u;
-                if (dnode[u] == kInvalidId || at[u] == kNone) continue;
-                for (uint32_t kAB = kAD + 1; kAB < deg; ++kAB)
-                    if (row[kAB] == bc[u]) {
-                        atomicAdd(&cnt[kAB], 1u);
-                        break;
+                uint32_t p = there[u] == bc[u] && at[u] < kShared ? at[u] : 0u;  // place 0 is behind no kAD
+                if (at[u] == kShared) {  // the id's first place behind kAD (cagra.cu:262-271): a row may hold it, or padding, several times
+                    uint32_t first = kNone;
+                    for (uint32_t x = 0; x < n_shared; ++x) {
+                        const uint32_t place = shared[x];
+                        first = row[place] == bc[u] && place > kAD ? min(first, place) : first;
                     }
+                    p = first != kNone ? first : 0u;
+                }
+                if (dnode[u] != kInvalidId && p > kAD) atomicAdd(&cnt[p], 1u);
             }
         }
     }
