@@ -110,7 +110,7 @@ def test_prune_duplicate_ids_and_hubs(oracle, grab):
     assert np.array_equal(d_g.numpy(), oracle.merge_graphs(g, erev, ecnt))
 
 
-@pytest.mark.parametrize("deg", [1, 2, 63, 64, 65, 127, 128, 129])
+@pytest.mark.parametrize("deg", [1, 2, 7, 8, 63, 64, 65, 127, 128, 129])
 def test_prune_of_ids_that_share_a_byte_of_the_map(oracle, grab, deg):
     # a row's ids are found through a byte of 4096 by a multiplicative hash; ids below 4096 hardly ever share one, so the rows
     # hold ids that do (groups of two and three), from few enough of them that neighbours' lists overlap
