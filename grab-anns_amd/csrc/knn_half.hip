@@ -613,6 +613,7 @@ struct FinishArgs {
     uint32_t* redo;
     uint32_t* doubt;      // [0] how many, then the rows: distances below what the forms resolve
     uint32_t n, dim, k, cap, min_list, id_bits;
+    uint32_t redo_keep;   // candidates that the plain pass keeps for a row
 };
 constexpr uint32_t kFinishCap = 1024;
 template <int METRIC>
@@ -739,7 +740,16 @@ __global__ void __launch_bounds__(256) knn_finish_kernel(const FinishArgs a) {
         }
         if (!proven) {  // (also where something is not a number)
             if (lane == 0) {
-                if (form > 0.005 * fabs(bound)) a.doubt[1 + atomicAdd(a.doubt, 1u)] = row;  // the plain pass has a form of its own, as far off: a longer list would hardly help
+                // the plain pass has a form of its own, as far off: a longer list would hardly help
+                bool hopeless = form > 0.005 * fabs(bound);
+                if (METRIC == kMetricIP) {
+                    // on bf16 halves it is off by half_err; how far its last candidate lies behind the k-th is reckoned from this list.  (Unit rows
+                    // in tight clusters, 20,000 x 128: none of 20,000 was proven there, 29.3 ms a call with that pass, 22.4 before f16 rows)
+                    const double half_err = 2.0 * (7.25 * dim + 816.0) * u * sqrt((double)a.norm[row] * (double)*a.max_norm);
+                    const double more = have < a.redo_keep ? (double)(a.redo_keep - have) / (double)(have - need) : 0.0;
+                    hopeless = hopeless || (bound - last) * (1.0 + more) < 0.5 * half_err;
+                }
+                if (hopeless) a.doubt[1 + atomicAdd(a.doubt, 1u)] = row;
                 else a.redo[atomicAdd(a.redo_count, 1u)] = row;
             }
             return;
@@ -942,7 +952,7 @@ int half_knn_lists_async(const float* data, HalfKnn* h, void* workspace, uint32_
     return GRAB_OK;
 }
 
-int half_knn_finish_async(const float* data, const HalfKnn& h, uint32_t k, const float* norm, const float* max_norm, uint32_t* out,
+int half_knn_finish_async(const float* data, const HalfKnn& h, uint32_t k, uint32_t redo_keep, const float* norm, const float* max_norm, uint32_t* out,
                           uint32_t* redo_count, uint32_t* redo, uint32_t* doubt, hipStream_t st) {
     FinishArgs f{};
     f.data = data;
@@ -964,6 +974,7 @@ int half_knn_finish_async(const float* data, const HalfKnn& h, uint32_t k, const
     f.n = h.n;
     f.dim = h.dim;
     f.k = k;
+    f.redo_keep = redo_keep;
     f.cap = kHalfListCap;
     f.min_list = h.min_list;
     f.id_bits = h.id_bits;

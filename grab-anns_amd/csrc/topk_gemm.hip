@@ -1267,7 +1267,7 @@ static int knn_graph_half(const TopkProblem& p, uint32_t kk, uint32_t num_cu, bo
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
     GRAB_TRY(rc);
-    GRAB_TRY(half_knn_finish_async(p.B, h, p.k, norm.as<float>(), reinterpret_cast<const float*>(max_norm), p.out_u32, w, redo, w + 1, stream));
+    GRAB_TRY(half_knn_finish_async(p.B, h, p.k, kk, norm.as<float>(), reinterpret_cast<const float*>(max_norm), p.out_u32, w, redo, w + 1, stream));
     uint32_t left[2] = {0, 0};
     GRAB_HIP(hipMemcpyAsync(left, w, 8, hipMemcpyDeviceToHost, stream));
     GRAB_HIP(hipStreamSynchronize(stream));

@@ -117,7 +117,7 @@ int half_knn_plan(uint32_t n, uint32_t dim, uint32_t k, int metric, HalfKnn* h);
 int half_knn_lists_async(const float* data, HalfKnn* h, void* workspace, uint32_t* list, uint32_t num_cu, hipStream_t st);
 // queued on `st`: out[row][k]; rows that their lists do not prove are listed in redo (a longer list may) or doubt[1..] (it
 // cannot), their numbers in *redo_count and doubt[0], zero before.  norm, max_norm: of the rows as they are
-int half_knn_finish_async(const float* data, const HalfKnn& h, uint32_t k, const float* norm, const float* max_norm, uint32_t* out,
+int half_knn_finish_async(const float* data, const HalfKnn& h, uint32_t k, uint32_t redo_keep, const float* norm, const float* max_norm, uint32_t* out,
                           uint32_t* redo_count, uint32_t* redo, uint32_t* doubt, hipStream_t st);
 
 // Queries against intervals of a row set, on f16 products: scan_half.hip.  The base rows in blocks, made once (mem holds
