@@ -267,7 +267,7 @@ __global__ void __launch_bounds__(256) order_thresholds_kernel(const float* __re
 }
 
 // ---- the sweep ---------------------------------------------------------------------------------------------------
-// Workgroup = 4 waves, two workgroups a CU; a workgroup owns 256 rows and sweeps the columns from the last one back to
+// Workgroup = 4 waves, three workgroups a CU (four up to 64 dimensions: half_groups); a workgroup owns 256 rows and sweeps the columns from the last one back to
 // its own rows, 32 a step.  Wave w owns rows 64 w .. + 63: their fragments stay in registers for the whole sweep (72 for
 // 128 dimensions), and a column's fragment, read from LDS, feeds two matrix instructions - 64 bytes a cycle for the CU's
 // four matrix pipes at full rate, half of what LDS delivers.  (32 rows a wave would need all of it.)  The columns of the
@@ -283,7 +283,7 @@ __global__ void __launch_bounds__(256) order_thresholds_kernel(const float* __re
 // What bounds it: the matrix pipes, busy 60 % of the launch's cycles at 1.9 GHz.  1M x 128: 1.44e14 operations in 118 ms, 1.2
 // PFLOP/s, against 402 ms on two bf16 halves a value; without the queue (a variant that appends nothing) 94 ms, 1.5 PFLOP/s,
 // where a large library product reaches 1.28 on the same card.  The columns come from L2: 0.15 TB fetched of 0.6 TB loaded.
-// Two workgroups a CU and steps of 64 columns: 123 ms.
+// Two workgroups a CU with steps of 64 columns: 123 ms.
 struct SymHalfArgs {
     const uint4* blocks;
     const uint4* row_frags;  // sym_half_long_kernel: the rows' norm fragments

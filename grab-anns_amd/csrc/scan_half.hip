@@ -7,10 +7,10 @@
 // through the queue into the row's list, nothing else is ever written.  Writing the values of all columns and selecting from
 // them (lists of 64 keys, k up to 16), or selecting inside the contraction with thresholds that start open (beyond), from
 // rows as two bf16 halves, took for 10,000 intervals of 10,000 rows of 1M x 128 512 us of kernels at k 10 and 2.8 ms at k 40,
-// for 4999 queries with 1 - 4 of 64 buckets of 200,000 x 768 540 us; this 326, 370 and 370 when it came, the first 288
+// for 4999 queries with 1 - 4 of 64 buckets of 200,000 x 768 540 us; this 326, 370 and 370 when it came, the first 276
 // since places are reserved once an item and the bounds take what a query needs.
-// What bounds it, intervals: of 174 us of sweep 59 are matrix instructions and LDS, 50 loads of chunks, one under way at a time,
-// 65 the queue (every query lists some 120 columns: a dozen in each block of 32 x 32); buckets: loads of chunks.
+// What bounds it, intervals: of 178 us of sweep some 59 are matrix instructions and LDS, 50 loads of chunks, one under way at a time,
+// the rest the queue (every query lists some 140 columns: a dozen in each block of 32 x 32); buckets: loads of chunks.
 #include <algorithm>
 #include <cmath>
 #include <type_traits>

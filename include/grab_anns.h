@@ -308,11 +308,14 @@ int grab_bucket_scan_topk(const float* d_dataset, size_t num_dataset, uint32_t d
 int grab_window_scan_topk(const float* d_dataset, size_t num_dataset, uint32_t dim, const float* d_queries,
                           size_t num_queries, uint32_t k, int metric, const uint64_t* h_id_lo, const uint64_t* h_id_hi,
                           int64_t* d_out_indices, float* d_out_dists, float* kernel_ms, void* stream);
-/* The two scans above over a prepared base (no counterpart in the reference): what a call makes of the base rows -
- * their bf16 halves, norms - is made once, and the calls' scratch memory is kept between calls, so a call costs its
- * kernels and one upload of the host's tables.  The base keeps num_dataset * dim * 4 bytes more than the rows (where
- * dim is a multiple of 32 and the base has 4096 rows or more) plus the scratch of the largest call so far (at most
- * 8 GiB).  d_dataset must stay as it is while the base exists; calls on one base must not overlap.  Same answers as
+/* The two scans above over a prepared base (no counterpart in the reference): what a call makes of the base rows is
+ * made once, and the calls' scratch memory is kept between calls, so a call costs its kernels and one upload of the
+ * host's tables.  Where dim is a multiple of 32 and the base has 4096 rows or more it keeps the rows rounded to f16, a
+ * quarter of them twice: num_dataset * (dim + 32) * 2.5 bytes.  The first call that f16 rows do not serve (narrow
+ * intervals, intervals of more than 127,000 rows, a query that is much longer than the rows, 128 queries and more not
+ * proven) has the rows as bf16 halves made as well, num_dataset * (dim + 1) * 4 bytes; without the room for these such a
+ * call takes the f16 rows or the rows as they are.  A base with a row that is not finite keeps the halves alone.  Beside
+ * that, the scratch of the largest call so far (at most 8 GiB).  d_dataset must stay as it is while the base exists; calls on one base must not overlap.  Same answers as
  * grab_window_scan_topk / grab_bucket_scan_topk. */
 typedef struct grab_scan_base grab_scan_base;
 int grab_scan_base_create(const float* d_dataset, size_t num_dataset, uint32_t dim, int metric, grab_scan_base** out);
@@ -435,11 +438,12 @@ int grab_last_knn_stats(double* flop, uint64_t* rows_redone);
  * grab_bruteforce_topk took that path (0 on data whose neighbour distances are well above the error, such as the
  * benchmark's). */
 uint64_t grab_last_knn_exact_rows(void);
-/* No counterpart in the reference.  A graph of 4096 rows or more with squared L2 and up to 128 dimensions runs its
- * bounding pass and its symmetric pass on f16 matrix instructions: the rows, centred, rounded to f16 once, with fp32 sums -
- * candidates only; the exact scoring and a check that knows how far every row moved when it was rounded decide the result.
- * Other row sets in whole chunks of 32 dimensions run on bf16 instructions, a row as two bf16 halves (16 of the 24
- * bits), a product as q_lo.c_hi + q_hi.c_lo + q_hi.c_hi; the check above then allows for these products.
+/* No counterpart in the reference.  A graph of 4096 to 2^23 rows - squared L2 and up to 128 dimensions, or either metric and a
+ * multiple of 32 - runs its bounding pass and its symmetric pass on f16 matrix instructions: the rows, centred for squared L2,
+ * rounded to f16 once, with fp32 sums - candidates only; the exact scoring and a check that knows how far every row moved when
+ * it was rounded decide the result.  The scans above do the same for most calls.  What such a pass does not prove, and two
+ * different row sets (a multiple of 32 dimensions, 1024 rows against 4096 or more), run on bf16 instructions, a row as two
+ * bf16 halves (16 of the 24 bits), a product as q_lo.c_hi + q_hi.c_lo + q_hi.c_hi; the check above then allows for these products.
  * Returns the calling thread's last call's half-precision floating-point operations, which grab_last_knn_stats leaves out,
  * counted as the three bf16 instructions that a product of split rows takes (f16 rows execute a third of it). */
 double grab_last_knn_bf16_flop(void);
