@@ -340,6 +340,15 @@ def test_knn_graph_of_rows_that_are_not_finite(grab):
         assert np.array_equal(got[finite], exp[finite])
 
 
+@pytest.mark.parametrize("n,dim,k,off,on_f16", [(16500, 64, 24, 300.0, False), (16500, 64, 24, 60.0, True), (5000, 32, 40, 400.0, True)])
+def test_knn_graph_by_inner_product_of_rows_that_point_one_way(oracle, grab, n, dim, k, off, on_f16):
+    # deviations along the mean of 4e-4 of it, where f16 rows leave most rows to be redone, of 2.1e-3, and of 4.4e-4 where the rows are few
+    data = datasets.gaussian(n, dim, 5) + np.float32(off)
+    got, _ = grab.generate_knn_graph(grab.DeviceArray.from_numpy(data), n, dim, k, 1)
+    assert (grab.last_knn_f16_flop() > 0) == on_f16 and grab.last_knn_bf16_flop() > 0
+    assert np.array_equal(got.numpy(), oracle.knn_graph(data, k, 1))
+
+
 @pytest.mark.parametrize("metric", [0, 1])
 def test_knn_graph_with_a_row_too_long_to_be_packed(oracle, grab, metric):
     # a squared norm between the 3e38 that the f16 pass takes and the largest float: the row is in no list, but among many rows'
