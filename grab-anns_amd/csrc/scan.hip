@@ -1082,8 +1082,9 @@ int grab_scan_base_create(const float* d_dataset, size_t num_dataset, uint32_t d
     };
     b->view.split = knn_bf16_allowed() && dim % KC == 0 && num_dataset >= 4096;
     if (b->view.split) {
-        // f16 rows are what the calls use first; rows as bf16 halves are made when one needs them - at once where a row is not finite
-        uint32_t bad = 0;
+        // f16 rows are what the calls use first; rows as bf16 halves are made when one needs them - at once where a row is not finite, or
+        // all point one way
+        uint32_t found[kScalOneWay + 1] = {};
         if (b->half_mem.alloc(half_base_bytes(num_dataset, dim)) != hipSuccess) {
             (void)hipGetLastError();
             set_error("scan base: out of device memory");
@@ -1091,11 +1092,11 @@ int grab_scan_base_create(const float* d_dataset, size_t num_dataset, uint32_t d
         }
         const int rc = half_base_async(d_dataset, num_dataset, dim, metric, b->half_mem.ptr, &b->half, nullptr);
         if (rc != GRAB_OK) return fail(rc);
-        if (hipMemcpy(&bad, b->half.scal + kScalBad, 4, hipMemcpyDeviceToHost) != hipSuccess) {
+        if (hipMemcpy(found, b->half.scal, sizeof(found), hipMemcpyDeviceToHost) != hipSuccess) {
             set_error("scan base: preparing the rows failed");
             return fail(GRAB_ERR_HIP);
         }
-        if (bad == 0) {
+        if (found[kScalBad] == 0 && found[kScalOneWay] == 0) {
             b->view.half = &b->half;
         } else {
             (void)hipFree(b->half_mem.ptr);

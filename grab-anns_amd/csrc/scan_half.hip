@@ -740,7 +740,8 @@ int half_base_async(const float* data, size_t n, uint32_t dim, int metric, void*
     float* cnorm = reinterpret_cast<float*>(m);
     float* eps = cnorm + n;
     GRAB_HIP(hipMemsetAsync(b.centre, 0, (size_t)dim * 4 + 64, st));
-    if (!b.ip) hipLaunchKernelGGL(half_centre_kernel, dim3(dim), dim3(256), 0, st, data, (uint64_t)n, (uint32_t)std::min<size_t>(n, 8192), dim, b.centre);
+    if (b.ip) launch_one_way(data, n, dim, reinterpret_cast<float*>(b.blocks), b.scal + kScalOneWay, st);  // (before there are blocks)
+    else hipLaunchKernelGGL(half_centre_kernel, dim3(dim), dim3(256), 0, st, data, (uint64_t)n, (uint32_t)std::min<size_t>(n, 8192), dim, b.centre);
     hipLaunchKernelGGL(half_norms_kernel, dim3((uint32_t)std::min<size_t>((n + 15) / 16, 2048)), dim3(256), 0, st, data, b.n, dim, b.centre, cnorm, b.scal);
     launch_half_pack<kAll>(data, n, dim, b.ks, b.frags, b.ip ? 0.0f : -0.5f, kScanLift, b.centre, cnorm, b.scal, nullptr, b.n, places, b.blocks, hn, eps, st);
     for (uint32_t shift = kSampleShiftMin; shift <= kSampleShiftMax; ++shift)  // (their norms go where the rows' own were, which nothing reads)

@@ -92,9 +92,14 @@ void launch_spaced_mean(const float* data, uint64_t n, uint32_t count, uint32_t 
 void launch_split_rows_chunked(const float* data, uint64_t n, uint32_t dim, const float* mean, uint16_t* out, float* norm,
                                hipStream_t stream);
 
+// *flag: whether rows rounded to f16 tell their inner products apart less well than rows as bf16 halves (1 or 0).  scratch: dim + kOneWayRows floats
+constexpr uint32_t kOneWayRows = 1024;
+void launch_one_way(const float* data, uint64_t n, uint32_t dim, float* scratch, uint32_t* flag, hipStream_t stream);
+
 // The candidates of a large kNN graph from f16 products: knn_half.hip.  Where it applies, a plan of the sizes, the lists, and
 // the neighbours that these prove.
-constexpr uint32_t kScalBad = 11, kScalLong = 12;  // words of `scal`: whether some row is not finite; whether one, not NaN, is too long to be packed
+// words of `scal`: whether some row is not finite; whether one, not NaN, is too long to be packed; scans, inner product: launch_one_way's
+constexpr uint32_t kScalBad = 11, kScalLong = 12, kScalOneWay = 13;
 constexpr uint32_t kHalfListCap = 1024;  // keys of a row's list
 constexpr uint32_t kHalfSample = 49152;  // sample rows that the bounds are taken from, at most
 struct HalfKnn {

@@ -465,10 +465,13 @@ def test_scans_of_rows_far_from_the_origin(oracle, grab, nq, k, widths):
 
 @pytest.mark.parametrize("nq,one_shot", [(60, False), (2000, False), (2000, True)])
 def test_scans_whose_f16_rows_do_not_prove_all_queries(oracle, grab, nq, one_shot):
-    # inner products of rows that all point one way: what rounding to f16 moved them by hides the order. Those queries go over the rows as
-    # they are, which proves them, or over bf16 halves where they are many, which leaves a few to be scored against every row
+    # inner products of unit rows in tight clusters: what rounding to f16 moved them by hides the order of some. Those queries go over the
+    # rows as they are, which proves them, or over bf16 halves where they are many, which leaves some to be scored against every row
     n, dim, k = 30000, 128, 32
-    data, q = datasets.gaussian(n, dim, 4) + np.float32(150.0), datasets.gaussian(nq, dim, 7) + np.float32(150.0)
+    rng = np.random.default_rng(5)
+    data = datasets.gaussian(60, dim, 4)[rng.integers(0, 60, n)] * np.float32(10.0) + datasets.gaussian(n, dim, 6) * np.float32(0.25)
+    data /= np.linalg.norm(data, axis=1, keepdims=True)
+    q = data[rng.integers(0, n, nq)].copy()
     lo, hi = _intervals(n, nq, 6000, 7000, nq)
     hi[::50] = lo[::50]
     d_data, d_q = grab.DeviceArray.from_numpy(data), grab.DeviceArray.from_numpy(q)
@@ -476,7 +479,7 @@ def test_scans_whose_f16_rows_do_not_prove_all_queries(oracle, grab, nq, one_sho
     eids, edist = oracle.bruteforce_topk(data, q, k, metric=1, filter_kind=oracle.FILTER_RANGE, ts=np.arange(n, dtype=np.uint64), win_start=lo, win_end=hi)
     for _ in range(2):
         ids, dist, _ = base.window_topk(d_q, nq, k, lo, hi) if base else grab.window_scan_topk(d_data, n, dim, d_q, nq, k, lo, hi, metric=1)
-        assert grab.last_knn_f16_flop() > 0 and grab.last_knn_stats()[1] > nq // 2 and grab.last_knn_exact_rows() <= (nq // 2 if nq >= 128 else 0)
+        assert grab.last_knn_f16_flop() > 0 and grab.last_knn_stats()[1] > 0 and grab.last_knn_exact_rows() <= (grab.last_knn_stats()[1] if nq >= 128 else 0)
         valid = eids >= 0
         assert np.array_equal(ids, eids) and np.array_equal(dist.view(np.uint32)[valid], edist.view(np.uint32)[valid])
     offsets = np.array([0, 6000, 6100, 15000, n], np.uint64)
@@ -488,3 +491,18 @@ def test_scans_whose_f16_rows_do_not_prove_all_queries(oracle, grab, nq, one_sho
     eids, edist = oracle.bruteforce_topk(data, q, k, metric=1, filter_kind=oracle.FILTER_MASK, labels=labels, masks=masks)
     valid = eids >= 0
     assert np.array_equal(ids, eids) and np.array_equal(dist.view(np.uint32)[valid], edist.view(np.uint32)[valid])
+
+
+def test_scan_base_of_rows_that_point_one_way(oracle, grab):
+    # a hundred deviations off zero in every coordinate: inner products on bf16 halves from the start, squared distances on f16 rows
+    n, dim, nq, k = 30000, 128, 300, 10
+    data, q = datasets.gaussian(n, dim, 4) + np.float32(100.0), datasets.gaussian(nq, dim, 7) + np.float32(100.0)
+    lo, hi = _intervals(n, nq, 13000, 14000, nq)
+    d_data, d_q = grab.DeviceArray.from_numpy(data), grab.DeviceArray.from_numpy(q)
+    for metric in (0, 1):
+        base = grab.ScanBase(d_data, n, dim, metric)
+        ids, dist, _ = base.window_topk(d_q, nq, k, lo, hi)
+        assert (grab.last_knn_f16_flop() > 0) == (metric == 0) and grab.last_knn_bf16_flop() > 0
+        base.close()
+        eids, edist = oracle.bruteforce_topk(data, q, k, metric=metric, filter_kind=oracle.FILTER_RANGE, ts=np.arange(n, dtype=np.uint64), win_start=lo, win_end=hi)
+        assert np.array_equal(ids, eids) and np.array_equal(dist.view(np.uint32), edist.view(np.uint32))
