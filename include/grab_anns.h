@@ -314,8 +314,9 @@ int grab_window_scan_topk(const float* d_dataset, size_t num_dataset, uint32_t d
  * quarter of them twice: num_dataset * (dim + 32) * 2.5 bytes.  The first call that f16 rows do not serve (narrow
  * intervals, intervals of more than 127,000 rows, a query that is much longer than the rows, 128 queries and more not
  * proven) has the rows as bf16 halves made as well, num_dataset * (dim + 1) * 4 bytes; without the room for these such a
- * call takes the f16 rows or the rows as they are.  A base with a row that is not finite keeps the halves alone.  Beside
- * that, the scratch of the largest call so far (at most 8 GiB).  d_dataset must stay as it is while the base exists; calls on one base must not overlap.  Same answers as
+ * call takes the f16 rows or the rows as they are.  A base with a row that is not finite, and for the inner
+ * product one whose rows all point one way, keeps the halves alone.  Beside that, the scratch of the largest call so
+ * far (at most 8 GiB).  d_dataset must stay as it is while the base exists; calls on one base must not overlap.  Same answers as
  * grab_window_scan_topk / grab_bucket_scan_topk. */
 typedef struct grab_scan_base grab_scan_base;
 int grab_scan_base_create(const float* d_dataset, size_t num_dataset, uint32_t dim, int metric, grab_scan_base** out);
